@@ -101,6 +101,11 @@ int lut6_split_sum(float* y, const float* part, long n, int nsplit, int accumula
 bool lut6_split_sum_norm_fits(int out_dim, int nsplit);
 int lut6_split_sum_norm(float* y, const float* part, long n, int nsplit, int accumulate, int rows, int out_dim,
                         const float* norm_w, float eps, float* xn, hipStream_t st);
+// The same product for larger batches (lut6_prompt.hip): the weights decoded to
+// fp16 once, then one fp16 MFMA product; and whether a call takes that path.
+bool lut6_prompt_fits(const uint8_t* w, const float* x, int batch, int out_dim, int in_dim, hipStream_t st);
+int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const float* x, int batch, int out_dim,
+                     int in_dim, int accumulate, hipStream_t st);
 // Y (+)= W X over a batch (anelm_lut6_gemm), then xn = RMSNorm(Y) * norm_w per
 // row: fused into the sum of the column slices where the GEMM is split.
 int lut6_gemm_norm(float* y, const uint8_t* w, const uint16_t* lut, const float* x, int batch, int out_dim,

@@ -795,7 +795,9 @@ int gemv(float* y, const uint8_t* w, const uint16_t* lut, const float* x, int ou
     return norm_w ? gemv_dispatch<kStageNorm>(a, 1, st) : gemv_dispatch<kStageCopy>(a, 1, st);
 }
 
-// Y[b] (+)= W X[b] for b < batch: the MFMA GEMM over tiles of 32 inputs.  The
+// Y[b] (+)= W X[b] for b < batch.  Larger batches decode the weights to fp16
+// once (lut6_prompt.hip; the rule stands at lut6_prompt_fits); the others
+// take the MFMA GEMM over tiles of 32 inputs.  Its
 // columns are cut into S equal slices (each a valid register-resident window,
 // a multiple of 256 columns when S > 1): S is the smallest count that fits,
 // raised until the (32-row group, slice) units cover every CU twice, so small
@@ -811,6 +813,11 @@ int batched_gemv(float* y, const uint8_t* w, const uint16_t* lut, const float* x
         return anelm_rmsnorm(xn + (size_t)b0 * out_dim, y + (size_t)b0 * out_dim, norm_w, out_dim, nb, out_dim,
                              out_dim, eps, st);
     };
+    if (lut6_prompt_fits(w, x, batch, out_dim, in_dim, st)) {
+        const int rc = lut6_prompt_gemm(y, w, lut, x, batch, out_dim, in_dim, accumulate, st);
+        if (rc == ANELM_OK) return norm_w ? norm_rows(0, batch) : ANELM_OK;
+        if (rc != ANELM_ENOMEM) return rc;   // without its workspace: the passes of 32 below
+    }
     int np = 0, waves = 0;
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     auto fits = [&](int s) {

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from gpu_util import assert_close, rel_l2, to_dev, to_host
-from workloads import lut6_matrix, pack_lut6, widen
+from workloads import lut6_dense, lut6_matrix, pack_lut6, widen
 
 pytestmark = pytest.mark.gpu
 
@@ -277,3 +277,39 @@ def test_layer_projections(anelm, orc, dev, out_dim, in_dim, norm, acc):
     if acc:
         want = y0 + want
     assert_close(to_host(yd), want, what=f"{out_dim}x{in_dim}")
+
+
+@pytest.mark.parametrize("batch,out_dim,in_dim,shift", [
+    (33, 32, 16, 0),        # one LUT group, half a column block, fewer stages than the pipeline is deep
+    (64, 96, 80, 4),        # rows of 60 bytes at a dword-aligned address, a part-filled tile both ways
+    (65, 160, 1040, 0),     # one input past a 64-row tile, a ragged last column pass
+    (65, 2560, 9216, 0),    # few tiles: column slices and their sum
+    (257, 1024, 3584, 0),   # one input past 256
+    (300, 12352, 2560, 0),  # more tiles than compute units, ragged in both
+    (1030, 18432, 1024, 0),  # the largest tile
+])
+def test_prompt_gemm(anelm, dev, batch, out_dim, in_dim, shift):
+    """Batches past two passes of 32: weights decoded to fp16 once and one fp16
+    product.  Against float64 on the dequantised weights and the fp16 inputs:
+    products of two fp16 values are exact in fp32, so each output is within
+    in_dim fp32 roundings of the sum of the magnitudes (one more with the
+    accumulated value)."""
+    packed, lut, idx = lut6_matrix(700 + batch, out_dim, in_dim)
+    rng = np.random.default_rng(701 + batch)
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    y0 = rng.standard_normal((batch, out_dim)).astype(np.float32)
+    raw = torch.zeros(packed.size + 64, dtype=torch.uint8, device=dev)
+    raw[shift:shift + packed.size] = to_dev(packed, dev).view(-1)
+    w = raw[shift:]
+    lut_d, xd, yd = to_dev(lut, dev), to_dev(x, dev), to_dev(y0, dev)
+    got = anelm.ops.lut6_gemm(w, lut_d, xd, out_dim, in_dim)
+    acc = anelm.ops.lut6_gemm(w, lut_d, xd, out_dim, in_dim, out=yd, accumulate=True)
+    wd = torch.from_numpy(lut6_dense(idx, lut)).to(dev).double()
+    xh = xd.half().double()
+    want, mag = xh @ wd.t(), xh.abs() @ wd.t().abs()
+    bound = (in_dim + 1) * 2.0 ** -24 * mag
+    assert bool(((got.double() - want).abs() <= bound).all())
+    want, mag = want + torch.from_numpy(y0).to(dev), mag + torch.from_numpy(np.abs(y0)).to(dev)
+    assert bool(((acc.double() - want).abs() <= (in_dim + 2) * 2.0 ** -24 * mag).all())
+    # repeated call: same bits
+    assert torch.equal(got, anelm.ops.lut6_gemm(w, lut_d, xd, out_dim, in_dim))
