@@ -7,7 +7,8 @@
 // 128 times, 5.1 ms for the 2560 -> 2 x 9216 -> 2560 FFN block.  Here the
 // weights are decoded once into fp16 (exactly: a LUT entry is an fp16 value),
 // the inputs are rounded to fp16 once (as every LUT6 path takes them), and one
-// fp16 MFMA product with fp32 accumulation follows: @FFN@.
+// fp16 MFMA product with fp32 accumulation follows: that block takes 805 us
+// (weights and inputs prepared in 56 + 31 us, products 390 + 269).
 // Reference math: matvec (core/cpu_ops.cpp:77-80) on the dequantised weights,
 // per input.
 //
@@ -68,10 +69,9 @@ __device__ __forceinline__ void convert_x(const PrepArgs& a, int id) {
 // Per pass of 512 columns the packed rows go to LDS with 16-byte loads (the
 // next pass's in flight meanwhile); then a thread takes one 16-byte output
 // chunk (8 columns = 6 packed bytes) at a time, 16 rows x 4 chunks per wave,
-// so every store instruction writes 1 KiB of consecutive memory (stores of
-// 16 bytes 64 bytes apart took @WOLD@ for 18432 x 2560 against @WNEW@).  The
-// pair table T[(i1 << 6) | i0] = (lut[i0], lut[i1]) turns 12 bits into two
-// weights per LDS read.
+// so every store instruction writes 1 KiB of consecutive memory.  The pair
+// table T[(i1 << 6) | i0] = (lut[i0], lut[i1]) turns 12 bits into two weights
+// per LDS read.
 constexpr int kDecCols = 512;
 constexpr int kDecRow = kDecCols * 3 / 4 + 16;   // staged row pitch (bytes): rows start 4 banks apart
 typedef uint32_t u32x4_dw __attribute__((ext_vector_type(4), aligned(4)));   // rows start at multiples of 12 bytes
@@ -390,7 +390,10 @@ int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const floa
     for (int b0 = 0; b0 < batch; b0 += kMaxRows)
         for (int n0 = 0; n0 < out_dim; n0 += n_max) bytes = std::max(bytes, plan(b0, n0).bytes);
     char* ws = static_cast<char*>(workspace2(bytes, st));
-    if (!ws) return ANELM_ENOMEM;
+    if (!ws) {
+        (void)hipGetLastError();   // a failed allocation is no launch error of the path taken instead
+        return ANELM_ENOMEM;
+    }
     for (int b0 = 0; b0 < batch; b0 += kMaxRows)
         for (int n0 = 0; n0 < out_dim; n0 += n_max) {
             const Plan p = plan(b0, n0);
