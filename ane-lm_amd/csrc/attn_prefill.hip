@@ -18,6 +18,9 @@
 
 #include <math.h>
 
+#include <atomic>
+#include <type_traits>
+
 namespace anelm {
 namespace {
 
@@ -27,13 +30,21 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kBN = 32;  // keys per tile
 
+// A ring of `cap` rows [Hkv][D] (k, v): key i of the sequence is row
+// (start + i) mod cap.  A plain array of L keys is the ring (0, L).
+struct KeyRing {
+    const _Float16* k;
+    const _Float16* v;
+    int start, cap;
+};
+
 // Query row r is key qoff + r of the L keys in k / v (the keys before qoff
 // are a cached prefix) and attends keys (qoff + r - win, qoff + r] (win 0: no
 // lower bound).  With gate, the output row is multiplied by sigmoid of
 // gate[r * gtok + h * ghead + d] (the reference's output gate).
 template <int D, int HB, int RB, bool OUT16>
 __global__ __launch_bounds__(HB * RB * 64) void prefill_kernel(void* out, const _Float16* q,
-                                                               const _Float16* k, const _Float16* v,
+                                                               const KeyRing rg,
                                                                int S, int L, int qoff, int win, int Hq, int Hkv,
                                                                const float* gate, int gtok, int ghead) {
     constexpr int NW = HB * RB;
@@ -80,8 +91,10 @@ __global__ __launch_bounds__(HB * RB * 64) void prefill_kernel(void* out, const 
             const int key = j0 + kr;
             uint4 kv4 = make_uint4(0, 0, 0, 0), vv4 = make_uint4(0, 0, 0, 0);
             if (key < L) {
-                kv4 = *reinterpret_cast<const uint4*>(k + ((size_t)key * Hkv + kvh) * D + kc);
-                vv4 = *reinterpret_cast<const uint4*>(v + ((size_t)key * Hkv + kvh) * D + kc);
+                const int at = key + rg.start;
+                const size_t row = at - (at >= rg.cap ? rg.cap : 0);
+                kv4 = *reinterpret_cast<const uint4*>(rg.k + (row * Hkv + kvh) * D + kc);
+                vv4 = *reinterpret_cast<const uint4*>(rg.v + (row * Hkv + kvh) * D + kc);
             }
             *reinterpret_cast<uint4*>(&Ks[kr][kc]) = kv4;
             const _Float16* vh = reinterpret_cast<const _Float16*>(&vv4);
@@ -169,452 +182,594 @@ __global__ __launch_bounds__(HB * RB * 64) void prefill_kernel(void* out, const 
 }
 
 // ---------------------------------------------------------------------------
-// Workload-balanced, pipelined kernel for head_dim 256 and 4 query heads per KV
-// head (the Qwen3.5 shapes).
+// Pipelined kernel for head_dim 256 and 4 query heads per KV head (the Qwen3.5
+// shapes), any prompt length and cached history.
 //
-// * Blocks of 64 query rows; a workgroup's 8 waves are 4 query heads x 2 row
-//   halves of 32 rows, and all of them consume ONE stream of 32-key tiles, so
-//   each K / V byte staged in LDS feeds 256 query rows.
-// * Balance: a unit is a KV head and a pair of blocks (a, nb-1-a) (or the
-//   middle block when nb is odd).  Its causal key tiles, a's then b's, are cut
-//   into two equal halves taken by two workgroups.  The block whose tiles are
-//   split is merged by whichever of the two finishes second: a relaxed
-//   device-scope counter orders their arrivals, the first writes its partial
-//   (m, l, unnormalised O) with device-coherent stores and counts again once
-//   they are out, the second waits for that count, combines the partial with
-//   its registers, writes the rows and re-zeroes the counter for the next
-//   call.
-// * Stream: K and V tiles (32 keys x 256) go straight to LDS with buffer loads
-//   (1 KiB per wave instruction: rows c and c+16 of a tile share a chunk) into
-//   a ring of 4 buffers, 3 tiles ahead of use.  K chunks are 1040 bytes (16 of
-//   padding) so the MFMA operand reads are conflict-free with immediate
-//   offsets; V chunks are 1088 bytes, so the four key rows a 16-lane group
-//   reads with ds_read_b64_tr_b16 (4 keys x 16 dims, delivered transposed:
-//   lane n gets dim n of the 4 keys) fall on distinct banks.  That transposing
-//   read builds the V^T operand of O^T += V^T P^T from the V rows as stored.
+// * A wave's 32 columns are 8 tokens x the 4 query heads of the KV head; a
+//   workgroup's 8 waves are 8 / KP column groups x KP key parts: a step stages
+//   KP consecutive 32-key tiles and each wave takes the one of its part, so
+//   the KP waves of a column group merge their (m, l, O) through LDS at the
+//   end (each ends with 256 / KP of the dims).
+// * A group of 64 / KP tokens whose steps exceed `sps` is cut into parts of
+//   sps steps, one workgroup each; parts write (m, l, unnormalised O) records
+//   and prefill_split_combine merges them.  The rule stands at plan_split.
+// * K and V tiles (32 keys x 256) go straight to LDS with buffer loads (1 KiB
+//   per wave instruction: rows c and c+16 of a tile share a chunk).  K chunks
+//   are 1040 bytes (16 of padding) so the MFMA operand reads are conflict-free
+//   with immediate offsets; V chunks are 1088 bytes, so the four key rows a
+//   16-lane group reads with ds_read_b64_tr_b16 (4 keys x 16 dims, delivered
+//   transposed: lane n gets dim n of the 4 keys) fall on distinct banks.  That
+//   transposing read builds the V^T operand of O^T += V^T P^T from the V rows
+//   as stored.  KP 2: two steps of tiles in LDS, the next step's loads behind
+//   the one barrier of a step.  KP 4: one step in LDS; the next step's K tiles
+//   are requested once the scores are formed, its V tiles once the outputs
+//   are (four barriers per step).
 // * Scores S^T = K Q^T (v_mfma_f32_32x32x16_f16).  The A-operand lane i reads
 //   key row pi(i) (bits 2 and 3 of i swapped): lane (r, h) of the accumulator
-//   then holds the scores of query row r for keys 8h..8h+7 and 16+8h..16+8h+7,
+//   then holds the scores of column r for keys 8h..8h+7 and 16+8h..16+8h+7,
 //   exactly the B-operand keys of O^T += V^T P^T.
 // * Softmax in the log2 domain; the running maximum only moves when it grows
 //   by more than 8, so probabilities stay below 2^8 (fp16-exact range) and the
 //   128-register output rescale is rare.
+// Bound: the matrix units and LDS in turn (a step's 32 products per wave are
+// 1 us of the CU's matrix time and its operand reads 1 us of its LDS; a step
+// takes 1.9 us, 2.8 us with every CU under load).  Whole layer call, before
+// (64-row blocks in causal pairs, two workgroups per pair, which left the chip
+// to 2 Hkv ceil(S / 128) workgroups) and now: 4096 tokens 16q/4kv 228 -> 217
+// us, 1000 tokens 82 -> 44, 777 tokens 8q/2kv behind 1500 keys 146 -> 44, 16
+// tokens behind 4000 keys 110 -> 22.
 constexpr int kGKeys = 32;                       // keys per tile
 constexpr int kGKBytes = 16 * 1040;              // K tile: chunk c = rows c, c + 16
 constexpr int kGVChunk = 1088;                   // V tile chunk: rows c, c + 16 + 64 bytes of bank offset
 constexpr int kGTile = kGKBytes + 16 * kGVChunk; // + V tile (32 x 256 fp16)
-constexpr int kGBuf = 4;                         // ring of tile buffers
-constexpr int kGLds = kGBuf * kGTile + 64;       // + the merge flag
-constexpr int kGSlotFloats = 8 * 128 * 64 + 8 * 128;   // partial: O (8 waves x 128 x 64 lanes), m, l
 constexpr int kGNT = 512;
-constexpr int kSc1 = 16;                         // buffer cache policy: device-scope coherent
-
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+// Running maximum of a column that has seen no key yet: far below any score
+// and finite, so a tile that is wholly masked for the column adds
+// exp2(-inf - kNoKey) = 0 (from -inf it would add NaN).
+constexpr float kNoKey = -1e30f;
 
 __device__ __forceinline__ int key_perm(int i) { return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1); }
 
-// Key tiles needed by 64-row block blk: keys 0 .. qoff + min(64 blk + 63, S - 1).
-__device__ __forceinline__ int block_tiles(int blk, int S, int qoff) {
-    return (qoff + min(64 * blk + 64, S) + 31) / 32;
+// One 32-key tile (staged at `base`) against a wave's 32 query columns, in
+// three parts.  S^T = K Q^T:
+__device__ __forceinline__ float16_t tile_scores(const char* base, int ln, const half8 (&qf)[16]) {
+    constexpr int KS = 16;
+    float16_t sc = float16_t{};
+    {
+        const int krow = key_perm(ln & 31);
+        const char* kb = base + (krow & 15) * 1040 + (krow >> 4) * 512 + (ln >> 5) * 16;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8*>(kb + 32 * ks), qf[ks], sc,
+                                                        0, 0, 0);
+        // K fragment ks + 1 is read while the product of fragment ks runs
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS - 2; ks++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    }
+    return sc;
 }
 
-// Query row r is key qoff + r of the L keys (the keys before qoff are a
-// cached prefix) and attends keys 0 .. qoff + r.  With gate, output row
-// (r, h) is multiplied by sigmoid(gate[r * gtok + h * ghead + d]).
+// The online softmax: running maximum m, this lane half's sum l, O rescaled
+// when the maximum moves; P^T in pf.  The tile's keys are j0 .. j0 + 31,
+// element e of the scores being key j0 + (e < 8 ? 8 h + e : 16 + 8 h + e - 8);
+// masked: some column stops before the last of them, qr being the last key of
+// this lane's column.
+__device__ __forceinline__ void tile_softmax(float16_t sc, half8 (&pf)[2], float16_t (&o)[8], float& m, float& l,
+                                             float sl2, int ln, int j0, bool masked, int qr) {
+    constexpr int DB = 8;
+    if (masked) {
+        const int h2 = ln >> 5;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int key = j0 + (e < 8 ? 8 * h2 + e : 16 + 8 * h2 + (e - 8));
+            sc[e] = key <= qr ? sc[e] : -INFINITY;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; e++) mx = fmaxf(mx, sc[e]);
+    mx = fmaxf(mx, shfl_xor(mx, 32)) * sl2;
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
+        const float m_new = fmaxf(m, mx);
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        l *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) o[db][e] *= alpha;
+        m = m_new;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const float pe = __builtin_amdgcn_exp2f(fmaf(sc[e], sl2, -m));
+        l += pe;
+        pf[e / 8][e % 8] = (_Float16)pe;
+    }
+}
+
+// O^T += V^T P^T.  The A operand of lane (m, h2) for keys 16u + 8 h2 .. +8
+// and dim 32 db + m comes from two transposing reads: 16-lane group i (m =
+// 16 (i & 1) + n, h2 = i >> 1) has its lane n address key 16u + 8 (i >> 1) +
+// 4r + n / 4, dims 32 db + 16 (i & 1) + 4 (n % 4) .. +4 of the V rows (key t
+// at chunk t % 16, half t / 16).
+__device__ __forceinline__ void tile_values(const char* base, int ln, const half8 (&pf)[2], float16_t (&o)[8]) {
+    constexpr int DB = 8;
+    {
+        const int gi = ln >> 4, nn = ln & 15;
+        const char* vbase = base + kGKBytes + (8 * (gi >> 1) + (nn >> 2)) * kGVChunk +
+                            (16 * (gi & 1) + 4 * (nn & 3)) * 2;
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        static_assert(4 * kGVChunk == 4352, "offset of the second read");
+        const uint32_t va = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const char*)vbase);
+        // product k = 2 db + u; the reads of product k + 1 are issued
+        // before product k (each asm statement waits only for the
+        // older pair, which it passes through to the product)
+        s16x4 lo[2], hi[2];
+        asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %2 offset:4352"
+                     : "=&v"(lo[0]), "=&v"(hi[0])
+                     : "v"(va)
+                     : "memory");
+#pragma unroll
+        for (int kk = 0; kk < 2 * DB; kk++) {
+            const int db = kk >> 1, u = kk & 1, c = kk & 1, n = c ^ 1;
+            if (kk + 1 < 2 * DB) {
+                const int u1 = (kk + 1) & 1, db1 = (kk + 1) >> 1;
+                asm volatile(
+                    "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %4 offset:4352\n\ts_waitcnt lgkmcnt(2)"
+                    : "=&v"(lo[n]), "=&v"(hi[n]), "+v"(lo[c]), "+v"(hi[c])
+                    : "v"(va + (uint32_t)(u1 * 512 + 64 * db1))
+                    : "memory");
+            } else {
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo[c]), "+v"(hi[c]) : : "memory");
+            }
+            const half8 av =
+                __builtin_bit_cast(half8, __builtin_shufflevector(lo[c], hi[c], 0, 1, 2, 3, 4, 5, 6, 7));
+            o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pf[u], o[db], 0, 0, 0);
+        }
+    }
+}
+
+// Byte offset, in its ring, of 16-byte chunk `ch` of key `key` (kv head kvh);
+// keys past the last one (L) are out of the buffers' range and read zeros.
+__device__ __forceinline__ int ring_off(const KeyRing& rg, int L, int Hkv, int kvh, int key, int ch) {
+    const int at = key + rg.start, row = at - (at >= rg.cap ? rg.cap : 0);
+    return key < L ? ((row * Hkv + kvh) * 256 + 8 * ch) * 2 : 0x7fffffff;
+}
+
+// LDS: four tiles, then m and l of the 8 waves.
+template <int KP>
+constexpr int split_lds() { return 4 * kGTile + 2 * 8 * 64 * (int)sizeof(float); }
+
+// Steps of KP tiles that group grp (64 / KP tokens) needs.
+__host__ __device__ inline int split_steps(int KP, int grp, int S, int qoff) {
+    const int tok = 64 / KP, end = (grp + 1) * tok < S ? (grp + 1) * tok : S;
+    return (qoff + end + 32 * KP - 1) / (32 * KP);
+}
+
+// Four output values (dims d .. d + 3 of row (tok, h)), normalised and gated.
 template <bool OUT16, bool GATE>
-__global__ __launch_bounds__(kGNT) void prefill_g4_kernel(void* out, const _Float16* q, const _Float16* k,
-                                                           const _Float16* v, float* part, uint32_t* ctr, int S,
-                                                           int L, int qoff, int Hq, int Hkv,
-                                                           const float* gate, int gtok, int ghead) {
-    constexpr int D = 256, KS = D / 16, DB = D / 32;
+__device__ __forceinline__ void split_store(void* out, const float* gate, int gtok, int ghead, int tok, int h, int Hq,
+                                            int d, float4 x, float inv) {
+    x = make_float4(x.x * inv, x.y * inv, x.z * inv, x.w * inv);
+    if constexpr (GATE) {   // (rows of any stride: four dword loads)
+        const float* g = gate + (size_t)tok * gtok + (size_t)h * ghead + d;
+        x.x = x.x / (1.0f + expf(-g[0]));
+        x.y = x.y / (1.0f + expf(-g[1]));
+        x.z = x.z / (1.0f + expf(-g[2]));
+        x.w = x.w / (1.0f + expf(-g[3]));
+    }
+    const size_t off = ((size_t)tok * Hq + h) * 256 + d;
+    if constexpr (OUT16)
+        *reinterpret_cast<half4*>(static_cast<_Float16*>(out) + off) =
+            half4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w};
+    else
+        *reinterpret_cast<float4*>(static_cast<float*>(out) + off) = x;
+}
+
+struct SplitArgs {
+    void* out;
+    const _Float16* q;
+    KeyRing rg;
+    float* rec;            // [Hkv][ngrp][parts] records
+    const float* gate;
+    int S, L, qoff, Hq, Hkv, gtok, ghead;
+    int ngrp, parts, sps;  // groups per kv head, most parts of a group, steps per part
+};
+
+// Record of one part: O in accumulator order ([wave][8 / KP blocks of 32
+// dims][4][64 lanes] float4), then m and l of [8 / KP column groups][32].
+template <int KP>
+constexpr int split_rec_floats() { return 8 * (8 / KP) * 4 * 256 + 2 * (8 / KP) * 32; }
+
+template <int KP, bool OUT16, bool GATE>
+__global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) {
+    constexpr int KS = 16, DB = 8, CG = 8 / KP, QB = 8 / KP;   // column groups; dim blocks a wave ends with
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int hl = w & 3, rh = w >> 2;
-    const int nb = (S + 63) / 64, npair = nb / 2, upk = npair + (nb & 1);
-    // consecutive units on one XCD (workgroup id mod 8 selects the XCD): one KV head per L2
-    int lw = blockIdx.x;
-    if (gridDim.x % 8 == 0) lw = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-    const int unit = lw >> 1, half_id = lw & 1;
-    const int kvh = unit / upk, pu = unit % upk;
-    const int h = kvh * 4 + hl;
-    const int blk_a = pu < npair ? pu : -1, blk_b = pu < npair ? nb - 1 - pu : npair;
-    const int nta = blk_a >= 0 ? block_tiles(blk_a, S, qoff) : 0, ntb = block_tiles(blk_b, S, qoff);
-    const int half = (nta + ntb) / 2, nb0 = half - nta;   // tiles of b taken by the first workgroup
-    const bool split = nb0 > 0;
-    // this workgroup's segments (block, first key tile, tile count)
-    int blk0, t00, n0, blk1 = 0, t01 = 0, n1 = 0;
-    if (half_id == 0) {
-        if (nta > 0) {
-            blk0 = blk_a; t00 = 0; n0 = nta;
-            if (nb0 > 0) { blk1 = blk_b; t01 = 0; n1 = nb0; }
-        } else {
-            blk0 = blk_b; t00 = 0; n0 = nb0;
-        }
+    const int cg = w % CG, kp = w / CG;
+    // workgroup -> (kv head, group, part): an XCD (workgroup id mod 8) serves
+    // one kv head where 8 is a multiple of their number; last groups (the
+    // longest) first
+    const int bpk = a.ngrp * a.parts;
+    int kvh, idx;
+    if (8 % a.Hkv == 0) {
+        const int spx = 8 / a.Hkv, xcd = blockIdx.x & 7;
+        kvh = xcd / spx;
+        idx = (int)(blockIdx.x >> 3) * spx + xcd % spx;
     } else {
-        const int f = nb0 > 0 ? nb0 : 0;
-        blk0 = blk_b; t00 = f; n0 = ntb - f;
+        kvh = blockIdx.x % a.Hkv;
+        idx = blockIdx.x / a.Hkv;
     }
-    if (n0 <= 0) return;
-    const int nseg = n1 > 0 ? 2 : 1;
-    const int ntot = n0 + n1;
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16*>(k), 0, (int)min((size_t)L * Hkv * D * 2, (size_t)0x7fffffff), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16*>(v), 0, (int)min((size_t)L * Hkv * D * 2, (size_t)0x7fffffff), 0x00020000);
-    const float sl2 = (1.0f / 16.0f) * 1.4426950408889634f;   // 1/sqrt(256) * log2(e)
-    auto key_tile = [&](int i) { return i < n0 ? t00 + i : t01 + (i - n0); };
-    // stream tile i -> buffer i % 4; wave w loads K and V chunks 2w, 2w+1
-    auto issue = [&](int i) {
-        char* base = lds + (i % kGBuf) * kGTile;
-        const int j0 = key_tile(i) * kGKeys;
+    if (idx >= bpk) return;
+    const int grp = a.ngrp - 1 - idx % a.ngrp, part = idx / a.ngrp;
+    const int steps = split_steps(KP, grp, a.S, a.qoff);
+    const int s0 = part * a.sps, s1 = min(steps, s0 + a.sps);
+    if (s0 >= s1) return;
+    const int tok0 = grp * (64 / KP) + 8 * cg;
+
+    const __amdgpu_buffer_rsrc_t rk =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.rg.k), 0, a.rg.cap * a.Hkv * 512, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.rg.v), 0, a.rg.cap * a.Hkv * 512, 0x00020000);
+    constexpr int PERW = 16 / CG;   // chunks of its part's K (and V) tile that a wave loads
+    char* const mine = lds + kp * kGTile;
+    constexpr int kStage = KP * kGTile;   // KP 2: step s in stage s % 2
+    auto issue = [&](int s, auto is_v) __attribute__((always_inline)) {
+        constexpr bool values = decltype(is_v)::value;
+        char* base = mine + (KP == 2 ? (s & 1) * kStage : 0) + (values ? kGKBytes : 0);
+        const int j0 = (s * KP + kp) * kGKeys, at = j0 + a.rg.start, row = at - (at >= a.rg.cap ? a.rg.cap : 0);
         int ln = threadIdx.x & 63;
         asm volatile("" : "+v"(ln));   // lane offsets are recomputed here, not held across the loop
+        if (j0 + kGKeys <= a.L && row + kGKeys <= a.rg.cap) {
+            // (wave-uniform) the whole tile is consecutive rows: one lane offset, the chunk's in a scalar
+            const int voff = (ln >> 5) * 16 * a.Hkv * 512 + (ln & 31) * 16;
 #pragma unroll
-        for (int x = 0; x < 2; x++) {
-            const int c = 2 * w + x, row = c + 16 * (ln >> 5), key = j0 + row;
-            const int off = key < L ? ((key * Hkv + kvh) * D + 8 * (ln & 31)) * 2 : 0x7fffffff;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(base + c * 1040), 16,
-                                                     off, 0, 0, 0);
+            for (int x = 0; x < PERW; x++) {
+                const int c = PERW * cg + x;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    values ? rv : rk, (__attribute__((address_space(3))) void*)(base + c * (values ? kGVChunk : 1040)),
+                    16, voff, ((row + c) * a.Hkv + kvh) * 512, 0, 0);
+            }
+            return;
         }
 #pragma unroll
-        for (int x = 0; x < 2; x++) {
-            const int c = 2 * w + x, row = c + 16 * (ln >> 5), key = j0 + row;
-            const int off = key < L ? ((key * Hkv + kvh) * D + 8 * (ln & 31)) * 2 : 0x7fffffff;
+        for (int x = 0; x < PERW; x++) {
+            const int c = PERW * cg + x, key = j0 + c + 16 * (ln >> 5);
+            const int off = ring_off(a.rg, a.L, a.Hkv, kvh, key, ln & 31);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rv, (__attribute__((address_space(3))) void*)(base + kGKBytes + c * kGVChunk), 16, off, 0, 0, 0);
+                values ? rv : rk, (__attribute__((address_space(3))) void*)(base + c * (values ? kGVChunk : 1040)), 16, off,
+                0, 0, 0);
         }
     };
-    for (int i = 0; i < 3 && i < ntot; i++) issue(i);
-    int i = 0;
-    for (int sg = 0; sg < nseg; sg++) {
-        const int blk = sg == 0 ? blk0 : blk1;
-        const int row0 = 64 * blk + 32 * rh;
-        half8 qf[KS];
-        {
-            const int lane = threadIdx.x & 63, qrow = row0 + (lane & 31);
+    constexpr std::integral_constant<bool, false> K{};
+    constexpr std::integral_constant<bool, true> V{};
+    issue(s0, K);
+    issue(s0, V);
+    half8 qf[KS];
+    {
+        const int lane = threadIdx.x & 63, tok = min(tok0 + ((lane & 31) >> 2), a.S - 1);
+        const _Float16* qr = a.q + ((size_t)tok * a.Hq + kvh * 4 + (lane & 3)) * 256 + 8 * (lane >> 5);
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                if (qrow < S)
-                    qf[ks] = *reinterpret_cast<const half8*>(q + ((size_t)qrow * Hq + h) * D + 16 * ks + 8 * (lane >> 5));
-                else
-                    qf[ks] = half8{};
+        for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const half8*>(qr + 16 * ks);
+    }
+    float16_t o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; db++) o[db] = float16_t{};
+    float m = kNoKey, l = 0.f;
+    const float sl2 = (1.0f / 16.0f) * 1.4426950408889634f;   // 1/sqrt(256) * log2(e)
+    const int first = a.qoff + tok0, last = a.qoff + min(tok0 + 7, a.S - 1);   // last keys of the wave's tokens
+    if constexpr (KP == 2) {
+        for (int s = s0; s < s1; s++) {
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's loads of step s have landed
+            lds_barrier();                      // every wave's; the other stage is free
+            if (s + 1 < s1) {
+                issue(s + 1, K);
+                issue(s + 1, V);
             }
-        }
-        // the Q fragments complete here, so no wait for them remains inside the tile loop
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        float16_t o[DB];
-#pragma unroll
-        for (int db = 0; db < DB; db++) o[db] = float16_t{};
-        float m = -INFINITY, l = 0.f;
-        const int iend = sg == 0 ? n0 : ntot;
-        for (; i < iend; i++) {
-            // tile i has landed once at most the loads of tiles i+1, i+2 (4 per wave each) remain
-            const int left = ntot - 1 - i;
-            if (left >= 2) __builtin_amdgcn_s_waitcnt(0x0F78);
-            else if (left == 1) __builtin_amdgcn_s_waitcnt(0x0F74);
-            else __builtin_amdgcn_s_waitcnt(0x0F70);
-            __syncthreads();   // every wave's part of tile i landed; buffer (i+3)%4 (tile i-1) is free
-            if (i + 3 < ntot) issue(i + 3);
-            const int kt = key_tile(i), j0 = kt * kGKeys;
-            if (j0 > qoff + row0 + 31) continue;   // every key of this tile lies after this wave's rows
-            const char* base = lds + (i % kGBuf) * kGTile;
+            const int j0 = (s * KP + kp) * kGKeys;
             int ln = threadIdx.x & 63;
             asm volatile("" : "+v"(ln));
-            // ---- S^T = K Q^T
+            // (wave-uniform) a tile past the wave's last token has nothing for it
+            if (tok0 < a.S && j0 <= last) {
+                const char* base = mine + (s & 1) * kStage;
+                half8 pf[2];
+                tile_softmax(tile_scores(base, ln, qf), pf, o, m, l, sl2, ln, j0, j0 + 31 > first,
+                             a.qoff + tok0 + ((ln & 31) >> 2));
+                tile_values(base, ln, pf, o);
+            }
+        }
+    } else {
+        constexpr int kHalf = 0x0F70 | PERW;   // vmcnt(PERW): all but the newest PERW loads
+        for (int s = s0; s < s1; s++) {
+            const bool next = s + 1 < s1;
+            const int j0 = (s * KP + kp) * kGKeys;
+            const bool live = tok0 < a.S && j0 <= last;   // (wave-uniform)
+            int ln = threadIdx.x & 63;
+            asm volatile("" : "+v"(ln));
+            __builtin_amdgcn_s_waitcnt(kHalf);   // K of step s (V of step s behind it)
+            lds_barrier();
             float16_t sc = float16_t{};
-            {
-                const int krow = key_perm(ln & 31);
-                const char* kb = base + (krow & 15) * 1040 + (krow >> 4) * 512 + (ln >> 5) * 16;
-#pragma unroll
-                for (int ks = 0; ks < KS; ks++)
-                    sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8*>(kb + 32 * ks), qf[ks], sc,
-                                                                0, 0, 0);
-                // K fragment ks + 1 is read while the product of fragment ks runs
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-                for (int ks = 0; ks < KS - 2; ks++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            }
-            // ---- online softmax; element e holds key j0 + (e < 8 ? 8 h + e : 16 + 8 h + e - 8)
-            if (j0 + 31 > qoff + row0) {
-                const int h2 = ln >> 5, qr = qoff + row0 + (ln & 31);
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int key = j0 + (e < 8 ? 8 * h2 + e : 16 + 8 * h2 + (e - 8));
-                    sc[e] = key <= qr ? sc[e] : -INFINITY;
-                }
-            }
-            float mx = -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 16; e++) mx = fmaxf(mx, sc[e]);
-            mx = fmaxf(mx, shfl_xor(mx, 32)) * sl2;
-            if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
-                const float m_new = fmaxf(m, mx);
-                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-                l *= alpha;
-#pragma unroll
-                for (int db = 0; db < DB; db++)
-#pragma unroll
-                    for (int e = 0; e < 16; e++) o[db][e] *= alpha;
-                m = m_new;
-            }
-            half8 pf[2];
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const float pe = __builtin_amdgcn_exp2f(fmaf(sc[e], sl2, -m));
-                l += pe;
-                pf[e / 8][e % 8] = (_Float16)pe;
-            }
-            // ---- O^T += V^T P^T.  The A operand of lane (m, h2) for keys
-            // 16u + 8 h2 .. +8 and dim 32 db + m comes from two transposing
-            // reads: 16-lane group i (m = 16 (i & 1) + n, h2 = i >> 1) has
-            // its lane n address key 16u + 8 (i >> 1) + 4r + n / 4, dims
-            // 32 db + 16 (i & 1) + 4 (n % 4) .. +4 of the V rows (key t at
-            // chunk t % 16, half t / 16).
-            {
-                const int gi = ln >> 4, nn = ln & 15;
-                const char* vbase = base + kGKBytes + (8 * (gi >> 1) + (nn >> 2)) * kGVChunk +
-                                    (16 * (gi & 1) + 4 * (nn & 3)) * 2;
-                typedef short s16x4 __attribute__((ext_vector_type(4)));
-                static_assert(4 * kGVChunk == 4352, "offset of the second read");
-                const uint32_t va = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const char*)vbase);
-                // product k = 2 db + u; the reads of product k + 1 are issued
-                // before product k (each asm statement waits only for the
-                // older pair, which it passes through to the product)
-                s16x4 lo[2], hi[2];
-                asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %2 offset:4352"
-                             : "=&v"(lo[0]), "=&v"(hi[0])
-                             : "v"(va)
-                             : "memory");
-#pragma unroll
-                for (int kk = 0; kk < 2 * DB; kk++) {
-                    const int db = kk >> 1, u = kk & 1, c = kk & 1, n = c ^ 1;
-                    if (kk + 1 < 2 * DB) {
-                        const int u1 = (kk + 1) & 1, db1 = (kk + 1) >> 1;
-                        asm volatile(
-                            "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %4 offset:4352\n\ts_waitcnt lgkmcnt(2)"
-                            : "=&v"(lo[n]), "=&v"(hi[n]), "+v"(lo[c]), "+v"(hi[c])
-                            : "v"(va + (uint32_t)(u1 * 512 + 64 * db1))
-                            : "memory");
-                    } else {
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo[c]), "+v"(hi[c]) : : "memory");
-                    }
-                    const half8 av =
-                        __builtin_bit_cast(half8, __builtin_shufflevector(lo[c], hi[c], 0, 1, 2, 3, 4, 5, 6, 7));
-                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pf[u], o[db], 0, 0, 0);
-                }
-            }
+            half8 pf[2] = {};
+            if (live) sc = tile_scores(mine, ln, qf);
+            lds_barrier();   // K is free
+            if (next) issue(s + 1, K);
+            if (live)
+                tile_softmax(sc, pf, o, m, l, sl2, ln, j0, j0 + 31 > first, a.qoff + tok0 + ((ln & 31) >> 2));
+            if (next) __builtin_amdgcn_s_waitcnt(kHalf);   // V of step s (K of step s + 1 behind it)
+            else __builtin_amdgcn_s_waitcnt(0x0F70);
+            lds_barrier();
+            if (live) tile_values(mine, ln, pf, o);
+            lds_barrier();   // V is free
+            if (next) issue(s + 1, V);
         }
-        l += shfl_xor(l, 32);
-        int ln = threadIdx.x & 63;
-        asm volatile("" : "+v"(ln));   // the epilogue's addresses are computed here, not held through the loop
-        const int erow = row0 + (ln & 31), eh = ln >> 5;
-        float a0 = 1.f, a1 = 0.f, inv;
-        __amdgpu_buffer_rsrc_t rot = __builtin_amdgcn_make_buffer_rsrc(part, 0, 0, 0x00020000);
-        bool have_other = false;
-        if (split && blk == blk_b) {
-            // The split block's two workgroups arrive on the unit's counter
-            // (0 -> 1 -> 2, one more when the first one's partial is out).
-            // The first to arrive publishes its partial and leaves; the
-            // second waits until that partial is stored (the first is
-            // resident, and nothing stands between its arrival and its
-            // stores), merges it with its own registers and re-zeroes the
-            // counter.  One partial per split block is written and read.
-            uint32_t* flag = reinterpret_cast<uint32_t*>(lds + kGBuf * kGTile);
-            if (tid == 0) flag[0] = __hip_atomic_fetch_add(&ctr[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __syncthreads();
-            const uint32_t arrived = flag[0];
-            rot = __builtin_amdgcn_make_buffer_rsrc(part + (size_t)unit * kGSlotFloats, 0, kGSlotFloats * 4, 0x00020000);
-            if (arrived == 0) {
+    }
+    // ---- merge the KP key parts of each column group: every wave scales its O
+    // to the group's maximum, then halves are exchanged until each wave holds
+    // the sum over the parts of its own QB dim blocks
+    l += shfl_xor(l, 32);
+    int ln = threadIdx.x & 63;
+    asm volatile("" : "+v"(ln));
+    float* const ms = reinterpret_cast<float*>(lds + 4 * kGTile);
+    __syncthreads();   // the tiles are no longer read
+    ms[w * 64 + ln] = m;
+    ms[512 + w * 64 + ln] = l;
+    __syncthreads();
+    float M = kNoKey, lt = 0.f;
 #pragma unroll
-                for (int db = 0; db < DB; db++)
+    for (int p = 0; p < KP; p++) M = fmaxf(M, ms[(p * CG + cg) * 64 + ln]);
 #pragma unroll
-                    for (int g4 = 0; g4 < 4; g4++) {
-                        const float4 v4 =
-                            make_float4(o[db][4 * g4], o[db][4 * g4 + 1], o[db][4 * g4 + 2], o[db][4 * g4 + 3]);
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v4), rot,
-                                                               (((w * DB + db) * 4 + g4) * 256 + ln * 4) * 4, 0, kSc1);
-                    }
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m), rot,
-                                                      (8 * 128 * 64 + w * 128 + ln) * 4, 0, kSc1);
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l), rot,
-                                                      (8 * 128 * 64 + w * 128 + 64 + ln) * 4, 0, kSc1);
-                __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's part of the partial is stored
-                __syncthreads();
-                if (tid == 0) __hip_atomic_fetch_add(&ctr[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                break;   // the other workgroup finishes this block (its segment is the last)
+    for (int p = 0; p < KP; p++)
+        lt += ms[512 + (p * CG + cg) * 64 + ln] * __builtin_amdgcn_exp2f(ms[(p * CG + cg) * 64 + ln] - M);
+    const float al = __builtin_amdgcn_exp2f(m - M);
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[db][e] *= al;
+    float4* const xch = reinterpret_cast<float4*>(lds);
+#pragma unroll
+    for (int n = DB / 2, bit = KP / 2; bit >= 1; n /= 2, bit /= 2) {
+        // partner: the wave of part kp ^ bit; this wave keeps blocks [0, n) of
+        // its current 2n when its bit is clear, [n, 2n) otherwise
+        const bool up = (kp & bit) != 0;
+        const int mate = (kp ^ bit) * CG + cg;
+#pragma unroll
+        for (int db = 0; db < n; db++)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++) {
+                float4 snd;
+                snd.x = up ? o[db][4 * g4] : o[n + db][4 * g4];
+                snd.y = up ? o[db][4 * g4 + 1] : o[n + db][4 * g4 + 1];
+                snd.z = up ? o[db][4 * g4 + 2] : o[n + db][4 * g4 + 2];
+                snd.w = up ? o[db][4 * g4 + 3] : o[n + db][4 * g4 + 3];
+                xch[((w * n + db) * 4 + g4) * 64 + ln] = snd;
             }
-            if (tid == 0) {
-                // bounded: the first workgroup only has its stores left
-                uint32_t c = arrived + 1;
-                for (int it = 0; c != 3 && it < (1 << 22); it++) {
-                    __builtin_amdgcn_s_sleep(2);
-                    c = __hip_atomic_load(&ctr[unit], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                __hip_atomic_store(&ctr[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-            have_other = true;
-            const float m1 = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(rot, (8 * 128 * 64 + w * 128 + ln) * 4, 0, kSc1));
-            const float l1 = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(rot, (8 * 128 * 64 + w * 128 + 64 + ln) * 4, 0, kSc1));
-            const float M = fmaxf(m, m1);
-            a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
-            a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M);
-            {
-#pragma clang fp contract(off)
-                inv = 1.0f / (l * a0 + l1 * a1);
-            }
-        } else {
-            inv = 1.0f / l;
-        }
-        if (erow < S) {
-            // o[db][e] = output dim 32 db + 8 (e / 4) + 4 h + e % 4 of row erow.
-            // The other partial's values and the gate logits of column block
-            // db + 1 are requested before the stores of block db: issued after
-            // them, each request would wait for those stores (the output may
-            // alias them as far as the compiler knows).
-            const float* grow = GATE ? gate + (size_t)erow * gtok + (size_t)h * ghead : nullptr;
-            auto fetch = [&](int db, float4 (&ov)[4], float4 (&gv)[4]) __attribute__((always_inline)) {
+        __syncthreads();
 #pragma unroll
-                for (int g4 = 0; g4 < 4; g4++) {
-                    const int dd = 32 * db + 8 * g4 + 4 * eh;
-                    ov[g4] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    gv[g4] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (have_other)
-                        ov[g4] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                rot, (((w * DB + db) * 4 + g4) * 256 + ln * 4) * 4, 0, kSc1));
-                    if constexpr (GATE)   // (rows of any stride: four dword loads)
-                        gv[g4] = make_float4(grow[dd], grow[dd + 1], grow[dd + 2], grow[dd + 3]);
-                }
-            };
-            float4 ovn[4], gvn[4];
-            fetch(0, ovn, gvn);
+        for (int db = 0; db < n; db++)
 #pragma unroll
-            for (int db = 0; db < DB; db++) {
-                float4 ovc[4], gvc[4];
+            for (int g4 = 0; g4 < 4; g4++) {
+                const float4 r = xch[((mate * n + db) * 4 + g4) * 64 + ln];
 #pragma unroll
-                for (int g4 = 0; g4 < 4; g4++) {
-                    ovc[g4] = ovn[g4];
-                    gvc[g4] = gvn[g4];
-                }
-                if (db + 1 < DB) fetch(db + 1, ovn, gvn);
-#pragma unroll
-                for (int g4 = 0; g4 < 4; g4++) {
-                    const int dd = 32 * db + 8 * g4 + 4 * eh;
-                    const size_t off = ((size_t)erow * Hq + h) * D + dd;
-                    const float4 ov = ovc[g4];
-                    float v0, v1, v2, v3;
-                    {
-                        // Either workgroup of a split block may be the one that
-                        // merges: products rounded separately keep the sum
-                        // symmetric in the two partials, so a row's bits do not
-                        // depend on which finished second.
-#pragma clang fp contract(off)
-                        v0 = (o[db][4 * g4] * a0 + ov.x * a1) * inv;
-                        v1 = (o[db][4 * g4 + 1] * a0 + ov.y * a1) * inv;
-                        v2 = (o[db][4 * g4 + 2] * a0 + ov.z * a1) * inv;
-                        v3 = (o[db][4 * g4 + 3] * a0 + ov.w * a1) * inv;
-                    }
-                    if constexpr (GATE) {
-                        const float4 gl = gvc[g4];
-                        v0 = v0 / (1.0f + expf(-gl.x));
-                        v1 = v1 / (1.0f + expf(-gl.y));
-                        v2 = v2 / (1.0f + expf(-gl.z));
-                        v3 = v3 / (1.0f + expf(-gl.w));
-                    }
-                    if (OUT16) {
-                        half4 hv = {(_Float16)v0, (_Float16)v1, (_Float16)v2, (_Float16)v3};
-                        *reinterpret_cast<half4*>(static_cast<_Float16*>(out) + off) = hv;
-                    } else {
-                        *reinterpret_cast<float4*>(static_cast<float*>(out) + off) = make_float4(v0, v1, v2, v3);
-                    }
+                for (int i = 0; i < 4; i++) {
+                    const float rv4 = i == 0 ? r.x : i == 1 ? r.y : i == 2 ? r.z : r.w;
+                    const float kept = up ? o[n + db][4 * g4 + i] : o[db][4 * g4 + i];
+                    // the sum of two parts is the same whichever wave forms it
+                    o[db][4 * g4 + i] = kept + rv4;
                 }
             }
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // stores retired before the stream's counted waits resume
+        __syncthreads();
+    }
+    // this wave holds dim blocks QB * b .. + QB - 1 with b = kp (its bits high to low)
+    const int tok = tok0 + ((ln & 31) >> 2), h = kvh * 4 + (ln & 3), eh = ln >> 5;
+    if (steps <= a.sps) {
+        if (tok >= a.S) return;
+        const float inv = 1.0f / lt;
+#pragma unroll
+        for (int j = 0; j < QB; j++)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++)
+                split_store<OUT16, GATE>(a.out, a.gate, a.gtok, a.ghead, tok, h, a.Hq,
+                                         32 * (QB * kp + j) + 8 * g4 + 4 * eh,
+                                         make_float4(o[j][4 * g4], o[j][4 * g4 + 1], o[j][4 * g4 + 2], o[j][4 * g4 + 3]),
+                                         inv);
+        return;
+    }
+    float* rec = a.rec + ((size_t)(kvh * a.ngrp + grp) * a.parts + part) * split_rec_floats<KP>();
+#pragma unroll
+    for (int j = 0; j < QB; j++)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++)
+            reinterpret_cast<float4*>(rec)[((w * QB + j) * 4 + g4) * 64 + ln] =
+                make_float4(o[j][4 * g4], o[j][4 * g4 + 1], o[j][4 * g4 + 2], o[j][4 * g4 + 3]);
+    if (kp == 0 && ln < 32) {
+        float* ml = rec + 8 * QB * 4 * 256;
+        ml[cg * 32 + ln] = M;
+        ml[CG * 32 + cg * 32 + ln] = lt;
     }
 }
 
-int launch_prefill_g4(void* out, bool out16, const void* q, const void* k, const void* v, int S, int L, int qoff,
-                      int Hq, int Hkv, const float* gate, int gtok, int ghead, hipStream_t st) {
-    constexpr int D = 256;
-    ANELM_REQUIRE((size_t)L * Hkv * D * 2 < 0x7fffffffu, "prefill: %d keys exceed the 2 GiB buffer range", L);
-    const int nb = (S + 63) / 64, upk = nb / 2 + (nb & 1), units = Hkv * upk;
-    const size_t part_bytes = (size_t)units * kGSlotFloats * sizeof(float);
-    float* part = static_cast<float*>(workspace(part_bytes, st));
-    if (!part) return ANELM_ENOMEM;
-    uint32_t* ctr = counters(units, kCtrPrefill, st);   // zeroed; each call leaves them zeroed
-    if (!ctr) return ANELM_ERANGE;
-    // the gated launches (prompt prefill through the layer core) are their own
-    // instantiation: the bare core carries no gate code
-    using K = void (*)(void*, const _Float16*, const _Float16*, const _Float16*, float*, uint32_t*, int, int, int,
-                       int, int, const float*, int, int);
-    static const K kern[2][2] = {{prefill_g4_kernel<false, false>, prefill_g4_kernel<false, true>},
-                                 {prefill_g4_kernel<true, false>, prefill_g4_kernel<true, true>}};
-    static bool attr_set = false;
-    if (!attr_set) {
+// Merge of a group's part records: workgroup (group of a kv head, float4 slot
+// of the wave's 4 QB), thread = (wave, lane) of the kernel above; the parts'
+// values are requested kCombineAhead at a time.
+constexpr int kCombineAhead = 8;
+template <int KP, bool OUT16, bool GATE>
+__global__ __launch_bounds__(kGNT) void prefill_split_combine(const SplitArgs a) {
+    constexpr int CG = 8 / KP, QB = 8 / KP, REC = split_rec_floats<KP>();
+    const int w = threadIdx.x >> 6, ln = threadIdx.x & 63, cg = w % CG, kp = w / CG;
+    const int kvh = blockIdx.x / a.ngrp, grp = blockIdx.x % a.ngrp, slot = blockIdx.y;
+    const int steps = split_steps(KP, grp, a.S, a.qoff), np = (steps + a.sps - 1) / a.sps;
+    const int tok = grp * (64 / KP) + 8 * cg + ((ln & 31) >> 2);
+    if (np <= 1 || tok >= a.S) return;
+    const float* base = a.rec + (size_t)(kvh * a.ngrp + grp) * a.parts * REC;
+    const float* ml = base + 8 * QB * 4 * 256 + cg * 32 + (ln & 31);
+    const float4* ov = reinterpret_cast<const float4*>(base) + (w * QB * 4 + slot) * 64 + ln;
+    float M = kNoKey, lt = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p0 = 0; p0 < np; p0 += kCombineAhead) {
+        float4 x[kCombineAhead];
+        float pm[kCombineAhead], pl[kCombineAhead];
+#pragma unroll
+        for (int i = 0; i < kCombineAhead; i++) {
+            const int p = min(p0 + i, np - 1);
+            x[i] = ov[(size_t)p * (REC / 4)];
+            pm[i] = ml[(size_t)p * REC];
+            pl[i] = p0 + i < np ? ml[(size_t)p * REC + CG * 32] : 0.f;
+            if (p0 + i >= np) pm[i] = kNoKey;
+        }
+        float Mn = M;
+#pragma unroll
+        for (int i = 0; i < kCombineAhead; i++) Mn = fmaxf(Mn, pm[i]);
+        const float sc = __builtin_amdgcn_exp2f(M - Mn);
+        lt *= sc;
+        acc = make_float4(acc.x * sc, acc.y * sc, acc.z * sc, acc.w * sc);
+#pragma unroll
+        for (int i = 0; i < kCombineAhead; i++) {
+            // (a part without keys for this column: m = kNoKey, l = 0, O = 0)
+            const float f = p0 + i < np ? __builtin_amdgcn_exp2f(pm[i] - Mn) : 0.f;
+            lt += pl[i] * f;
+            acc.x += x[i].x * f;
+            acc.y += x[i].y * f;
+            acc.z += x[i].z * f;
+            acc.w += x[i].w * f;
+        }
+        M = Mn;
+    }
+    split_store<OUT16, GATE>(a.out, a.gate, a.gtok, a.ghead, tok, kvh * 4 + (ln & 3), a.Hq,
+                             32 * (QB * kp + slot / 4) + 8 * (slot % 4) + 4 * (ln >> 5), acc, 1.0f / lt);
+}
+
+// How a prompt is cut: the least estimated time over both KP and 1 .. 16 parts
+// of the longest group.  From sweeps of both (us): a step takes 1.9 (KP 2) or
+// 2.8 (KP 4, half the tokens over twice the keys), a workgroup 9 besides; more
+// workgroups than compute units run one after another (the longest first, so
+// half of one is the tail); parts cost a second launch of 4.5 and 0.35 per MB
+// of records.  Measured against the model, layer prologue taken off: 777
+// tokens behind 1500 keys 2 kv heads, KP 2: 5 parts 38 (38), 2 parts 49 (52);
+// 4096 tokens 4 kv heads KP 2 184 (194), KP 4 233 (238); 1000 tokens KP 4 34
+// (31), KP 2 43 (39); 2000 tokens KP 2 in 2 parts 77 (77).
+struct SplitPlan {
+    int kp, ngrp, parts, sps;
+};
+
+SplitPlan plan_split(int S, int qoff, int Hkv, int cus) {
+    SplitPlan best{0, 0, 0, 0};
+    float best_us = 0.f;
+    for (int kp = 2; kp <= 4; kp += 2) {
+        const int tok = 64 / kp, ngrp = (S + tok - 1) / tok, most = split_steps(kp, ngrp - 1, S, qoff);
+        int last = 0;
+        for (int p = 1; p <= 16; p++) {
+            const int sps = (most + p - 1) / p;
+            if (sps == last) continue;
+            last = sps;
+            const int parts = (most + sps - 1) / sps;
+            if (parts > 1 && (long)Hkv * ngrp * parts > 2L * cus) break;   // (records: 64 MB on 256 CUs)
+            long wgs = 0, steps = 0, recs = 0;
+            for (int g = 0; g < ngrp; g++) {
+                const int n = split_steps(kp, g, S, qoff), np = (n + sps - 1) / sps;
+                steps += n;
+                wgs += np;
+                if (np > 1) recs += np;
+            }
+            const float load = wgs * Hkv <= cus ? (float)sps
+                                                : (float)(steps * Hkv) / (float)cus + 0.5f * (float)sps;
+            float us = 9.f + load * (kp == 2 ? 1.9f : 2.8f);
+            if (parts > 1) us += 4.5f + 0.35f * (float)(recs * Hkv) * (kp == 2 ? 0.131f : 0.066f);
+            if (best.kp == 0 || us < best_us) best = SplitPlan{kp, ngrp, parts, sps}, best_us = us;
+        }
+    }
+    return best;
+}
+
+template <int KP>
+int launch_split(const SplitArgs& a, bool out16, hipStream_t st) {
+    using K = void (*)(const SplitArgs);
+    static const K kern[2][2] = {{prefill_split_kernel<KP, false, false>, prefill_split_kernel<KP, false, true>},
+                                 {prefill_split_kernel<KP, true, false>, prefill_split_kernel<KP, true, true>}};
+    static const K comb[2][2] = {{prefill_split_combine<KP, false, false>, prefill_split_combine<KP, false, true>},
+                                 {prefill_split_combine<KP, true, false>, prefill_split_combine<KP, true, true>}};
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set.load(std::memory_order_acquire)) {
         for (int o = 0; o < 2; o++)
             for (int g = 0; g < 2; g++)
                 ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern[o][g]),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kGLds));
-        attr_set = true;
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, split_lds<KP>()));
+        attr_set.store(true, std::memory_order_release);
     }
-    const _Float16* qh = static_cast<const _Float16*>(q);
-    const _Float16* kh = static_cast<const _Float16*>(k);
-    const _Float16* vh = static_cast<const _Float16*>(v);
-    const dim3 grid(2 * units);
-    hipLaunchKernelGGL(kern[out16 ? 1 : 0][gate != nullptr ? 1 : 0], grid, dim3(kGNT), kGLds, st, out, qh, kh, vh,
-                       part, ctr, S, L, qoff, Hq, Hkv, gate, gtok, ghead);
-    ANELM_LAUNCHED("prefill_g4_kernel");
+    const int o = out16 ? 1 : 0, g = a.gate != nullptr ? 1 : 0, bpk = a.ngrp * a.parts;
+    const int spx = 8 % a.Hkv == 0 ? 8 / a.Hkv : 1;
+    const dim3 grid(8 % a.Hkv == 0 ? (bpk + spx - 1) / spx * 8 : bpk * a.Hkv);
+    hipLaunchKernelGGL(kern[o][g], grid, dim3(kGNT), split_lds<KP>(), st, a);
+    ANELM_LAUNCHED("prefill_split_kernel");
+    if (a.parts > 1) {
+        hipLaunchKernelGGL(comb[o][g], dim3(a.ngrp * a.Hkv, 4 * (8 / KP)), dim3(kGNT), 0, st, a);
+        ANELM_LAUNCHED("prefill_split_combine");
+    }
     return ANELM_OK;
 }
 
+int launch_prefill_split(void* out, bool out16, const void* q, const KeyRing& rg, int S, int L, int qoff, int Hq,
+                      int Hkv, const float* gate, int gtok, int ghead, hipStream_t st) {
+    ANELM_REQUIRE((size_t)rg.cap * Hkv * 512 < 0x7fffffffu, "prefill: %d keys exceed the 2 GiB buffer range", rg.cap);
+    Device* dev = device();
+    if (!dev) return ANELM_EHIP;
+    const SplitPlan sp = plan_split(S, qoff, Hkv, dev->num_cus);
+    SplitArgs a{out, static_cast<const _Float16*>(q), rg, nullptr, gate, S, L, qoff, Hq, Hkv, gtok, ghead,
+                sp.ngrp, sp.parts, sp.sps};
+    if (sp.parts > 1) {
+        const size_t rec = sp.kp == 2 ? split_rec_floats<2>() : split_rec_floats<4>();
+        a.rec = static_cast<float*>(workspace((size_t)Hkv * sp.ngrp * sp.parts * rec * sizeof(float), st));
+        if (!a.rec) return ANELM_ENOMEM;
+    }
+    return sp.kp == 2 ? launch_split<2>(a, out16, st) : launch_split<4>(a, out16, st);
+}
+
 template <int D, int HB, int RB>
-int launch_prefill(void* out, bool out16, const void* q, const void* k, const void* v, int S, int L, int qoff,
+int launch_prefill(void* out, bool out16, const void* q, const KeyRing& rg, int S, int L, int qoff,
                    int win, int Hq, int Hkv, const float* gate, int gtok, int ghead, hipStream_t st) {
     const int rows = 32 * RB;
     dim3 grid((S + rows - 1) / rows, Hq / HB), block(HB * RB * 64);
     const _Float16* qh = static_cast<const _Float16*>(q);
-    const _Float16* kh = static_cast<const _Float16*>(k);
-    const _Float16* vh = static_cast<const _Float16*>(v);
     if (out16)
-        hipLaunchKernelGGL((prefill_kernel<D, HB, RB, true>), grid, block, 0, st, out, qh, kh, vh, S, L, qoff, win,
+        hipLaunchKernelGGL((prefill_kernel<D, HB, RB, true>), grid, block, 0, st, out, qh, rg, S, L, qoff, win,
                            Hq, Hkv, gate, gtok, ghead);
     else
-        hipLaunchKernelGGL((prefill_kernel<D, HB, RB, false>), grid, block, 0, st, out, qh, kh, vh, S, L, qoff, win,
+        hipLaunchKernelGGL((prefill_kernel<D, HB, RB, false>), grid, block, 0, st, out, qh, rg, S, L, qoff, win,
                            Hq, Hkv, gate, gtok, ghead);
     ANELM_LAUNCHED("prefill_kernel");
     return ANELM_OK;
 }
 
 template <int D>
-int dispatch_g(void* out, bool out16, const void* q, const void* k, const void* v, int S, int L, int qoff, int win,
+int dispatch_g(void* out, bool out16, const void* q, const KeyRing& rg, int S, int L, int qoff, int win,
                int Hq, int Hkv, const float* gate, int gtok, int ghead, hipStream_t st) {
     switch (Hq / Hkv) {
-        case 1: return launch_prefill<D, 1, 8>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
-        case 2: return launch_prefill<D, 2, 4>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+        case 1: return launch_prefill<D, 1, 8>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+        case 2: return launch_prefill<D, 2, 4>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
         case 4:
             // the pipelined kernel walks every key from 0: no window
             if (D == 256 && win == 0)
-                return launch_prefill_g4(out, out16, q, k, v, S, L, qoff, Hq, Hkv, gate, gtok, ghead, st);
-            return launch_prefill<D, 4, 2>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
-        case 8: return launch_prefill<D, 4, 2>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+                return launch_prefill_split(out, out16, q, rg, S, L, qoff, Hq, Hkv, gate, gtok, ghead, st);
+            return launch_prefill<D, 4, 2>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+        case 8: return launch_prefill<D, 4, 2>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
         default: return set_error(ANELM_EINVAL, "prefill: n_heads/n_kv_heads = %d unsupported", Hq / Hkv);
     }
 }
 
 }  // namespace
 
-int prefill_core(void* out, bool out16, const uint16_t* q, const uint16_t* k, const uint16_t* v, int S, int L,
-                 int qoff, int win, int Hq, int Hkv, int D, const float* gate, int gtok, int ghead, hipStream_t st) {
+int prefill_core(void* out, bool out16, const uint16_t* q, const uint16_t* k, const uint16_t* v, int start, int cap,
+                 int S, int L, int qoff, int win, int Hq, int Hkv, int D, const float* gate, int gtok, int ghead,
+                 hipStream_t st) {
+    ANELM_REQUIRE(L <= cap && start >= 0 && start < cap, "prefill: %d keys in a ring of %d from %d", L, cap, start);
+    const KeyRing rg{reinterpret_cast<const _Float16*>(k), reinterpret_cast<const _Float16*>(v), start, cap};
     switch (D) {
-        case 128: return dispatch_g<128>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
-        case 256: return dispatch_g<256>(out, out16, q, k, v, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+        case 128: return dispatch_g<128>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
+        case 256: return dispatch_g<256>(out, out16, q, rg, S, L, qoff, win, Hq, Hkv, gate, gtok, ghead, st);
         default: return set_error(ANELM_EINVAL, "prefill: head_dim %d unsupported (128, 256)", D);
     }
 }
@@ -634,6 +789,6 @@ extern "C" int anelm_attn_prefill(void* out, int out_dtype, const uint16_t* q, c
     ANELM_REQUIRE(n_kv_heads > 0 && n_heads % n_kv_heads == 0, "prefill: heads %d/%d", n_heads,
                   n_kv_heads);
     ANELM_REQUIRE(out_dtype == ANELM_F32 || out_dtype == ANELM_F16, "prefill: out_dtype %d", out_dtype);
-    return prefill_core(out, out_dtype == ANELM_F16, q, k, v, S, S, 0, 0, n_heads, n_kv_heads, head_dim, nullptr, 0,
+    return prefill_core(out, out_dtype == ANELM_F16, q, k, v, 0, S, S, S, 0, 0, n_heads, n_kv_heads, head_dim, nullptr, 0,
                         0, as_stream(stream));
 }

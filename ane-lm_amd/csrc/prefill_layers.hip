@@ -6,14 +6,14 @@
 //
 // Full attention (qwen3_5.cpp:944-1002 per token):
 //   1. prep: per (token, head) row, q/k RMSNorm and RoPE at the token's
-//      position; q to fp16, the new keys and values to fp16 behind the
-//      cached keys (gathered oldest to newest from the ring), so keys are
-//      one contiguous sequence [cached | prompt];
-//   2. the causal MFMA core over that sequence, query row t being key
-//      len0 + t, with the output gate in its epilogue; when the ring would
-//      overflow inside the prompt, row t sees only the last `capacity` keys,
-//      as the sliding ring gives the decode core;
-//   3. the prompt's keys that survive in the ring are written to their slots.
+//      position; q to fp16, the new keys and values to fp16 in their ring
+//      slots behind the cached keys;
+//   2. the causal MFMA core over the ring's keys, query row t being key
+//      len0 + t, with the output gate in its epilogue.
+//   When the ring would overflow inside the prompt, the cached keys are first
+//   gathered oldest to newest into one sequence [cached | prompt], row t sees
+//   only its last `capacity` keys, as the sliding ring gives the decode core,
+//   and the prompt's keys that survive are written to their slots at the end.
 // Gated DeltaNet (qwen3_5.cpp:849-908 per token):
 //   1. the causal conv1d over [conv ring | prompt] + SiLU per channel
 //      (cpu_ops.cpp:89-129, :6-13), split into q / k / v, with z, a, b
@@ -38,85 +38,140 @@ struct PrepArgs {
     const float* rope_tab;     // [rope_rows][2 rot_pairs] or null
     int rope_rows;
     uint16_t* qh;              // [S][Hq][D] fp16
-    uint16_t* kall;            // [len0 + S][Hkv][D] fp16
-    uint16_t* vall;
-    int S, Hq, Hkv, len0, pos0, rot_pairs, rope_mode;
+    uint16_t* kd;              // token t's keys (values in vd) at row (row0 + t) mod cap of [cap][Hkv][D]
+    uint16_t* vd;
+    int row0, cap;
+    int S, Hq, Hkv, pos0, rot_pairs, rope_mode;
     float theta, eps;
 };
 
-// One wave per (token, row), four rows of one token per workgroup (the
-// token's RoPE row is loaded once for them): rows 0..Hq-1 are the token's q
-// heads, the rest its kv heads (with the value row converted alongside).  The
-// norm and the rotation are the decode core's (models/llm/qwen3_5.cpp:952-971):
-// (x * inv) * w with inv = 1 / sqrtf(ss / D + eps), pairs rotated without
-// contraction.
-constexpr int kPrepRowsPerWg = 4;
-template <int D>
-__global__ __launch_bounds__(64 * kPrepRowsPerWg) void prefill_prep_kernel(PrepArgs a) {
-    __shared__ float rows[kPrepRowsPerWg][D];
-    __shared__ float cs[128], sn[128];
-    const int t = blockIdx.x, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int y = blockIdx.y * kPrepRowsPerWg + wv;
-    const bool live = y < a.Hq + a.Hkv;   // (a wave past the last row still meets the barriers)
-    const int pos = a.pos0 + t;
-    for (int j = threadIdx.x; j < a.rot_pairs; j += 64 * kPrepRowsPerWg) {
-        if (a.rope_tab != nullptr && pos < a.rope_rows) {
-            cs[j] = a.rope_tab[(size_t)pos * 2 * a.rot_pairs + j];
-            sn[j] = a.rope_tab[(size_t)pos * 2 * a.rot_pairs + a.rot_pairs + j];
-        } else {
-            // the table's formula (cpu_ops.cpp:51-55) evaluated here
-            const float freq = 1.0f / powf(a.theta, (float)(2 * j) / (float)(2 * a.rot_pairs));
-            const float angle = (float)pos * freq;
-            cs[j] = cosf(angle);
-            sn[j] = sinf(angle);
-        }
+// cos / sin of rotation pair j at position pos: the table's row, or its
+// formula (cpu_ops.cpp:51-55) evaluated here past the table.
+__device__ __forceinline__ void prep_cs(const PrepArgs& a, int pos, int j, float& c, float& s) {
+    if (a.rope_tab != nullptr && pos < a.rope_rows) {
+        c = a.rope_tab[(size_t)pos * 2 * a.rot_pairs + j];
+        s = a.rope_tab[(size_t)pos * 2 * a.rot_pairs + a.rot_pairs + j];
+    } else {
+        const float freq = 1.0f / powf(a.theta, (float)(2 * j) / (float)(2 * a.rot_pairs));
+        const float angle = (float)pos * freq;
+        c = cosf(angle);
+        s = sinf(angle);
     }
+}
+
+template <int E> struct Row;   // E = D / 64 consecutive elements of a row
+template <> struct Row<4> {
+    typedef float4 F;
+    typedef uint2 H;
+    static __device__ __forceinline__ void get(float (&x)[4], F v) { x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w; }
+};
+template <> struct Row<2> {
+    typedef float2 F;
+    typedef uint32_t H;
+    static __device__ __forceinline__ void get(float (&x)[2], F v) { x[0] = v.x, x[1] = v.y; }
+};
+
+// One wave per row, four rows of one token per workgroup: rows 0..Hq-1 are
+// the token's q heads, the rest its kv heads (with the value row converted
+// alongside).  The norm and the rotation are the decode core's
+// (models/llm/qwen3_5.cpp:952-971): (x * inv) * w with inv = 1 / sqrtf(ss / D
+// + eps), pairs rotated without contraction.  Lane l holds elements E l ..
+// E l + E - 1: a row is one load and one store per lane (VEC: rows and
+// weights aligned to it; otherwise E dword loads), interleaved pairs stay in
+// the lane and half-split pairs are rot_pairs / E lanes apart, so no row
+// passes through LDS.  Bound: memory (4096 tokens 16q/4kv move 150 MB in 30 us;
+// with dword loads and rows through LDS 33, and 6.4 more for the keys' second
+// copy into the ring).
+constexpr int kPrepRowsPerWg = 4;
+template <int D, bool VEC>
+__global__ __launch_bounds__(64 * kPrepRowsPerWg) void prefill_prep_kernel(PrepArgs a) {
+    constexpr int E = D / 64;
+    typedef Row<E> R;
+    const int t = blockIdx.x, lane = threadIdx.x & 63;
+    const int y = blockIdx.y * kPrepRowsPerWg + (threadIdx.x >> 6);
+    if (y >= a.Hq + a.Hkv) return;
+    const int pos = a.pos0 + t;
     const bool isq = y < a.Hq;
     const int kvh = y - a.Hq;
-    float* row = rows[wv];
-    constexpr int E = D / 64;
     float x[E], vv[E];
-    if (live) {
-        const float* src = isq ? a.q_gate + t * a.qs + (long)y * 2 * D : a.k + t * a.ks + (long)kvh * D;
-        const float* w = isq ? a.q_norm_w : a.k_norm_w;
+    auto load = [&](const float* p, float (&o)[E]) __attribute__((always_inline)) {
+        if constexpr (VEC) {
+            R::get(o, *reinterpret_cast<const typename R::F*>(p + E * lane));
+        } else {
 #pragma unroll
-        for (int e = 0; e < E; e++) x[e] = src[lane + 64 * e];
-        if (!isq) {
-            const float* vs = a.v + t * a.ks + (long)kvh * D;
-#pragma unroll
-            for (int e = 0; e < E; e++) vv[e] = vs[lane + 64 * e];
+            for (int e = 0; e < E; e++) o[e] = p[E * lane + e];
         }
-        if (w != nullptr) {
-            float ss = 0.f;
+    };
+    load(isq ? a.q_gate + t * a.qs + (long)y * 2 * D : a.k + t * a.ks + (long)kvh * D, x);
+    if (!isq) load(a.v + t * a.ks + (long)kvh * D, vv);
+    const float* w = isq ? a.q_norm_w : a.k_norm_w;
+    if (w != nullptr) {
+        float wv[E];
+        load(w, wv);
+        float ss = 0.f;
 #pragma unroll
-            for (int e = 0; e < E; e++) ss += x[e] * x[e];
-            ss = wave_sum(ss);
-            const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
+        for (int e = 0; e < E; e++) ss += x[e] * x[e];
+        ss = wave_sum(ss);
+        const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
 #pragma unroll
-            for (int e = 0; e < E; e++) x[e] = (x[e] * inv) * w[lane + 64 * e];
+        for (int e = 0; e < E; e++) x[e] = (x[e] * inv) * wv[e];
+    }
+    const int rp = a.rot_pairs;
+    if (a.rope_mode == ANELM_ROPE_INTERLEAVED) {
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+            const int j = (E * lane + e) / 2;
+            if (j < rp) {
+                float c, s;
+                prep_cs(a, pos, j, c, s);
+                const float v0 = x[e], v1 = x[e + 1];
+                rotate_pair(x[e], x[e + 1], v0, v1, c, s);
+            }
+        }
+    } else {
+        // element i's mate is i + rp (i < rp) or i - rp (rp <= i < 2 rp)
+        float mate[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int i = E * lane + e, mi = i < rp ? i + rp : i < 2 * rp ? i - rp : i;
+            mate[e] = 0.f;
+#pragma unroll
+            for (int u = 0; u < E; u++) {
+                const float got = __shfl(x[u], mi / E, 64);
+                if (mi % E == u) mate[e] = got;
+            }
         }
 #pragma unroll
-        for (int e = 0; e < E; e++) row[lane + 64 * e] = x[e];
-    }
-    __syncthreads();
-    if (live) {
-        for (int j = lane; j < a.rot_pairs; j += 64) {
-            const int i0 = a.rope_mode == 0 ? 2 * j : j;
-            const int i1 = a.rope_mode == 0 ? 2 * j + 1 : j + a.rot_pairs;
-            const float v0 = row[i0], v1 = row[i1];
-            rotate_pair(row[i0], row[i1], v0, v1, cs[j], sn[j]);
+        for (int e = 0; e < E; e++) {
+            const int i = E * lane + e;
+            if (i >= 2 * rp) continue;
+            const bool lo = i < rp;
+            float c, s, o0, o1;
+            prep_cs(a, pos, lo ? i : i - rp, c, s);
+            rotate_pair(o0, o1, lo ? x[e] : mate[e], lo ? mate[e] : x[e], c, s);
+            x[e] = lo ? o0 : o1;
         }
     }
-    __syncthreads();
-    if (!live) return;
-    uint16_t* dst = isq ? a.qh + ((size_t)t * a.Hq + y) * D : a.kall + ((size_t)(a.len0 + t) * a.Hkv + kvh) * D;
+    auto store = [&](uint16_t* p, const float (&o)[E]) __attribute__((always_inline)) {
+        typename R::H h;   // (destination rows are this library's or cache rows of 2 D bytes)
+        uint16_t* hp = reinterpret_cast<uint16_t*>(&h);
 #pragma unroll
-    for (int e = 0; e < E; e++) dst[lane + 64 * e] = f2h(row[lane + 64 * e]);
-    if (!isq) {
-        uint16_t* vd = a.vall + ((size_t)(a.len0 + t) * a.Hkv + kvh) * D;
+        for (int e = 0; e < E; e++) hp[e] = f2h(o[e]);
+        if constexpr (VEC) {
+            *reinterpret_cast<typename R::H*>(p + E * lane) = h;
+        } else {
 #pragma unroll
-        for (int e = 0; e < E; e++) vd[lane + 64 * e] = f2h(vv[e]);
+            for (int e = 0; e < E; e++) p[E * lane + e] = hp[e];
+        }
+    };
+    if (isq) {
+        store(a.qh + ((size_t)t * a.Hq + y) * D, x);
+        return;
     }
+    const int at = a.row0 + t;
+    const size_t row = (size_t)(at - (at >= a.cap ? a.cap : 0)) * a.Hkv + kvh;
+    store(a.kd + row * D, x);
+    store(a.vd + row * D, vv);
 }
 
 // Cached keys and values oldest to newest: key i of the ring is slot
@@ -292,36 +347,53 @@ extern "C" int anelm_full_attn_prefill(float* out, const float* q_gate, const fl
     ANELM_REQUIRE(L * n_kv_heads * D * 2 < 0x7fffffffL && (long)S * n_heads * D * 2 < 0x7fffffffL,
                   "full_attn_prefill: %ld keys exceed the 2 GiB buffer range", L);
     hipStream_t st = as_stream(stream);
+    // While the ring holds every key of [cached | prompt] (and its bytes are in
+    // a buffer's range) the core reads the ring itself, and the prologue writes
+    // the prompt's keys straight to their slots (free ones: L <= cap).  Once it
+    // overflows inside the prompt, early rows still see keys that later ones
+    // overwrite: the keys are gathered into one sequence, and those that
+    // survive are written to the ring afterwards.
+    const bool direct = L <= cap && (size_t)cap * n_kv_heads * D * 2 < 0x7fffffffu;
     const size_t qb = ((size_t)S * n_heads * D * 2 + 255) & ~(size_t)255;
-    const size_t kb = ((size_t)L * n_kv_heads * D * 2 + 255) & ~(size_t)255;
+    const size_t kb = direct ? 0 : ((size_t)L * n_kv_heads * D * 2 + 255) & ~(size_t)255;
     char* ws = static_cast<char*>(workspace2(qb + 2 * kb, st));
     if (!ws) return ANELM_ENOMEM;
     uint16_t* qh = reinterpret_cast<uint16_t*>(ws);
     uint16_t* kall = reinterpret_cast<uint16_t*>(ws + qb);
     uint16_t* vall = reinterpret_cast<uint16_t*>(ws + qb + kb);
     const int row16 = n_kv_heads * D / 8;
-    if (len0 > 0) {
+    if (!direct && len0 > 0) {
         const long n16 = (long)len0 * row16;
         hipLaunchKernelGGL(ring_gather_kernel, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, kall, vall,
                            k_cache, v_cache, n16, row16, start0, cap);
         ANELM_LAUNCHED("ring_gather_kernel");
     }
-    PrepArgs a{q_gate, k, v, qs, ks, q_norm_w, k_norm_w, rope_table, rope_table ? rope_rows : 0, qh, kall, vall,
-               S, n_heads, n_kv_heads, len0, pos0, rot_dim / 2, rope_mode, theta, eps};
+    PrepArgs a{q_gate, k, v, qs, ks, q_norm_w, k_norm_w, rope_table, rope_table ? rope_rows : 0, qh,
+               direct ? k_cache : kall, direct ? v_cache : vall,
+               direct ? (int)(((long)start0 + len0) % cap) : len0, direct ? cap : (int)L,
+               S, n_heads, n_kv_heads, pos0, rot_dim / 2, rope_mode, theta, eps};
     const dim3 pg(S, (n_heads + n_kv_heads + kPrepRowsPerWg - 1) / kPrepRowsPerWg);
-    if (D == 256) hipLaunchKernelGGL(prefill_prep_kernel<256>, pg, dim3(64 * kPrepRowsPerWg), 0, st, a);
-    else hipLaunchKernelGGL(prefill_prep_kernel<128>, pg, dim3(64 * kPrepRowsPerWg), 0, st, a);
+    // whole-row loads and stores: every row starts at a multiple of what a lane takes
+    auto at = [](const void* p, unsigned n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; };
+    const int E = D / 64;
+    const bool vec = qs % E == 0 && ks % E == 0 && at(q_gate, 4 * E) && at(k, 4 * E) && at(v, 4 * E) &&
+                     at(q_norm_w, 4 * E) && at(k_norm_w, 4 * E) && at(a.kd, 2 * E) && at(a.vd, 2 * E);
+    auto kern = D == 256 ? (vec ? prefill_prep_kernel<256, true> : prefill_prep_kernel<256, false>)
+                         : (vec ? prefill_prep_kernel<128, true> : prefill_prep_kernel<128, false>);
+    hipLaunchKernelGGL(kern, pg, dim3(64 * kPrepRowsPerWg), 0, st, a);
     ANELM_LAUNCHED("prefill_prep_kernel");
     // rows whose ring overflowed inside the prompt see the last `cap` keys
     const int win = L > cap ? cap : 0;
-    int rc = prefill_core(out, false, qh, kall, vall, S, (int)L, len0, win, n_heads, n_kv_heads, D,
-                          gate ? q_gate + D : nullptr, (int)qs, 2 * D, st);
+    int rc = prefill_core(out, false, qh, a.kd, a.vd, direct ? start0 : 0, direct ? cap : (int)L, S, (int)L, len0, win,
+                          n_heads, n_kv_heads, D, gate ? q_gate + D : nullptr, (int)qs, 2 * D, st);
     if (rc) return rc;
-    const int t0 = S > cap ? S - cap : 0;
-    const long n16 = (long)(S - t0) * row16;
-    hipLaunchKernelGGL(ring_write_kernel, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, k_cache, v_cache,
-                       kall, vall, n16, row16, t0, len0, start0, cap);
-    ANELM_LAUNCHED("ring_write_kernel");
+    if (!direct) {
+        const int t0 = S > cap ? S - cap : 0;
+        const long n16 = (long)(S - t0) * row16;
+        hipLaunchKernelGGL(ring_write_kernel, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, k_cache,
+                           v_cache, kall, vall, n16, row16, t0, len0, start0, cap);
+        ANELM_LAUNCHED("ring_write_kernel");
+    }
     if (L <= cap) {
         *cache_len = (int)L;
     } else {

@@ -127,6 +127,75 @@ def test_full_attn_prefill_4096_rows(anelm, orc, dev):
         assert_close(got[t], want, what=f"row {t}")
 
 
+@pytest.mark.parametrize("S,Hq,Hkv,cap,start,len0,rope_mode,pad,table_rows", [
+    (1, 8, 2, 64, 3, 0, 0, 0, 0),              # one token, nothing cached
+    (15, 8, 2, 4096, 4090, 4000, 0, 0, 4096),  # part-filled group, many key parts, wrap inside a tile
+    (17, 16, 4, 512, 500, 10, 1, 0, 512),      # one token past a group; wrap inside the prompt
+    (40, 16, 4, 64, 0, 10, 0, 1, 64),          # rows not 16-byte aligned; a column's first tile wholly masked
+    (33, 4, 1, 256, 255, 95, 1, 3, 20),        # one kv head; positions past the RoPE table
+    (24, 12, 3, 300, 7, 200, 0, 0, 300),       # kv heads that do not divide the XCDs
+    (500, 16, 4, 1024, 600, 300, 0, 0, 1024),  # several key parts of 16-token groups, wrapped ring
+    (2100, 16, 4, 4096, 0, 0, 0, 0, 4096),     # more workgroups than compute units
+])
+def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_mode, pad, table_rows):
+    """Head_dim 256 with 4 query heads per kv head at the edges of its token
+    groups, key tiles and key parts, reading the ring in place.  Against the
+    layer's formulas in float64 on the GPU, over q and new keys rounded to fp16
+    as the layer keeps them.  Each output row is a weighted mean of values whose
+    weights are fp16 (relative 2^-11), so its error is below the usual bar."""
+    D, rot, pos0 = 256, 64, len0 + 3
+    c = _attn_case(1900 + S + len0, S, Hq, Hkv, D, cap, start, len0)
+    stride = Hq * 2 * D + 2 * Hkv * D + pad
+    proj = np.zeros((S, stride), np.float32)
+    proj[:, :Hq * 2 * D] = c["q_gate"].reshape(S, -1)
+    proj[:, Hq * 2 * D:Hq * 2 * D + Hkv * D] = c["k"].reshape(S, -1)
+    proj[:, Hq * 2 * D + Hkv * D:Hq * 2 * D + 2 * Hkv * D] = c["v"].reshape(S, -1)
+    pd, kc, vc = to_dev(proj, dev), to_dev(c["kc"], dev), to_dev(c["vc"], dev)
+    qw, kw = to_dev(c["qw"], dev), to_dev(c["kw"], dev)
+    ring = anelm.ops.KVRing(cap, start, len0)
+    tab = anelm.ops.rope_table(rot, table_rows, 1e7, dev) if table_rows else None
+    out = torch.empty(S, Hq * D, device=dev)
+    p = ctypes.c_void_p
+    anelm.call("anelm_full_attn_prefill", p(out.data_ptr()), p(pd.data_ptr()),
+               p(pd.data_ptr() + 4 * Hq * 2 * D), p(pd.data_ptr() + 4 * (Hq * 2 * D + Hkv * D)), stride,
+               p(kc.data_ptr()), p(vc.data_ptr()), p(qw.data_ptr()), p(kw.data_ptr()), S, Hq, Hkv, D, rot, pos0,
+               ctypes.c_float(1e7), ctypes.c_float(1e-6), rope_mode, 1, p(tab.data_ptr() if table_rows else None),
+               table_rows, ctypes.byref(ring.start), ctypes.byref(ring.len), cap,
+               p(torch.cuda.current_stream().cuda_stream))
+    assert (ring.start.value, ring.len.value) == (start, len0 + S)
+
+    def rows(x, w, heads):
+        x = x.double()
+        x = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-6) * w.double()
+        i = torch.arange(0, rot, 2, dtype=torch.float32)
+        freq = (1.0 / torch.pow(torch.tensor(1e7), i / rot)).to(dev)
+        ang = (torch.arange(pos0, pos0 + S, dtype=torch.float32, device=dev)[:, None] * freq).double()[:, None]
+        a, b = (x[..., 0:rot:2], x[..., 1:rot:2]) if rope_mode == 0 else (x[..., :rot // 2], x[..., rot // 2:rot])
+        a, b = a * torch.cos(ang) - b * torch.sin(ang), a * torch.sin(ang) + b * torch.cos(ang)
+        x = x.clone()
+        if rope_mode == 0:
+            x[..., 0:rot:2], x[..., 1:rot:2] = a, b
+        else:
+            x[..., :rot // 2], x[..., rot // 2:rot] = a, b
+        return x.float().half()
+
+    slots = (start + torch.arange(len0 + S, device=dev)) % cap
+    q = rows(pd[:, :Hq * 2 * D].view(S, Hq, 2 * D)[..., :D], qw, Hq).double()
+    want_k, want_v = to_dev(c["kc"], dev).view(torch.float16), to_dev(c["vc"], dev).view(torch.float16)
+    want_k[slots[len0:]] = rows(to_dev(c["k"], dev), kw, Hkv)
+    want_v[slots[len0:]] = to_dev(c["v"], dev).half()
+    got_k = kc.view(torch.float16)
+    assert_close(got_k.float().cpu().numpy(), want_k.float().cpu().numpy(), rel=1e-3, max_abs=2e-3, what="k ring")
+    assert torch.equal(vc.view(torch.float16), want_v)
+    kk, vv = got_k[slots].double(), want_v[slots].double()
+    gate = torch.sigmoid(to_dev(c["q_gate"], dev)[..., D:].double())
+    mask = torch.arange(len0 + S, device=dev)[None] > len0 + torch.arange(S, device=dev)[:, None]
+    for h in range(Hq):
+        sc = (q[:, h] @ kk[:, h * Hkv // Hq].t().contiguous() / 16.0).masked_fill(mask, -np.inf)
+        want = (torch.softmax(sc, -1) @ vv[:, h * Hkv // Hq].contiguous()) * gate[:, h]
+        assert_close(out.view(S, Hq, D)[:, h].cpu().numpy(), want.float().cpu().numpy(), what=f"head {h}")
+
+
 @pytest.mark.parametrize("S,Hk,Hv,flags,pos0", [
     (100, 16, 32, 5, 2),      # 4B layer: l2 norm + gated norm, conv ring position 2
     (130, 16, 16, 7, 0),      # 0.8B heads, transformers order
