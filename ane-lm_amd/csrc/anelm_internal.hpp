@@ -142,6 +142,17 @@ int prefill_core(void* out, bool out16, const uint16_t* q, const uint16_t* k, co
                  int S, int L, int qoff, int win, int Hq, int Hkv, int D, const float* gate, int gtok, int ghead,
                  hipStream_t st);
 
+// DeltaNet prompt prefill from the projection rows (deltanet.hip): conv width
+// 4, rows and conv weights 16-byte aligned (`fits`); y [S][Hv][128] before the
+// gated norm, the conv ring advanced.  And the gated norm of such rows in place
+// with z read at z + t * zs + h * 128 (everything 8-byte aligned).
+bool deltanet_prefill_proj_fits(const float* proj, const float* conv_w, int pd, int conv_kernel);
+int deltanet_prefill_proj(float* y, float* state, float* conv_state, int conv_pos, const float* proj,
+                          const float* conv_w, const float* A, const float* dt_bias, int S, int Hk, int Hv, int pd,
+                          int flags, hipStream_t st);
+int rmsnorm_gated_heads(float* x, const float* z, long zs, const float* weight, int tokens, int heads,
+                        hipStream_t st);
+
 // `n` counters of the pool of `stream` on the current device, in the range
 // reserved for one user (ranges never overlap, so no user sees another's
 // values); nullptr if n exceeds the range.  Every range starts zeroed.

@@ -14,6 +14,8 @@
 
 #include <math.h>
 
+#include <atomic>
+
 namespace anelm {
 namespace {
 
@@ -321,99 +323,195 @@ __global__ __launch_bounds__(kScanNT) void dn_scan_kernel(float* y, float* state
 //   y  = Op + Qh S0,      Op = P Ut,  Qh = diag(exp(lg)) Q - P Wm,
 //                         P_ti = exp(lg_t - lg_i) (q_t . k_i), i <= t
 //   S_end = gC S0 + Kh^T U,  Kh = diag(exp(lg_L - lg)) K,  gC = exp(lg_L)
-// Everything but the three products with S0 is independent of the state and
-// is computed for all chunks at once (dn_chunk_prep_mfma_kernel), and
-// dn_chunk_mfma_kernel then carries the state through the chunks.  Decay
-// ratios are formed in log space (all exponents <= 0).  Rows past the
-// sequence end are zero (beta 0, log decay 0), so they change nothing.
+// Everything but the products with S0 and U is independent of the state and is
+// computed for all chunks at once (dn_chunk_prep_kernel); dn_chunk_scan_kernel
+// then carries the state through the chunks.  The scan forms
+//   U = Ut - Wm S0,  y = diag(exp(lg)) (Q S0) + P U,
+//   S_end = gC S0 + K^T (diag(exp(lg_L - lg)) U),
+// so a value head's record holds Ut, Wm, P and the decay factors only, and the
+// normalised Q and K rows are stored once per key head (Op, Qh and Kh per value
+// head were 160 KB a chunk and half of the preparation's products; now 76 KB
+// and 64 KB shared by the key head's value heads).  Decay ratios are formed in
+// log space (all exponents <= 0).  Rows past the sequence end are zero (beta
+// 0, log decay 0), so they change nothing.
+//
+// The chunk matrices are stored as the scan's operand fragments: 16x16 tiles
+// of 64 lanes x 4 floats, so each of its loads is 1 KiB of consecutive memory
+// (row-major records made every load 16 pieces of 64 bytes: the address units
+// were busy all through the scan, 270 us for 4096 tokens of 32 heads, 193 with
+// the same bytes consecutive).
+//   "D" fragment: lane n + 16 k holds rows 4 k + (0..3) of column n, the
+//       layout of a product's result;
+//   "A" fragment: lane m + 16 k holds columns 4 k + (0..3) of row m, the left
+//       operand of four products v_mfma_f32_16x16x4_f32 (the contraction index
+//       of product e is 4 k + e in both operands; a D fragment is the right
+//       operand of the same).
 constexpr int kChunk = 64;
 constexpr int kCMat = kChunk * kDK;             // floats per chunk matrix
-constexpr int kCRec = 5 * kCMat + 64;           // Ut, Wm, Op, Qh, Kh, gC
+// record of a (chunk, value head): Ut D[4][8], Wm A[4][8] (row tile, column
+// tile), P A[10] (tile (r, x <= r) at r (r + 1) / 2 + x), exp(lg_t) [64],
+// exp(lg_L - lg_t) [64], gC
+constexpr int kVW = kCMat, kVP = 2 * kCMat, kVE = kVP + 10 * 256, kVRec = kVE + 192;
+// record of a (chunk, key head): Q A[4][8], K^T A[8][4] (state row tile, chunk row tile)
+constexpr int kKT = kCMat, kKRec = 2 * kCMat;
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// 4x4 transpose within each quad of lanes: lane i's element j <-> lane j's
+// element i.
+__device__ __forceinline__ v4f quad_transpose(v4f x, int lane) {
+    const bool b0 = lane & 1, b1 = lane & 2;
+    // exchange with lane ^ 1: (0,1) and (2,3)
+    const float s0 = partner<1>(b0 ? x[0] : x[1]), s1 = partner<1>(b0 ? x[2] : x[3]);
+    x = v4f{b0 ? s0 : x[0], b0 ? x[1] : s0, b0 ? s1 : x[2], b0 ? x[3] : s1};
+    // exchange with lane ^ 2: (0,2) and (1,3)
+    const float t0 = partner<2>(b1 ? x[0] : x[2]), t1 = partner<2>(b1 ? x[1] : x[3]);
+    return v4f{b1 ? t0 : x[0], b1 ? t1 : x[1], b1 ? x[2] : t0, b1 ? x[3] : t1};
+}
+
+// Inputs of the preparation.  CONV: q, k, v are channels of the raw projection
+// rows `proj` [S][pd] (mixed qkv | z | a | b) passed through the causal conv1d
+// of width 4 over [conv ring | prompt] and SiLU here (cpu_ops.cpp:89-129,
+// :6-13); rows and weights 16-byte aligned.
+struct ChunkArgs {
+    float* vrec;               // [chunks][Hv][kVRec]
+    float* krec;               // [chunks][Hk][kKRec]
+    const float* q;            // [S][Hk][dk]
+    const float* k;
+    const float* v;            // [S][Hv][dv]
+    const float* a;            // token t, head h at a[t * as + h]
+    const float* b;
+    const float* A;
+    const float* dt_bias;
+    const float* proj;
+    const float* conv_state;   // [C][3], oldest at slot conv_pos
+    const float* conv_w;       // [C][4]
+    long as, pd;
+    int conv_pos, S, Hk, Hv, flags;
+    int per_wg;                // value heads per workgroup (Hv / Hk, or 1)
+};
+
+// Input of token tt < 0 of channel c: the ring holds inputs -3 .. -1 oldest
+// first from slot conv_pos.
+__device__ __forceinline__ float ring_input(const ChunkArgs& p, int c, int tt) {
+    int idx = p.conv_pos + tt + 3;
+    if (idx >= 3) idx -= 3;
+    return p.conv_state[(size_t)c * 3 + idx];
+}
+
+// The conv over four consecutive inputs, the oldest three first, then SiLU.
+__device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x3, float4 w) {
+    float sum = 0.0f;
+    sum += x0 * w.x;
+    sum += x1 * w.y;
+    sum += x2 * w.z;
+    const float y = sum + x3 * w.w;
+    return y / (expf(-y) + 1.0f);
+}
 
 // ------------------------------------------- chunk preparation on fp32 MFMA
 // The per-chunk matrices above, on v_mfma_f32_16x16x4_f32, from the raw
-// inputs: the pre-pass of the token scan (dn_prep_kernel: l2 norm and q scale,
-// beta, log decay) is folded in, so q and k are read once and nothing is
-// staged through memory.
-// One workgroup (8 waves) per (chunk, key head); the key head's G = Hv / Hk
-// value heads share its key and query rows, so the Gram tiles K K^T and Q K^T
-// (the 10 lower 16x16 tiles of each) are computed once and kept in registers.
+// inputs: conv and SiLU (CONV), l2 norm and q scale, beta, log decay are
+// formed here, so the inputs are read once and nothing is staged through
+// memory.  One workgroup (8 waves) per (chunk, key head, per_wg value heads);
+// the value heads of a workgroup share its key and query rows: the Gram tiles
+// K K^T and Q K^T (the 10 lower 16x16 tiles of each) are computed once and
+// kept in registers, transposed (K as the left operand), so four consecutive
+// columns of a row are a lane's four elements.
 // Per value head:
-//   Am = -A (strictly lower, row-major) and P (lower) go to LDS;
+//   Am = -A (strictly lower, row-major) goes to LDS, P to the record;
 //   wave 0 turns the diagonal 16x16 blocks of Am into T_rr = (I + A_rr)^-1
 //   by substitution, in place;
 //   for B = [beta V | beta exp(lgT) K] (64 x 256) the blocked forward
-//   substitution and the product with P run per 16-column tile of B (wave w
-//   owns tiles 2w, 2w + 1; it loads its tiles of B straight into the
-//   accumulator layout: V columns from memory, K columns from LDS):
-//     X_r = T_rr (B_r + sum_{s<r} Am_rs X_s),  Y_r = sum_{s<=r} P_rs X_s
-//   with X = [Ut | Wm] and Y = [Op | P Wm] (Qh = diag(exp(lg)) Q - P Wm).
-// MFMA operand layouts as in dn_chunk_mfma_kernel: A[m][k] in lane m + 16 k,
-// B[k][n] in lane n + 16 k, D[m][n] in lane n + 16 (m / 4), element m % 4.
-// The contraction index of k-step e is 4 k + e in both operands, so an A
-// operand is one 16-byte LDS read per lane for four MFMAs, and a result tile
-// in the D layout is already the B operand of the next product: X stays in
-// registers from its substitution to its product with P.
+//   substitution runs per 16-column tile of B (wave w owns tiles 2w, 2w + 1;
+//   it forms its tiles of B straight in the accumulator layout: V columns from
+//   memory, K columns from LDS):
+//     X_r = T_rr (B_r + sum_{s<r} Am_rs X_s),  X = [Ut | Wm]
+//   X tiles stay in registers: a result tile is the right operand of the next
+//   product.  Ut tiles are stored as they are, Wm tiles transposed in quads.
 // LDS matrices are row-major with 16-byte chunks XOR-swizzled by (row & 15);
 // 66 KB, so two workgroups share a CU (one's serial phases overlap the other).
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 constexpr int kPmNT = 512;
 constexpr int kPmK = 0;                        // K rows [64][128]
 constexpr int kPmR = kCMat;                    // Q rows [64][128] for the Gram tiles, then:
 constexpr int kPmA = kPmR;                     //   Am [64][64] (T_rr on its diagonal blocks)
-constexpr int kPmP = kPmA + kChunk * kChunk;   //   P [64][64]
 constexpr int kPmLg = kPmR + kCMat;            // lg[65] (+3 pad)
 constexpr int kPmBt = kPmLg + 68;              // beta[64]
-constexpr int kPmQs = kPmBt + kChunk;          // q row scale[64] (l2 norm and 1/sqrt(dk))
-constexpr int kPmEb = kPmQs + kChunk;          // exp(lg[t + 1]) (decay-first) or exp(lg[t]): scales K in B
-constexpr int kPmEq = kPmEb + kChunk;          // exp(lg[t + 1]): scales q in Qh
-constexpr int kPmEk = kPmEq + kChunk;          // exp(lg_L - lg[t + 1]): scales K in Kh
-constexpr int kPmLds = (kPmEk + kChunk) * 4;
+constexpr int kPmEb = kPmBt + kChunk;          // exp(lg[t + 1]) (decay-first) or exp(lg[t]): scales K in B
+constexpr int kPmLds = (kPmEb + kChunk) * 4;
 
 __device__ __forceinline__ int sw128(int t, int d) { return t * kDK + 4 * ((d >> 2) ^ (t & 15)) + (d & 3); }
 __device__ __forceinline__ int sw64(int r, int c) { return r * kChunk + 4 * ((c >> 2) ^ (r & 15)) + (c & 3); }
 
-template <bool TF>
-__global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
-    float* __restrict__ rec, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const float* __restrict__ a, const float* __restrict__ b, const float* __restrict__ A,
-    const float* __restrict__ dt_bias, int S, int Hk, int Hv, int flags) {
+template <bool TF, bool CONV>
+__global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs p) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float* Ks = sm + kPmK;
     float* Rs = sm + kPmR;
     float* Am = sm + kPmA;
-    float* Pm = sm + kPmP;
     float* lg = sm + kPmLg;
     float* bt = sm + kPmBt;
-    float* qs = sm + kPmQs;
     float* eb = sm + kPmEb;
-    float* eq = sm + kPmEq;
-    float* ek = sm + kPmEk;
+    const int S = p.S, Hk = p.Hk, Hv = p.Hv;
     const int c = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lm = lane & 15, lk = lane >> 4;
-    const int G = Hv / Hk;
     const int t0 = c * kChunk, L = min(kChunk, S - t0);
     // ---- key and query rows of the chunk, l2-normalised (qwen3_5.cpp:879-887),
     // q also scaled by 1/sqrt(dk); zero past the sequence end.  A row is 32
-    // float4 chunks held by 32 consecutive lanes (half a wave)
+    // float4 chunks held by 32 consecutive lanes (half a wave), which take four
+    // consecutive tokens
     {
+        const int ch = tid & 31, tb = 4 * (tid >> 5);
         float4 kv[4], qv[4];
+        if constexpr (CONV) {
+            const int cq = kh * kDK + 4 * ch, ck = Hk * kDK + cq;
+            float4 qx[7], kx[7];   // inputs of tokens tb - 3 .. tb + 3
 #pragma unroll
-        for (int x = 0; x < 4; x++) {
-            const int e = tid + kPmNT * x, t = e >> 5, ch = e & 31;
-            const size_t off = ((size_t)(t0 + min(t, L - 1)) * Hk + kh) * kDK + 4 * ch;
-            kv[x] = *reinterpret_cast<const float4*>(k + off);
-            qv[x] = *reinterpret_cast<const float4*>(q + off);
+            for (int i = 0; i < 7; i++) {
+                const int tt = t0 + tb + i - 3;
+                const float* row = p.proj + (size_t)min(max(tt, 0), S - 1) * p.pd;
+                qx[i] = *reinterpret_cast<const float4*>(row + cq);
+                kx[i] = *reinterpret_cast<const float4*>(row + ck);
+                if (i < 3 && tt < 0) {
+                    qx[i] = make_float4(ring_input(p, cq, tt), ring_input(p, cq + 1, tt), ring_input(p, cq + 2, tt),
+                                        ring_input(p, cq + 3, tt));
+                    kx[i] = make_float4(ring_input(p, ck, tt), ring_input(p, ck + 1, tt), ring_input(p, ck + 2, tt),
+                                        ring_input(p, ck + 3, tt));
+                }
+            }
+            float4 wq[4], wk[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                wq[j] = *reinterpret_cast<const float4*>(p.conv_w + (size_t)(cq + j) * 4);
+                wk[j] = *reinterpret_cast<const float4*>(p.conv_w + (size_t)(ck + j) * 4);
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                qv[x] = make_float4(conv_tap4(qx[x].x, qx[x + 1].x, qx[x + 2].x, qx[x + 3].x, wq[0]),
+                                    conv_tap4(qx[x].y, qx[x + 1].y, qx[x + 2].y, qx[x + 3].y, wq[1]),
+                                    conv_tap4(qx[x].z, qx[x + 1].z, qx[x + 2].z, qx[x + 3].z, wq[2]),
+                                    conv_tap4(qx[x].w, qx[x + 1].w, qx[x + 2].w, qx[x + 3].w, wq[3]));
+                kv[x] = make_float4(conv_tap4(kx[x].x, kx[x + 1].x, kx[x + 2].x, kx[x + 3].x, wk[0]),
+                                    conv_tap4(kx[x].y, kx[x + 1].y, kx[x + 2].y, kx[x + 3].y, wk[1]),
+                                    conv_tap4(kx[x].z, kx[x + 1].z, kx[x + 2].z, kx[x + 3].z, wk[2]),
+                                    conv_tap4(kx[x].w, kx[x + 1].w, kx[x + 2].w, kx[x + 3].w, wk[3]));
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const size_t off = ((size_t)(t0 + min(tb + x, L - 1)) * Hk + kh) * kDK + 4 * ch;
+                kv[x] = *reinterpret_cast<const float4*>(p.k + off);
+                qv[x] = *reinterpret_cast<const float4*>(p.q + off);
+            }
         }
         const float qk_scale = 1.0f / sqrtf((float)kDK);
 #pragma unroll
         for (int x = 0; x < 4; x++) {
-            const int e = tid + kPmNT * x, t = e >> 5, ch = e & 31;
+            const int t = tb + x;
             float ik = 1.f, iq = 1.f;
-            if (flags & ANELM_DN_L2NORM) {
+            if (p.flags & ANELM_DN_L2NORM) {
                 float sk = kv[x].x * kv[x].x + kv[x].y * kv[x].y + kv[x].z * kv[x].z + kv[x].w * kv[x].w;
                 float sq = qv[x].x * qv[x].x + qv[x].y * qv[x].y + qv[x].z * qv[x].z + qv[x].w * qv[x].w;
 #pragma unroll
@@ -429,12 +527,27 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
                 make_float4(kv[x].x * mk, kv[x].y * mk, kv[x].z * mk, kv[x].w * mk);
             *reinterpret_cast<float4*>(Rs + sw128(t, 4 * ch)) =
                 make_float4(qv[x].x * mq, qv[x].y * mq, qv[x].z * mq, qv[x].w * mq);
-            if (ch == 0) qs[t] = mq;
         }
     }
     lds_barrier();
+    // ---- the key head's record (one workgroup of the key head): wave w stores
+    // Q tiles (w / 2, 4 (w % 2) ..) and K^T row tile w
+    if (blockIdx.z == 0) {
+        float* kr = p.krec + ((size_t)c * Hk + kh) * kKRec;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            const int rt = w >> 1, xt = 4 * (w & 1) + x;
+            *reinterpret_cast<v4f*>(kr + ((rt * 8 + xt) * 64 + lane) * 4) =
+                *reinterpret_cast<const v4f*>(Rs + sw128(16 * rt + lm, 16 * xt + 4 * lk));
+            v4f kt;
+#pragma unroll
+            for (int j = 0; j < 4; j++) kt[j] = Ks[sw128(16 * x + 4 * lk + j, 16 * w + lm)];
+            *reinterpret_cast<v4f*>(kr + kKT + ((w * 4 + x) * 64 + lane) * 4) = kt;
+        }
+    }
     // ---- Gram tiles: 10 lower tiles of K K^T (ids 0..9) and of Q K^T (10..19);
-    // wave w takes ids w, w + 8, w + 16
+    // wave w takes ids w, w + 8, w + 16.  Element e of lane (lm, lk) is row
+    // 16 ti + lm, column 16 tj + 4 lk + e
     v4f gram[3];
 #pragma unroll
     for (int u = 0; u < 3; u++) {
@@ -446,8 +559,8 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
         v4f a0 = gram[u], a1 = gram[u];
 #pragma unroll
         for (int x = 0; x < 8; x++) {
-            const float4 a4 = *reinterpret_cast<const float4*>(src + sw128(16 * ti + lm, 16 * x + 4 * lk));
-            const float4 b4 = *reinterpret_cast<const float4*>(Ks + sw128(16 * tj + lm, 16 * x + 4 * lk));
+            const float4 a4 = *reinterpret_cast<const float4*>(Ks + sw128(16 * tj + lm, 16 * x + 4 * lk));
+            const float4 b4 = *reinterpret_cast<const float4*>(src + sw128(16 * ti + lm, 16 * x + 4 * lk));
             a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.x, b4.x, a0, 0, 0, 0);
             a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.y, b4.y, a1, 0, 0, 0);
             a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.z, b4.z, a0, 0, 0, 0);
@@ -456,44 +569,62 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
         gram[u] = a0 + a1;
         __builtin_amdgcn_sched_barrier(0);   // one tile's operands live at a time
     }
-    lds_barrier();   // the query rows are no longer read: their space takes Am and P
-    // rows past the sequence end fall outside these ranges and load as zeros
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(v), 0,
-                                                                         (int)((size_t)S * Hv * kDV * 4), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(q), 0,
-                                                                         (int)((size_t)S * Hk * kDK * 4), 0x00020000);
-    for (int g = 0; g < G; g++) {
-        const int h = kh * G + g;
-        float* out = rec + ((size_t)c * Hv + h) * kCRec;
-        const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(out, 0, kCRec * 4, 0x00020000);
+    lds_barrier();   // the query rows are no longer read: their space takes Am
+    for (int g = 0; g < p.per_wg; g++) {
+        const int h = kh * (Hv / Hk) + blockIdx.z * p.per_wg + g;
+        float* out = p.vrec + ((size_t)c * Hv + h) * kVRec;
         // lane-derived addresses are recomputed per value head, not held across the loop
         int ltid = tid;
         asm volatile("" : "+v"(ltid));
         const int lane = ltid & 63, lm = lane & 15, lk = lane >> 4;
         // this wave's memory operands, issued first: V rows of its B tiles
-        // (waves 0..3, tiles 0..7) or the raw q rows of its Qh tiles (waves 4..7)
+        // (waves 0..3, tiles 0..7), rows 16 r + 4 lk + e (CONV: the inputs of
+        // the three tokens before them too)
         const bool wpart = w >= 4;
         float pre[2][4][4];
+        if (!wpart) {
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+            for (int u = 0; u < 2; u++) {
+                const int col = 16 * (2 * w + u) + lm;
+                if constexpr (CONV) {
+                    const int cv = 2 * Hk * kDK + h * kDV + col;
+                    const float4 wv = *reinterpret_cast<const float4*>(p.conv_w + (size_t)cv * 4);
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+                    for (int r = 0; r < 4; r++) {
+                        float x[7];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = 16 * r + 4 * lk + e, col = 16 * ((2 * w + u) & 7) + lm;
-                    const int off = wpart ? ((t0 + t) * Hk + kh) * kDK + col : ((t0 + t) * Hv + h) * kDV + col;
-                    pre[u][r][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wpart ? rq : rv,
-                                                                                                 off * 4, 0, 0));
+                        for (int i = 0; i < 7; i++) {
+                            const int tt = t0 + 16 * r + 4 * lk + i - 3;
+                            x[i] = p.proj[(size_t)min(max(tt, 0), S - 1) * p.pd + cv];
+                            if (r == 0 && i < 3 && tt < 0) x[i] = ring_input(p, cv, tt);
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float y = conv_tap4(x[e], x[e + 1], x[e + 2], x[e + 3], wv);
+                            pre[u][r][e] = 16 * r + 4 * lk + e < L ? y : 0.f;
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const int t = 16 * r + 4 * lk + e;
+                            const float y = p.v[((size_t)(t0 + min(t, L - 1)) * Hv + h) * kDV + col];
+                            pre[u][r][e] = t < L ? y : 0.f;
+                        }
                 }
+            }
+        }
         // ---- beta = sigmoid(b) and log decay = -A softplus(a + dt_bias)
-        // (qwen3_5.cpp:896-898); lg[t + 1] = sum_{j <= t} log decay_j (wave 0)
-        if (w == 0) {
+        // (qwen3_5.cpp:896-898); lg[t + 1] = sum_{j <= t} log decay_j (wave 7)
+        if (w == 7) {
             const bool in = lane < L;
             float x = 0.f, bv = 0.f;
             if (in) {
-                const size_t gi = (size_t)(t0 + lane) * Hv + h;
-                bv = 1.0f / (1.0f + expf(-b[gi]));
-                x = -A[h] * logf(1.0f + expf(a[gi] + dt_bias[h]));
+                const size_t gi = (size_t)(t0 + lane) * p.as + h;
+                bv = 1.0f / (1.0f + expf(-p.b[gi]));
+                x = -p.A[h] * logf(1.0f + expf(p.a[gi] + p.dt_bias[h]));
             }
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
@@ -503,15 +634,15 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
             lg[lane + 1] = x;
             if (lane == 0) lg[0] = 0.f;
             bt[lane] = bv;
-            // the per-row decay factors every lane of the value head uses
-            // (the same expressions as per element, evaluated once per row)
+            // the per-row decay factors, evaluated once per row
             const float xs = __shfl_up(x, 1, 64);   // (every lane takes part in the shuffles)
             const float xl = __shfl(x, 63, 64);     // lg_L
             const float xp = lane == 0 ? 0.f : xs;  // lg[t]
             const float e1 = expf(x);
-            eq[lane] = e1;
             eb[lane] = TF ? e1 : expf(xp);
-            ek[lane] = expf(xl - x);
+            out[kVE + lane] = e1;
+            out[kVE + 64 + lane] = expf(xl - x);
+            if (lane == 63) out[kVE + 128] = e1;    // gC
         }
         lds_barrier();
         // ---- Am = -A and P from the Gram tiles
@@ -520,18 +651,19 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
             const int id = w + 8 * u;
             if (id >= 20) continue;
             const int pi = id % 10, ti = (pi >= 1) + (pi >= 3) + (pi >= 6), tj = pi - ti * (ti + 1) / 2;
-            const int i = 16 * tj + lm;
-            const float lgi = lg[i + 1];
+            const int t = 16 * ti + lm, i0 = 16 * tj + 4 * lk;
+            const bool isA = id < 10;
+            const float lgt = isA && !TF ? lg[t] : lg[t + 1], bs = -bt[t];
+            v4f o4;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int t = 16 * ti + 4 * lk + e;
-                if (id < 10) {
-                    const float lgT = TF ? lg[t + 1] : lg[t];
-                    Am[sw64(t, i)] = i < t ? -(bt[t] * expf(lgT - lgi) * gram[u][e]) : 0.f;
-                } else {
-                    Pm[sw64(t, i)] = i <= t ? expf(lg[t + 1] - lgi) * gram[u][e] : 0.f;
-                }
+                const int i = i0 + e;
+                const float f = expf(lgt - lg[i + 1]);
+                if (isA) o4[e] = i < t ? bs * f * gram[u][e] : 0.f;
+                else o4[e] = i <= t ? f * gram[u][e] : 0.f;
             }
+            if (isA) *reinterpret_cast<v4f*>(Am + sw64(t, i0)) = o4;
+            else *reinterpret_cast<v4f*>(out + kVP + (pi * 64 + lane) * 4) = o4;
         }
         lds_barrier();
         if (w == 0) {
@@ -555,26 +687,9 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
             }
 #pragma unroll
             for (int t = 0; t < 16; t++) Am[sw64(16 * b + t, 16 * b + j)] = x[t];
-        } else {
-            // ---- Kh = diag(exp(lg_L - lg)) K, stored transposed (Kh^T [128][64]:
-            // the scan reads it as rows of its state-row tiles), gC (waves 1..7)
-            const float lgL = lg[kChunk];
-            for (int e = ltid - 64; e < kCMat / 4; e += kPmNT - 64) {
-                const int kd = e >> 4, t4 = e & 15;
-                v4f o4;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int t = 4 * t4 + j;
-                    o4[j] = Ks[sw128(t, kd)] * ek[t];
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o4), ro,
-                                                       (4 * kCMat + kd * kChunk + 4 * t4) * 4, 0, 0);
-            }
-            if (ltid == 64)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, expf(lgL)), ro, 5 * kCMat * 4, 0, 0);
         }
         lds_barrier();
-        // ---- X and Y for column tiles jt = 2w + u of B
+        // ---- X for column tiles jt = 2w + u of B
         v4f X[2][4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -603,35 +718,17 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_mfma_kernel(
                 xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.z, acc[2], xr, 0, 0, 0);
                 xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.w, acc[3], xr, 0, 0, 0);
                 X[u][r] = xr;
-                // Y_r = sum_{s <= r} P_rs X_s
-                v4f y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s2 = 0; s2 <= r; s2++) {
-                    const float4 p4 = *reinterpret_cast<const float4*>(Pm + sw64(16 * r + lm, 16 * s2 + 4 * lk));
-                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(p4.x, X[u][s2][0], y, 0, 0, 0);
-                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(p4.y, X[u][s2][1], y, 0, 0, 0);
-                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(p4.z, X[u][s2][2], y, 0, 0, 0);
-                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(p4.w, X[u][s2][3], y, 0, 0, 0);
-                }
-                // rows t = 16 r + 4 lk + e, column 16 (jt % 8) + lm of Ut / Wm and Op / Qh
-                const int col = 16 * (jt & 7) + lm;
-                const int ox = wpart ? kCMat : 0, oy = wpart ? 3 * kCMat : 2 * kCMat;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = 16 * r + 4 * lk + e;
-                    // through a scalar: a bit_cast of a vector element is lowered as element 0
-                    const float xv = xr[e];
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, xv), ro, (ox + t * kDK + col) * 4,
-                                                          0, 0);
-                    float yv = y[e];
-                    if (wpart) yv = eq[t] * (qs[t] * pre[u][r][e]) - yv;
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ro, (oy + t * kDK + col) * 4,
-                                                          0, 0);
-                }
+                // Ut: the D fragment; Wm: transposed in quads, lane (4 c + i, k)
+                // then holds row 4 k + i, columns 4 c .. 4 c + 3 of its A fragment
+                if (wpart)
+                    *reinterpret_cast<v4f*>(out + kVW + ((r * 8 + jt - 8) * 64 + 4 * lk + (lm & 3) + 16 * (lm >> 2)) * 4) =
+                        quad_transpose(xr, lane);
+                else
+                    *reinterpret_cast<v4f*>(out + ((r * 8 + jt) * 64 + lane) * 4) = xr;
                 __builtin_amdgcn_sched_barrier(0);   // bounds the loads hoisted ahead of this tile
             }
         }
-        lds_barrier();   // Am, P, lg and beta are rewritten for the next value head
+        lds_barrier();   // Am, lg and beta are rewritten for the next value head
     }
 }
 
@@ -640,73 +737,96 @@ constexpr int kSeqCB = 16;
 constexpr int kSlabs = kDV / kSeqCB;
 
 // ------------------------------------------------ chunk scan on fp32 MFMA
-// The same three products per chunk on v_mfma_f32_16x16x4_f32 (fp32 inputs,
-// fp32 accumulation).  A workgroup (8 waves, two per SIMD) owns a 16-column
-// slab of one head's state, kept in LDS column-major (Sc[c][i]):
-//   waves 0-3: X = Wm S0 for chunk rows [16 w, 16 w + 16), U = Ut - X (LDS);
-//   waves 4-7: Y = Qh S0 for chunk rows [16 (w - 4), ...), y = Op + Y (LDS,
-//   then stored by all 8 waves);
-//   then wave w: S = gC S0 + Kh^T U for state rows [16 w, 16 w + 16).
-// Every operand but the state and U is read by one wave only (its Wm or Qh
-// rows, its Kh^T rows, its Ut or Op entries), so it goes from memory straight
-// into registers, the next chunk's loads spread over this chunk's products;
-// LDS carries only the state slab and U.
-// MFMA operand layouts (16x16x4, one block): A[m][k] in lane m + 16 k,
-// B[k][n] in lane n + 16 k, D[m][n] in lane n + 16 (m / 4), element m % 4.
-// The contraction index is permuted identically in both operands: lane (m, k)
-// of k-step (x, e) takes state row (or chunk row) 16 x + 4 k + e, so an A
-// operand is one 16-byte read per lane for four k-steps.
+// The state products per chunk on v_mfma_f32_16x16x4_f32 (fp32 inputs, fp32
+// accumulation).  A workgroup (8 waves, two per SIMD) owns a 16-column slab of
+// one head's state, kept in LDS column-major (Sc[c][i]):
+//   waves 0-3: X = Wm S0 for chunk rows [16 w, 16 w + 16), U = Ut - X and its
+//              decayed copy to LDS (column-major);
+//   waves 4-7: Y = Q S0 for chunk rows [16 (w - 4), ...), kept in registers;
+//   then wave w: S = gC S0 + K^T (decayed U) for state rows [16 w, 16 w + 16),
+//   and waves 4-7 y = diag(exp(lg)) Y + P U.
+// Every operand but the state and U is read by one wave only, so it goes from
+// memory straight into registers (1 KiB fragments), the next chunk's loads
+// spread over this chunk's products; LDS carries only the state slab and U.
+// Bound: @SCAN@
 constexpr int kMsNT = 512;
 constexpr int kScP = kDK + 4;        // Sc row pitch (floats): 16-byte reads of 16 lanes hit distinct banks
-constexpr int kUlP = kSeqCB + 4;     // U row pitch: rows 4 apart land 16 banks apart
-constexpr int kMsLds = (kSeqCB * kScP + 2 * kChunk * kUlP) * 4;
+constexpr int kUlP = kChunk + 4;     // U column pitch, likewise
+constexpr int kMsLds = kSeqCB * (kScP + 2 * kUlP) * 4;
 
 // One wave's operands of one chunk.
 struct ScanOps {
-    v4f m[8];     // Wm (waves 0-3) or Qh (4-7) row 16 (w & 3) + lr, state rows 16 x + 4 lq + (0..3)
-    v4f kt[4];    // Kh^T row 16 w + lr, chunk rows 16 x + 4 lq + (0..3)
-    float uo[4];  // Ut (waves 0-3) or Op (4-7) at chunk row 16 (w & 3) + 4 lq + j, slab column lr
+    v4f m[8];     // Wm (waves 0-3) or Q (4-7), row tile w & 3
+    v4f kt[4];    // K^T row tile w
+    v4f u;        // waves 0-3: Ut, row tile w, this slab's column tile
+    v4f p[4];     // waves 4-7: P tiles (w - 4, x <= w - 4)
+    v4f ev;       // rows 16 (w & 3) + 4 lq + (0..3) of exp(lg_L - lg) (waves 0-3) or exp(lg) (4-7)
     float gc;
 };
 
-// Where one wave's operands of chunk ch lie: one chunk record per buffer
-// resource (offsets stay small for any sequence length).
+// Where one wave's operands of chunk ch lie: its records as buffer resources
+// (offsets stay small for any sequence length); operands a wave does not have
+// are out of range and read zeros.
 struct ScanSrc {
-    __amdgpu_buffer_rsrc_t rr;
-    int mo, ko, uo;   // float offsets of this lane's first Wm / Qh, Kh^T and Ut / Op element
+    __amdgpu_buffer_rsrc_t rv, rk;
+    __amdgpu_buffer_rsrc_t rm;        // the one that holds m
+    int mo, ko, uo, po, eo;           // byte offsets of this lane's first element
 };
 
-__device__ __forceinline__ ScanSrc scan_src(const float* rec, int ch, int Hv, int h, int w, int lr, int lq, int c0) {
+__device__ __forceinline__ ScanSrc scan_src(const float* vrec, const float* krec, int ch, int Hk, int Hv, int h, int w,
+                                            int lane, int slab) {
     ScanSrc s;
-    s.rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rec) + ((size_t)ch * Hv + h) * kCRec, 0, kCRec * 4,
-                                             0x00020000);
     const int mt = w & 3;
-    s.mo = (w < 4 ? kCMat : 3 * kCMat) + (16 * mt + lr) * kDK + 4 * lq;
-    s.ko = 4 * kCMat + (16 * w + lr) * kChunk + 4 * lq;
-    s.uo = (w < 4 ? 0 : 2 * kCMat) + (16 * mt + 4 * lq) * kDK + c0 + lr;
+    s.rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vrec) + ((size_t)ch * Hv + h) * kVRec, 0, kVRec * 4,
+                                             0x00020000);
+    s.rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(krec) + ((size_t)ch * Hk + h / (Hv / Hk)) * kKRec, 0,
+                                             kKRec * 4, 0x00020000);
+    s.rm = w < 4 ? s.rv : s.rk;
+    s.mo = ((w < 4 ? kVW : 0) + (mt * 8 * 64 + lane) * 4) * 4;
+    s.ko = (kKT + (w * 4 * 64 + lane) * 4) * 4;
+    s.uo = w < 4 ? ((mt * 8 + slab) * 64 + lane) * 16 : 0x7ffffff0;
+    s.po = (kVP + (mt * (mt + 1) / 2 * 64 + lane) * 4) * 4;
+    s.eo = (kVE + (w < 4 ? 64 : 0) + 16 * mt + 4 * (lane >> 4)) * 4;
     return s;
 }
 
-// Part x (0..7) of a wave's loads of one chunk: m[x], then kt[x] (x < 4) or
-// uo[x - 4] (x >= 4), and gc with the last part.  The parts are issued
-// between the MFMA groups of the previous chunk's products: issued all at
-// once, the workgroup's loads fill the CU's memory queue and the waves stall
-// at their next memory instruction instead of computing.
-__device__ __forceinline__ void scan_part(ScanOps& o, const ScanSrc& s, int x) {
-    o.m[x] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(s.rr, (s.mo + 16 * x) * 4, 0, 0));
-    if (x < 4)
-        o.kt[x] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(s.rr, (s.ko + 16 * x) * 4, 0, 0));
-    else
-        o.uo[x - 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s.rr, (s.uo + (x - 4) * kDK) * 4, 0, 0));
-    if (x == 7) o.gc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s.rr, 5 * kCMat * 4, 0, 0));
+// Part x (0..7) of a wave's loads of one chunk.  The parts are issued between
+// the MFMA groups of the previous chunk's products: issued all at once, the
+// workgroup's loads fill the CU's memory queue and the waves stall at their
+// next memory instruction instead of computing.
+__device__ __forceinline__ void scan_part(ScanOps& o, const ScanSrc& s, int w, int x) {
+    auto ld = [](__amdgpu_buffer_rsrc_t r, int off) __attribute__((always_inline)) {
+        return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    };
+    o.m[x] = ld(s.rm, s.mo + x * 1024);
+    if (x < 4) o.kt[x] = ld(s.rk, s.ko + x * 1024);
+    else o.p[x - 4] = ld(s.rv, w >= 4 + (x - 4) ? s.po + (x - 4) * 1024 : 0x7ffffff0);
+    if (x == 0) o.u = ld(s.rv, s.uo);
+    if (x == 1) o.ev = ld(s.rv, s.eo);
+    if (x == 2) o.gc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s.rv, (kVE + 128) * 4, 0, 0));
 }
 
-__global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dn_chunk_mfma_kernel(
-    float* __restrict__ y, float* __restrict__ state, const float* __restrict__ rec, int S, int Hv, int n_chunks) {
+struct ScanArgs {
+    float* y;              // [S][Hv][dv]
+    float* state;
+    const float* vrec;
+    const float* krec;
+    int S, Hk, Hv, n_chunks;
+    // the conv ring after the prompt (null: none): input t sits at slot
+    // (conv_pos + t) mod 3, so the last 3 inputs overwrite their slots
+    float* conv_state;     // [C][3]
+    const float* proj;     // [S][pd]
+    long pd;
+    int C, conv_pos;
+};
+
+__global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dn_chunk_scan_kernel(
+    const ScanArgs a) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     float (*Sc)[kScP] = reinterpret_cast<float (*)[kScP]>(smem);                   // state slab
-    float (*Ul)[kUlP] = reinterpret_cast<float (*)[kUlP]>(smem + kSeqCB * kScP);   // U of the chunk
-    float (*Yl)[kUlP] = Ul + kChunk;                                               // its y tile
+    float (*Ul)[kUlP] = reinterpret_cast<float (*)[kUlP]>(smem + kSeqCB * kScP);   // U of the chunk, by column
+    float (*Ud)[kUlP] = Ul + kSeqCB;                                               // its decayed copy
+    const int S = a.S, Hv = a.Hv, n_chunks = a.n_chunks;
     // XCD-aware: the 8 slabs of a head share its chunk records, so they go to
     // one XCD (workgroup id mod 8 selects the XCD; Hv * 8 workgroups)
     const int nwg = gridDim.x, id = blockIdx.x;
@@ -717,27 +837,35 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     const int lr = lane & 15, lq = lane >> 4;
     const int mt = w & 3;
     const int c0 = slab * kSeqCB;
-    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, 0, (int)((size_t)S * Hv * kDV * 4), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ry =
+        __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (int)((size_t)S * Hv * kDV * 4), 0x00020000);
 
     // two operand sets, A and B: a chunk is computed from one while the next
     // chunk's loads land in the other (no register copies between them)
     ScanOps opA, opB;
     {
-        const ScanSrc s0 = scan_src(rec, 0, Hv, h, w, lr, lq, c0);
+        const ScanSrc s0 = scan_src(a.vrec, a.krec, 0, a.Hk, Hv, h, w, lane, slab);
 #pragma unroll
-        for (int x = 0; x < 8; x++) scan_part(opA, s0, x);
+        for (int x = 0; x < 8; x++) scan_part(opA, s0, w, x);
     }
-    float* Sp = state + (size_t)h * kDK * kDV;
+    float* Sp = a.state + (size_t)h * kDK * kDV;
     for (int e = tid; e < kDK * kSeqCB; e += kMsNT) {
         const int i = e / kSeqCB, c = e % kSeqCB;
         Sc[c][i] = Sp[(size_t)i * kDV + c0 + c];
+    }
+    if (a.conv_state != nullptr) {
+        const int nt = min(S, 3);
+        for (int e = id * kMsNT + tid; e < a.C * nt; e += nwg * kMsNT) {
+            const int t = S - nt + e / a.C, c = e % a.C;
+            a.conv_state[(size_t)c * 3 + (a.conv_pos + t) % 3] = a.proj[(size_t)t * a.pd + c];
+        }
     }
     __syncthreads();
 
     auto chunk = [&](const ScanOps& cur, ScanOps& nxt, int ch) __attribute__((always_inline)) {
         // the next chunk's operands (the last chunk reloads its own: no branch)
-        const ScanSrc src = scan_src(rec, ch + 1 < n_chunks ? ch + 1 : ch, Hv, h, w, lr, lq, c0);
-        // ---- X = Wm S0 (waves 0-3) or Y = Qh S0 (waves 4-7): 32 MFMAs in 4
+        const ScanSrc src = scan_src(a.vrec, a.krec, ch + 1 < n_chunks ? ch + 1 : ch, a.Hk, Hv, h, w, lane, slab);
+        // ---- X = Wm S0 (waves 0-3) or Y = Q S0 (waves 4-7): 32 MFMAs in 4
         // chains, one part of the next chunk's loads ahead of each group of 4
         v4f sb[8];
 #pragma unroll
@@ -747,37 +875,25 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         for (int e = 0; e < 4; e++) Z[e] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int x = 0; x < 8; x++) {
-            scan_part(nxt, src, x);
+            scan_part(nxt, src, w, x);
             __builtin_amdgcn_sched_barrier(0);   // the part is issued here, not hoisted or sunk
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.m[x][e], sb[x][e], Z[e], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        const v4f Zs = (Z[0] + Z[1]) + (Z[2] + Z[3]);
-        // element j is chunk row 16 mt + 4 lq + j, slab column lr:
-        // U = Ut - X (waves 0-3) and y = Op + Y (waves 4-7) go to LDS
-        {
-            float (*dst)[kUlP] = w < 4 ? Ul : Yl;
-            const float sg = w < 4 ? -1.f : 1.f;
-#pragma unroll
-            for (int j = 0; j < 4; j++) dst[16 * mt + 4 * lq + j][lr] = cur.uo[j] + sg * Zs[j];
+        // element j is chunk row 16 mt + 4 lq + j, slab column lr
+        v4f Zs = (Z[0] + Z[1]) + (Z[2] + Z[3]);
+        if (w < 4) {
+            const v4f U = cur.u - Zs;
+            *reinterpret_cast<v4f*>(&Ul[lr][16 * mt + 4 * lq]) = U;
+            *reinterpret_cast<v4f*>(&Ud[lr][16 * mt + 4 * lq]) = U * cur.ev;
         }
-        lds_barrier();   // U and y complete; every wave's reads of S0 are done
-        {
-            // the y tile to memory, one 8-byte store per lane of every wave:
-            // all waves then have the same memory operations in flight, so the
-            // waits for this chunk's operands count the same everywhere
-            // (y rows past S fall out of the buffer range and are dropped)
-            const int t = tid >> 3, cp = tid & 7;
-            const float2 yv = *reinterpret_cast<const float2*>(&Yl[t][2 * cp]);
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, yv), ry,
-                                                  (((ch * kChunk + t) * Hv + h) * kDV + c0 + 2 * cp) * 4, 0, 0);
-        }
-        // ---- S = gC S0 + Kh^T U for state rows 16 w + (0..15): 16 MFMAs in 4 chains
-        float ub[16];
+        lds_barrier();   // U complete; every wave's reads of S0 are done
+        // ---- S = gC S0 + K^T Ud for state rows 16 w + (0..15): 16 MFMAs in 4 chains
+        v4f ub[4];
 #pragma unroll
-        for (int s = 0; s < 16; s++) ub[s] = Ul[16 * (s >> 2) + 4 * lq + (s & 3)][lr];
+        for (int x = 0; x < 4; x++) ub[x] = *reinterpret_cast<const v4f*>(&Ud[lr][16 * x + 4 * lq]);
         v4f* srow = reinterpret_cast<v4f*>(&Sc[lr][16 * w + 4 * lq]);
         v4f Sn[4];
         Sn[0] = cur.gc * *srow;
@@ -787,10 +903,34 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         for (int x = 0; x < 4; x++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                Sn[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.kt[x][e], ub[4 * x + e], Sn[e], 0, 0, 0);
+                Sn[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.kt[x][e], ub[x][e], Sn[e], 0, 0, 0);
         // rows written here are read (as C) only by this wave
         *srow = (Sn[0] + Sn[1]) + (Sn[2] + Sn[3]);
-        lds_barrier();   // new state complete, U and y consumed
+        // ---- y = diag(exp(lg)) Y + P U (waves 4-7; the others' products and
+        // stores are skipped and dropped)
+        if (w >= 4) {
+            v4f y0 = Zs * cur.ev, y1 = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                if (x > mt) break;
+                const v4f uv = *reinterpret_cast<const v4f*>(&Ul[lr][16 * x + 4 * lq]);
+                y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][0], uv[0], y0, 0, 0, 0);
+                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][1], uv[1], y1, 0, 0, 0);
+                y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][2], uv[2], y0, 0, 0, 0);
+                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][3], uv[3], y1, 0, 0, 0);
+            }
+            Zs = y0 + y1;
+        }
+        lds_barrier();   // new state complete, U consumed
+        // y rows past S fall out of the buffer range and are dropped, as are
+        // the stores of waves 0-3 (every wave has the same operations in
+        // flight, so the waits for operands count the same everywhere)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float yv = Zs[j];
+            const int off = (((ch * kChunk + 16 * mt + 4 * lq + j) * Hv + h) * kDV + c0 + lr) * 4;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ry, w >= 4 ? off : 0x7ffffff0, 0, 0);
+        }
     };
     // pairs of chunks, then an odd last one: inside the loop both halves run
     // unconditionally, so the loads a half issues for the other are not sunk
@@ -805,6 +945,46 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         const int i = e / kSeqCB, c = e % kSeqCB;
         Sp[(size_t)i * kDV + c0 + c] = Sc[c][i];
     }
+}
+
+// Both launches over the inputs of `p` (vrec, krec and per_wg are set here).
+int chunk_prefill(ChunkArgs p, ScanArgs s, bool conv, hipStream_t st) {
+    Device* dev = device();
+    if (!dev) return ANELM_EHIP;
+    const int n_chunks = (p.S + kChunk - 1) / kChunk, G = p.Hv / p.Hk;
+    const size_t nv = (size_t)n_chunks * p.Hv * kVRec, nk = (size_t)n_chunks * p.Hk * kKRec;
+    float* rec = static_cast<float*>(workspace((nv + nk) * sizeof(float), st));
+    if (!rec) return ANELM_ENOMEM;
+    p.vrec = rec;
+    p.krec = rec + nv;
+    using K = void (*)(const ChunkArgs);
+    static const K kern[2][2] = {{dn_chunk_prep_kernel<false, false>, dn_chunk_prep_kernel<false, true>},
+                                 {dn_chunk_prep_kernel<true, false>, dn_chunk_prep_kernel<true, true>}};
+    static std::atomic<bool> attr{false};
+    if (!attr.load(std::memory_order_acquire)) {
+        for (int t = 0; t < 2; t++)
+            for (int c = 0; c < 2; c++)
+                ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern[t][c]),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, kPmLds));
+        attr.store(true, std::memory_order_release);
+    }
+    // a workgroup takes all value heads of its key head where that fills the
+    // chip (two workgroups per CU), else one (the Gram tiles formed again)
+    const bool each = G > 1 && (long)n_chunks * p.Hk < 2L * dev->num_cus;
+    p.per_wg = each ? 1 : G;
+    hipLaunchKernelGGL(kern[p.flags & ANELM_DN_ORDER_TRANSFORMERS ? 1 : 0][conv ? 1 : 0],
+                       dim3(n_chunks, p.Hk, each ? G : 1), dim3(kPmNT), kPmLds, st, p);
+    ANELM_LAUNCHED("dn_chunk_prep_kernel");
+    s.vrec = p.vrec;
+    s.krec = p.krec;
+    s.S = p.S;
+    s.Hk = p.Hk;
+    s.Hv = p.Hv;
+    s.n_chunks = n_chunks;
+    // grid = Hv * kSlabs, a multiple of 8 (XCD mapping inside the kernel)
+    hipLaunchKernelGGL(dn_chunk_scan_kernel, dim3(kSlabs * p.Hv), dim3(kMsNT), kMsLds, st, s);
+    ANELM_LAUNCHED("dn_chunk_scan_kernel");
+    return ANELM_OK;
 }
 
 }  // namespace
@@ -993,33 +1173,61 @@ extern "C" int anelm_deltanet_prefill(float* y, float* state, const float* q, co
         ANELM_LAUNCHED("dn_scan_kernel");
         return ANELM_OK;
     }
-    const int n_chunks = (S + kChunk - 1) / kChunk;
-    float* rec = static_cast<float*>(workspace((size_t)n_chunks * Hv * kCRec * sizeof(float), st));
-    if (!rec) return ANELM_ENOMEM;
-    static bool pm_attr = false;
-    if (!pm_attr) {
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dn_chunk_prep_mfma_kernel<true>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, kPmLds));
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dn_chunk_prep_mfma_kernel<false>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, kPmLds));
-        pm_attr = true;
-    }
-    if (flags & ANELM_DN_ORDER_TRANSFORMERS)
-        hipLaunchKernelGGL(dn_chunk_prep_mfma_kernel<true>, dim3(n_chunks, Hk), dim3(kPmNT), kPmLds, st, rec, q, k, v,
-                           a, b, A, dt_bias, S, Hk, Hv, flags);
-    else
-        hipLaunchKernelGGL(dn_chunk_prep_mfma_kernel<false>, dim3(n_chunks, Hk), dim3(kPmNT), kPmLds, st, rec, q, k,
-                           v, a, b, A, dt_bias, S, Hk, Hv, flags);
-    ANELM_LAUNCHED("dn_chunk_prep_mfma_kernel");
-    // grid = Hv * kSlabs, a multiple of 8 (XCD mapping inside the kernel)
-    static bool ms_attr = false;
-    if (!ms_attr) {
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dn_chunk_mfma_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, kMsLds));
-        ms_attr = true;
-    }
-    hipLaunchKernelGGL(dn_chunk_mfma_kernel, dim3(kSlabs * Hv), dim3(kMsNT), kMsLds, st, y, state, rec, S, Hv,
-                       n_chunks);
-    ANELM_LAUNCHED("dn_chunk_mfma_kernel");
-    return ANELM_OK;
+    ChunkArgs p{};
+    p.q = q;
+    p.k = k;
+    p.v = v;
+    p.a = a;
+    p.b = b;
+    p.as = Hv;
+    p.A = A;
+    p.dt_bias = dt_bias;
+    p.S = S;
+    p.Hk = Hk;
+    p.Hv = Hv;
+    p.flags = flags;
+    ScanArgs s{};
+    s.y = y;
+    s.state = state;
+    return chunk_prefill(p, s, false, st);
 }
+
+namespace anelm {
+// Chunked prefill straight from the projection rows (conv width 4).
+bool deltanet_prefill_proj_fits(const float* proj, const float* conv_w, int pd, int conv_kernel) {
+    return conv_kernel == 4 && pd % 4 == 0 &&
+           ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(conv_w)) & 15) == 0;
+}
+
+int deltanet_prefill_proj(float* y, float* state, float* conv_state, int conv_pos, const float* proj,
+                          const float* conv_w, const float* A, const float* dt_bias, int S, int Hk, int Hv, int pd,
+                          int flags, hipStream_t st) {
+    ANELM_REQUIRE(Hv / Hk <= kDK && (size_t)(S + kChunk) * Hv * kDV * sizeof(float) < 0x7fffffffu,
+                  "deltanet_prefill: %d tokens x %d heads exceed the 2 GiB output range", S, Hv);
+    ChunkArgs p{};
+    const int C = 2 * Hk * kDK + Hv * kDV;
+    p.proj = proj;
+    p.pd = pd;
+    p.conv_state = conv_state;
+    p.conv_w = conv_w;
+    p.conv_pos = conv_pos;
+    p.a = proj + C + Hv * kDV;
+    p.b = p.a + Hv;
+    p.as = pd;
+    p.A = A;
+    p.dt_bias = dt_bias;
+    p.S = S;
+    p.Hk = Hk;
+    p.Hv = Hv;
+    p.flags = flags;
+    ScanArgs s{};
+    s.y = y;
+    s.state = state;
+    s.conv_state = conv_state;
+    s.proj = proj;
+    s.pd = pd;
+    s.C = C;
+    s.conv_pos = conv_pos;
+    return chunk_prefill(p, s, true, st);
+}
+}  // namespace anelm

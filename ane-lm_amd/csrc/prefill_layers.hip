@@ -14,7 +14,9 @@
 //   gathered oldest to newest into one sequence [cached | prompt], row t sees
 //   only its last `capacity` keys, as the sliding ring gives the decode core,
 //   and the prompt's keys that survive are written to their slots at the end.
-// Gated DeltaNet (qwen3_5.cpp:849-908 per token):
+// Gated DeltaNet (qwen3_5.cpp:849-908 per token), conv width 4: the chunked
+// prefill reads the projection rows itself (deltanet.hip), then rmsnorm_gated
+// in place.  Other widths and unaligned rows:
 //   1. the causal conv1d over [conv ring | prompt] + SiLU per channel
 //      (cpu_ops.cpp:89-129, :6-13), split into q / k / v, with z, a, b
 //      gathered alongside; the ring keeps the prompt's last inputs;
@@ -428,6 +430,19 @@ extern "C" int anelm_deltanet_prefill_from_proj(float* y, float* state, float* c
     const int nqk = Hk * dk, C = 2 * nqk + Hv * dv, nz = Hv * dv, pd = C + nz + 2 * Hv;
     ANELM_REQUIRE((long)S * pd < 0x7fffffffL, "deltanet_prefill_from_proj: %d tokens too many", S);
     hipStream_t st = as_stream(stream);
+    // conv width 4 on aligned rows (the models'): the conv runs inside the
+    // chunk preparation and z is read where it lies, so nothing but y is
+    // written between (4096 tokens of 32 heads: the separate passes below took
+    // 77 us for the conv and the copies, and their arrays 330 MB)
+    const bool y8 = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(norm_w)) & 7) == 0;
+    if (deltanet_prefill_proj_fits(proj, conv_w, pd, conv_kernel) && (!gated || y8)) {
+        int rc = deltanet_prefill_proj(y, state, conv_state, *conv_pos, proj, conv_w, A, dt_bias, S, Hk, Hv, pd,
+                                       flags & 3, st);
+        if (rc == ANELM_OK && gated) rc = rmsnorm_gated_heads(y, proj + C, pd, norm_w, S, Hv, st);
+        if (rc) return rc;
+        *conv_pos = (int)((*conv_pos + (long)S) % (conv_kernel - 1));
+        return ANELM_OK;
+    }
     // q, k [S][nqk]; v, z, y [S][nz]; a, b [S][Hv] -- apart from the chunked
     // prefill's own workspace
     const size_t f = sizeof(float);
