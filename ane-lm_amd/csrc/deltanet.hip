@@ -407,7 +407,7 @@ __device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x
     sum += x1 * w.y;
     sum += x2 * w.z;
     const float y = sum + x3 * w.w;
-    return y / (expf(-y) + 1.0f);
+    return y * sigmoid_short(y);
 }
 
 // ------------------------------------------- chunk preparation on fp32 MFMA
@@ -424,9 +424,9 @@ __device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x
 //   wave 0 turns the diagonal 16x16 blocks of Am into T_rr = (I + A_rr)^-1
 //   by substitution, in place;
 //   for B = [beta V | beta exp(lgT) K] (64 x 256) the blocked forward
-//   substitution runs per 16-column tile of B (wave w owns tiles 2w, 2w + 1;
-//   it forms its tiles of B straight in the accumulator layout: V columns from
-//   memory, K columns from LDS):
+//   substitution runs per 16-column tile of B (wave w owns V tile w and K tile
+//   w; it forms them straight in the accumulator layout, V columns from memory,
+//   K columns from LDS):
 //     X_r = T_rr (B_r + sum_{s<r} Am_rs X_s),  X = [Ut | Wm]
 //   X tiles stay in registers: a result tile is the right operand of the next
 //   product.  Ut tiles are stored as they are, Wm tiles transposed in quads.
@@ -514,11 +514,8 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
             if (p.flags & ANELM_DN_L2NORM) {
                 float sk = kv[x].x * kv[x].x + kv[x].y * kv[x].y + kv[x].z * kv[x].z + kv[x].w * kv[x].w;
                 float sq = qv[x].x * qv[x].x + qv[x].y * qv[x].y + qv[x].z * qv[x].z + qv[x].w * qv[x].w;
-#pragma unroll
-                for (int m = 1; m < 32; m <<= 1) {
-                    sk += __shfl_xor(sk, m, 64);
-                    sq += __shfl_xor(sq, m, 64);
-                }
+                sk = wave_sum_from<16>(sk);   // over the row's 32 lanes
+                sq = wave_sum_from<16>(sq);
                 ik = 1.0f / sqrtf(sk + 1e-12f);
                 iq = 1.0f / sqrtf(sq + 1e-12f);
             }
@@ -577,44 +574,43 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
         int ltid = tid;
         asm volatile("" : "+v"(ltid));
         const int lane = ltid & 63, lm = lane & 15, lk = lane >> 4;
-        // this wave's memory operands, issued first: V rows of its B tiles
-        // (waves 0..3, tiles 0..7), rows 16 r + 4 lk + e (CONV: the inputs of
-        // the three tokens before them too)
-        const bool wpart = w >= 4;
-        float pre[2][4][4];
-        if (!wpart) {
+        // this wave's memory operands, issued first: V rows 16 r + 4 lk + e of
+        // its tile (CONV: the inputs of the three tokens before them too)
+        float pre[4][4];
+        if constexpr (CONV) {
+            const int cv = 2 * Hk * kDK + h * kDV + 16 * w + lm;
+            const float4 wv = *reinterpret_cast<const float4*>(p.conv_w + (size_t)cv * 4);
+            float x[4][7];
+            const float* pv = p.proj + (size_t)t0 * p.pd + cv;
+            const int ipd = (int)p.pd, last = S - 1 - t0;   // (rows of a chunk: 32-bit offsets)
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int col = 16 * (2 * w + u) + lm;
-                if constexpr (CONV) {
-                    const int cv = 2 * Hk * kDK + h * kDV + col;
-                    const float4 wv = *reinterpret_cast<const float4*>(p.conv_w + (size_t)cv * 4);
+            for (int r = 0; r < 4; r++)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        float x[7];
-#pragma unroll
-                        for (int i = 0; i < 7; i++) {
-                            const int tt = t0 + 16 * r + 4 * lk + i - 3;
-                            x[i] = p.proj[(size_t)min(max(tt, 0), S - 1) * p.pd + cv];
-                            if (r == 0 && i < 3 && tt < 0) x[i] = ring_input(p, cv, tt);
-                        }
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const float y = conv_tap4(x[e], x[e + 1], x[e + 2], x[e + 3], wv);
-                            pre[u][r][e] = 16 * r + 4 * lk + e < L ? y : 0.f;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const int t = 16 * r + 4 * lk + e;
-                            const float y = p.v[((size_t)(t0 + min(t, L - 1)) * Hv + h) * kDV + col];
-                            pre[u][r][e] = t < L ? y : 0.f;
-                        }
+                for (int i = 0; i < 7; i++) {
+                    int t = min(16 * r + 4 * lk + i - 3, last);
+                    if (r == 0 && i < 3) t = max(t, -t0);
+                    x[r][i] = pv[t * ipd];
                 }
+            if (t0 == 0 && lk == 0) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) x[0][i] = ring_input(p, cv, i - 3);
             }
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float y = conv_tap4(x[r][e], x[r][e + 1], x[r][e + 2], x[r][e + 3], wv);
+                    pre[r][e] = 16 * r + 4 * lk + e < L ? y : 0.f;
+                }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int t = 16 * r + 4 * lk + e;
+                    const float y = p.v[((size_t)(t0 + min(t, L - 1)) * Hv + h) * kDV + 16 * w + lm];
+                    pre[r][e] = t < L ? y : 0.f;
+                }
         }
         // ---- beta = sigmoid(b) and log decay = -A softplus(a + dt_bias)
         // (qwen3_5.cpp:896-898); lg[t + 1] = sum_{j <= t} log decay_j (wave 7)
@@ -658,7 +654,7 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int i = i0 + e;
-                const float f = expf(lgt - lg[i + 1]);
+                const float f = exp_short(lgt - lg[i + 1]);
                 if (isA) o4[e] = i < t ? bs * f * gram[u][e] : 0.f;
                 else o4[e] = i <= t ? f * gram[u][e] : 0.f;
             }
@@ -689,44 +685,43 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
             for (int t = 0; t < 16; t++) Am[sw64(16 * b + t, 16 * b + j)] = x[t];
         }
         lds_barrier();
-        // ---- X for column tiles jt = 2w + u of B
+        // ---- X of this wave's two tiles (u 0: V, u 1: K), block row by block row
         v4f X[2][4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
+            // B_r in the accumulator layout: rows 16 r + 4 lk + e, column lm
+            v4f acc[2], xr[2];
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int jt = 2 * w + u;
-                // B_r of this tile in the accumulator layout: rows 16 r + 4 lk + e, column lm
-                v4f acc;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = 16 * r + 4 * lk + e;
-                    acc[e] = bt[t] * (wpart ? Ks[sw128(t, 16 * (jt - 8) + lm)] * eb[t] : pre[u][r][e]);
-                }
-#pragma unroll
-                for (int s2 = 0; s2 < r; s2++) {
-                    const float4 a4 = *reinterpret_cast<const float4*>(Am + sw64(16 * r + lm, 16 * s2 + 4 * lk));
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.x, X[u][s2][0], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.y, X[u][s2][1], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.z, X[u][s2][2], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.w, X[u][s2][3], acc, 0, 0, 0);
-                }
-                const float4 t4 = *reinterpret_cast<const float4*>(Am + sw64(16 * r + lm, 16 * r + 4 * lk));
-                v4f xr = {0.f, 0.f, 0.f, 0.f};
-                xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.x, acc[0], xr, 0, 0, 0);
-                xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.y, acc[1], xr, 0, 0, 0);
-                xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.z, acc[2], xr, 0, 0, 0);
-                xr = __builtin_amdgcn_mfma_f32_16x16x4f32(t4.w, acc[3], xr, 0, 0, 0);
-                X[u][r] = xr;
-                // Ut: the D fragment; Wm: transposed in quads, lane (4 c + i, k)
-                // then holds row 4 k + i, columns 4 c .. 4 c + 3 of its A fragment
-                if (wpart)
-                    *reinterpret_cast<v4f*>(out + kVW + ((r * 8 + jt - 8) * 64 + 4 * lk + (lm & 3) + 16 * (lm >> 2)) * 4) =
-                        quad_transpose(xr, lane);
-                else
-                    *reinterpret_cast<v4f*>(out + ((r * 8 + jt) * 64 + lane) * 4) = xr;
-                __builtin_amdgcn_sched_barrier(0);   // bounds the loads hoisted ahead of this tile
+            for (int e = 0; e < 4; e++) {
+                const int t = 16 * r + 4 * lk + e;
+                const float bv = bt[t];
+                acc[0][e] = bv * pre[r][e];
+                acc[1][e] = bv * (Ks[sw128(t, 16 * w + lm)] * eb[t]);
             }
+#pragma unroll
+            for (int s2 = 0; s2 < r; s2++) {
+                const v4f a4 = *reinterpret_cast<const v4f*>(Am + sw64(16 * r + lm, 16 * s2 + 4 * lk));
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], X[u][s2][e], acc[u], 0, 0, 0);
+            }
+            const v4f t4 = *reinterpret_cast<const v4f*>(Am + sw64(16 * r + lm, 16 * r + 4 * lk));
+            xr[0] = xr[1] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    xr[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(t4[e], acc[u][e], xr[u], 0, 0, 0);
+            X[0][r] = xr[0];
+            X[1][r] = xr[1];
+            // Ut: the D fragment; Wm: transposed in quads, lane (4 c + i, k)
+            // then holds row 4 k + i, columns 4 c .. 4 c + 3 of its A fragment
+            *reinterpret_cast<v4f*>(out + ((r * 8 + w) * 64 + lane) * 4) = xr[0];
+            *reinterpret_cast<v4f*>(out + kVW + ((r * 8 + w) * 64 + 4 * lk + (lm & 3) + 16 * (lm >> 2)) * 4) =
+                quad_transpose(xr[1], lane);
+            __builtin_amdgcn_sched_barrier(0);   // bounds the loads hoisted ahead of this row
         }
         lds_barrier();   // Am, lg and beta are rewritten for the next value head
     }
@@ -739,72 +734,25 @@ constexpr int kSlabs = kDV / kSeqCB;
 // ------------------------------------------------ chunk scan on fp32 MFMA
 // The state products per chunk on v_mfma_f32_16x16x4_f32 (fp32 inputs, fp32
 // accumulation).  A workgroup (8 waves, two per SIMD) owns a 16-column slab of
-// one head's state, kept in LDS column-major (Sc[c][i]):
-//   waves 0-3: X = Wm S0 for chunk rows [16 w, 16 w + 16), U = Ut - X and its
-//              decayed copy to LDS (column-major);
-//   waves 4-7: Y = Q S0 for chunk rows [16 (w - 4), ...), kept in registers;
-//   then wave w: S = gC S0 + K^T (decayed U) for state rows [16 w, 16 w + 16),
-//   and waves 4-7 y = diag(exp(lg)) Y + P U.
-// Every operand but the state and U is read by one wave only, so it goes from
+// one head's state.  Only X = Wm S0 -> U -> S_end stands between one chunk and
+// the next, so the waves split by role:
+//   waves 0-3 (one per SIMD, raised priority) carry the state: X of chunk rows
+//     [16 w, 16 w + 16), U = Ut - X and its decayed copy to LDS | barrier |
+//     S = gC S + K^T (decayed U) of state rows [32 w, 32 w + 32), kept in
+//     registers and published to the other of two LDS slabs | barrier;
+//   waves 4-7 form the outputs of chunk rows [16 (w - 4), ...) in their wake:
+//     the first half of Q S0 beside the state update, the second half and
+//     diag(exp(lg)) (.) + P U beside the next chunk's X (the slab and U of a
+//     chunk stay in LDS until then).
+// Every operand but the slab and U is read by one wave only, so it goes from
 // memory straight into registers (1 KiB fragments), the next chunk's loads
-// spread over this chunk's products; LDS carries only the state slab and U.
+// spread over this chunk's products: issued all at once they fill the CU's
+// memory queue and the waves stall at their next memory instruction.
 // Bound: @SCAN@
 constexpr int kMsNT = 512;
-constexpr int kScP = kDK + 4;        // Sc row pitch (floats): 16-byte reads of 16 lanes hit distinct banks
+constexpr int kScP = kDK + 4;        // slab column pitch (floats): 16-byte reads of 16 lanes hit distinct banks
 constexpr int kUlP = kChunk + 4;     // U column pitch, likewise
-constexpr int kMsLds = kSeqCB * (kScP + 2 * kUlP) * 4;
-
-// One wave's operands of one chunk.
-struct ScanOps {
-    v4f m[8];     // Wm (waves 0-3) or Q (4-7), row tile w & 3
-    v4f kt[4];    // K^T row tile w
-    v4f u;        // waves 0-3: Ut, row tile w, this slab's column tile
-    v4f p[4];     // waves 4-7: P tiles (w - 4, x <= w - 4)
-    v4f ev;       // rows 16 (w & 3) + 4 lq + (0..3) of exp(lg_L - lg) (waves 0-3) or exp(lg) (4-7)
-    float gc;
-};
-
-// Where one wave's operands of chunk ch lie: its records as buffer resources
-// (offsets stay small for any sequence length); operands a wave does not have
-// are out of range and read zeros.
-struct ScanSrc {
-    __amdgpu_buffer_rsrc_t rv, rk;
-    __amdgpu_buffer_rsrc_t rm;        // the one that holds m
-    int mo, ko, uo, po, eo;           // byte offsets of this lane's first element
-};
-
-__device__ __forceinline__ ScanSrc scan_src(const float* vrec, const float* krec, int ch, int Hk, int Hv, int h, int w,
-                                            int lane, int slab) {
-    ScanSrc s;
-    const int mt = w & 3;
-    s.rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vrec) + ((size_t)ch * Hv + h) * kVRec, 0, kVRec * 4,
-                                             0x00020000);
-    s.rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(krec) + ((size_t)ch * Hk + h / (Hv / Hk)) * kKRec, 0,
-                                             kKRec * 4, 0x00020000);
-    s.rm = w < 4 ? s.rv : s.rk;
-    s.mo = ((w < 4 ? kVW : 0) + (mt * 8 * 64 + lane) * 4) * 4;
-    s.ko = (kKT + (w * 4 * 64 + lane) * 4) * 4;
-    s.uo = w < 4 ? ((mt * 8 + slab) * 64 + lane) * 16 : 0x7ffffff0;
-    s.po = (kVP + (mt * (mt + 1) / 2 * 64 + lane) * 4) * 4;
-    s.eo = (kVE + (w < 4 ? 64 : 0) + 16 * mt + 4 * (lane >> 4)) * 4;
-    return s;
-}
-
-// Part x (0..7) of a wave's loads of one chunk.  The parts are issued between
-// the MFMA groups of the previous chunk's products: issued all at once, the
-// workgroup's loads fill the CU's memory queue and the waves stall at their
-// next memory instruction instead of computing.
-__device__ __forceinline__ void scan_part(ScanOps& o, const ScanSrc& s, int w, int x) {
-    auto ld = [](__amdgpu_buffer_rsrc_t r, int off) __attribute__((always_inline)) {
-        return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    };
-    o.m[x] = ld(s.rm, s.mo + x * 1024);
-    if (x < 4) o.kt[x] = ld(s.rk, s.ko + x * 1024);
-    else o.p[x - 4] = ld(s.rv, w >= 4 + (x - 4) ? s.po + (x - 4) * 1024 : 0x7ffffff0);
-    if (x == 0) o.u = ld(s.rv, s.uo);
-    if (x == 1) o.ev = ld(s.rv, s.eo);
-    if (x == 2) o.gc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s.rv, (kVE + 128) * 4, 0, 0));
-}
+constexpr int kMsLds = kSeqCB * (2 * kScP + 3 * kUlP) * 4;
 
 struct ScanArgs {
     float* y;              // [S][Hv][dv]
@@ -820,12 +768,45 @@ struct ScanArgs {
     int C, conv_pos;
 };
 
+// The two records of chunk ch for head h, as buffer resources (offsets stay
+// small for any sequence length).
+struct ScanSrc {
+    __amdgpu_buffer_rsrc_t rv, rk;
+};
+__device__ __forceinline__ ScanSrc scan_src(const ScanArgs& a, int ch, int h) {
+    ch = min(ch, a.n_chunks - 1);   // (past the last chunk: its operands again, unused)
+    ScanSrc s;
+    s.rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.vrec) + ((size_t)ch * a.Hv + h) * kVRec, 0, kVRec * 4,
+                                             0x00020000);
+    s.rk = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.krec) + ((size_t)ch * a.Hk + h / (a.Hv / a.Hk)) * kKRec, 0, kKRec * 4, 0x00020000);
+    return s;
+}
+__device__ __forceinline__ v4f scan_ld(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+// Operands of one chunk: a state wave's, an output wave's.
+struct StateOps {
+    v4f m[8];       // Wm row tile w
+    v4f kt[2][4];   // K^T row tiles 2w, 2w + 1
+    v4f u, ev;      // Ut (row tile w, this slab's columns); exp(lg_L - lg) of its rows
+    float gc;
+};
+struct OutOps {
+    v4f q[8];       // Q row tile mt
+    v4f p[4];       // P tiles (mt, x <= mt)
+    v4f ev;         // exp(lg) of its rows
+};
+
 __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dn_chunk_scan_kernel(
     const ScanArgs a) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
-    float (*Sc)[kScP] = reinterpret_cast<float (*)[kScP]>(smem);                   // state slab
-    float (*Ul)[kUlP] = reinterpret_cast<float (*)[kUlP]>(smem + kSeqCB * kScP);   // U of the chunk, by column
-    float (*Ud)[kUlP] = Ul + kSeqCB;                                               // its decayed copy
+    typedef float (*Slab)[kScP];
+    typedef float (*Ucols)[kUlP];
+    Slab Sc = reinterpret_cast<Slab>(smem);                            // [2 x 16] columns: slab of even / odd chunks
+    Ucols Ul = reinterpret_cast<Ucols>(smem + 2 * kSeqCB * kScP);      // [2 x 16] U of even / odd chunks
+    Ucols Ud = Ul + 2 * kSeqCB;                                        // decayed U of this chunk
     const int S = a.S, Hv = a.Hv, n_chunks = a.n_chunks;
     // XCD-aware: the 8 slabs of a head share its chunk records, so they go to
     // one XCD (workgroup id mod 8 selects the XCD; Hv * 8 workgroups)
@@ -837,17 +818,6 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     const int lr = lane & 15, lq = lane >> 4;
     const int mt = w & 3;
     const int c0 = slab * kSeqCB;
-    const __amdgpu_buffer_rsrc_t ry =
-        __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (int)((size_t)S * Hv * kDV * 4), 0x00020000);
-
-    // two operand sets, A and B: a chunk is computed from one while the next
-    // chunk's loads land in the other (no register copies between them)
-    ScanOps opA, opB;
-    {
-        const ScanSrc s0 = scan_src(a.vrec, a.krec, 0, a.Hk, Hv, h, w, lane, slab);
-#pragma unroll
-        for (int x = 0; x < 8; x++) scan_part(opA, s0, w, x);
-    }
     float* Sp = a.state + (size_t)h * kDK * kDV;
     for (int e = tid; e < kDK * kSeqCB; e += kMsNT) {
         const int i = e / kSeqCB, c = e % kSeqCB;
@@ -860,90 +830,193 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
             a.conv_state[(size_t)c * 3 + (a.conv_pos + t) % 3] = a.proj[(size_t)t * a.pd + c];
         }
     }
-    __syncthreads();
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
 
-    auto chunk = [&](const ScanOps& cur, ScanOps& nxt, int ch) __attribute__((always_inline)) {
-        // the next chunk's operands (the last chunk reloads its own: no branch)
-        const ScanSrc src = scan_src(a.vrec, a.krec, ch + 1 < n_chunks ? ch + 1 : ch, a.Hk, Hv, h, w, lane, slab);
-        // ---- X = Wm S0 (waves 0-3) or Y = Q S0 (waves 4-7): 32 MFMAs in 4
-        // chains, one part of the next chunk's loads ahead of each group of 4
-        v4f sb[8];
+    if (w < 4) {
+        // ------------------------------------------------ state waves
+        const int mo = (kVW + (mt * 8 * 64 + lane) * 4) * 4, ko = (kKT + (mt * 8 * 64 + lane) * 4) * 4;
+        const int uo = ((mt * 8 + slab) * 64 + lane) * 16, eo = (kVE + 64 + 16 * mt + 4 * lq) * 4;
+        // two operand sets: a chunk is computed from one while the next
+        // chunk's loads land in the other (no register copies between them)
+        StateOps opA, opB;
+        {
+            const ScanSrc s = scan_src(a, 0, h);
 #pragma unroll
-        for (int x = 0; x < 8; x++) sb[x] = *reinterpret_cast<const v4f*>(&Sc[lr][16 * x + 4 * lq]);
-        v4f Z[4];
+            for (int x = 0; x < 8; x++) opA.m[x] = scan_ld(s.rv, mo + x * 1024);
+            opA.u = scan_ld(s.rv, uo);
+            opA.ev = scan_ld(s.rv, eo);
+            opA.gc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s.rv, (kVE + 128) * 4, 0, 0));
 #pragma unroll
-        for (int e = 0; e < 4; e++) Z[e] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int x = 0; x < 8; x++) {
-            scan_part(nxt, src, w, x);
-            __builtin_amdgcn_sched_barrier(0);   // the part is issued here, not hoisted or sunk
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.m[x][e], sb[x][e], Z[e], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int x = 0; x < 8; x++) opA.kt[x >> 2][x & 3] = scan_ld(s.rk, ko + x * 1024);
         }
-        // element j is chunk row 16 mt + 4 lq + j, slab column lr
-        v4f Zs = (Z[0] + Z[1]) + (Z[2] + Z[3]);
-        if (w < 4) {
-            const v4f U = cur.u - Zs;
-            *reinterpret_cast<v4f*>(&Ul[lr][16 * mt + 4 * lq]) = U;
+        __builtin_amdgcn_s_setprio(2);
+        __syncthreads();
+        v4f Sr[2];   // this wave's state rows: 32 w + 16 t + 4 lq + (0..3), column lr
+#pragma unroll
+        for (int t = 0; t < 2; t++) Sr[t] = *reinterpret_cast<const v4f*>(&Sc[lr][32 * mt + 16 * t + 4 * lq]);
+        auto chunk = [&](const StateOps& cur, StateOps& nxt, int ch, int par) __attribute__((always_inline)) {
+            const ScanSrc src = scan_src(a, ch + 1, h);
+            Slab sc = Sc + par * kSeqCB;
+            v4f sb[8], Z[4];
+#pragma unroll
+            for (int x = 0; x < 8; x++) sb[x] = *reinterpret_cast<const v4f*>(&sc[lr][16 * x + 4 * lq]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) Z[e] = zero;
+            // ---- X = Wm S0: 32 products in 4 chains
+#pragma unroll
+            for (int x = 0; x < 8; x++) {
+                nxt.m[x] = scan_ld(src.rv, mo + x * 1024);
+                if (x == 6) nxt.u = scan_ld(src.rv, uo);
+                __builtin_amdgcn_sched_barrier(0);   // the loads are issued here, not hoisted or sunk
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.m[x][e], sb[x][e], Z[e], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // element j is chunk row 16 w + 4 lq + j, slab column lr
+            const v4f U = cur.u - ((Z[0] + Z[1]) + (Z[2] + Z[3]));
             *reinterpret_cast<v4f*>(&Ud[lr][16 * mt + 4 * lq]) = U * cur.ev;
+            *reinterpret_cast<v4f*>(&(Ul + par * kSeqCB)[lr][16 * mt + 4 * lq]) = U;
+            lds_barrier();   // U complete
+            // ---- S = gC S + K^T Ud: 2 row tiles, 16 products each in 2 chains
+            v4f ub[4], T[2][2];
+#pragma unroll
+            for (int x = 0; x < 4; x++) ub[x] = *reinterpret_cast<const v4f*>(&Ud[lr][16 * x + 4 * lq]);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                T[t][0] = cur.gc * Sr[t];
+                T[t][1] = zero;
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                nxt.kt[0][x] = scan_ld(src.rk, ko + x * 1024);
+                nxt.kt[1][x] = scan_ld(src.rk, ko + (4 + x) * 1024);
+                if (x == 2) nxt.ev = scan_ld(src.rv, eo);
+                if (x == 3)
+                    nxt.gc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src.rv, (kVE + 128) * 4, 0, 0));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+                        T[t][e & 1] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(cur.kt[t][x][e], ub[x][e], T[t][e & 1], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            sc = Sc + (par ^ 1) * kSeqCB;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                Sr[t] = T[t][0] + T[t][1];
+                *reinterpret_cast<v4f*>(&sc[lr][32 * mt + 16 * t + 4 * lq]) = Sr[t];
+            }
+            lds_barrier();   // new state complete
+        };
+        // pairs of chunks, then an odd last one: inside the loop both halves run
+        // unconditionally, so the loads a half issues for the other are not sunk
+        // into a conditional block next to their use
+        int ch = 0;
+        for (; ch + 1 < n_chunks; ch += 2) {
+            chunk(opA, opB, ch, 0);
+            chunk(opB, opA, ch + 1, 1);
         }
-        lds_barrier();   // U complete; every wave's reads of S0 are done
-        // ---- S = gC S0 + K^T Ud for state rows 16 w + (0..15): 16 MFMAs in 4 chains
-        v4f ub[4];
+        if (ch < n_chunks) chunk(opA, opB, ch, 0);
 #pragma unroll
-        for (int x = 0; x < 4; x++) ub[x] = *reinterpret_cast<const v4f*>(&Ud[lr][16 * x + 4 * lq]);
-        v4f* srow = reinterpret_cast<v4f*>(&Sc[lr][16 * w + 4 * lq]);
-        v4f Sn[4];
-        Sn[0] = cur.gc * *srow;
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int e = 1; e < 4; e++) Sn[e] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < 4; j++) Sp[(size_t)(32 * mt + 16 * t + 4 * lq + j) * kDV + c0 + lr] = Sr[t][j];
+    } else {
+        // ------------------------------------------------ output waves
+        const __amdgpu_buffer_rsrc_t ry =
+            __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (int)((size_t)S * Hv * kDV * 4), 0x00020000);
+        const int qo = (mt * 8 * 64 + lane) * 16, po = (kVP + (mt * (mt + 1) / 2 * 64 + lane) * 4) * 4;
+        const int eo = (kVE + 16 * mt + 4 * lq) * 4;
+        OutOps opA, opB;
+        v4f Z[4];
+        // second half of the operands of chunk ch (the first half is loaded a step earlier)
+        auto load2 = [&](OutOps& o, const ScanSrc& s, int x) __attribute__((always_inline)) {
+            o.q[4 + x] = scan_ld(s.rk, qo + (4 + x) * 1024);
+            o.p[x] = x <= mt ? scan_ld(s.rv, po + x * 1024) : zero;
+            if (x == 0) o.ev = scan_ld(s.rv, eo);
+        };
+        // Q S0 of chunk ch, state rows 0..63, the first operands of chunk ch + 1 requested
+        auto first = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
+            const ScanSrc src = scan_src(a, ch + 1, h);
+            Slab sc = Sc + par * kSeqCB;
 #pragma unroll
-        for (int x = 0; x < 4; x++)
+            for (int e = 0; e < 4; e++) Z[e] = zero;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                Sn[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.kt[x][e], ub[x][e], Sn[e], 0, 0, 0);
-        // rows written here are read (as C) only by this wave
-        *srow = (Sn[0] + Sn[1]) + (Sn[2] + Sn[3]);
-        // ---- y = diag(exp(lg)) Y + P U (waves 4-7; the others' products and
-        // stores are skipped and dropped)
-        if (w >= 4) {
-            v4f y0 = Zs * cur.ev, y1 = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int x = 0; x < 4; x++) {
+                nxt.q[x] = scan_ld(src.rk, qo + x * 1024);
+                const v4f sb = *reinterpret_cast<const v4f*>(&sc[lr][16 * x + 4 * lq]);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[x][e], sb[e], Z[e], 0, 0, 0);
+            }
+        };
+        // the rest of chunk ch's outputs, the other operands of chunk ch + 1 requested
+        auto finish = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
+            const ScanSrc src = scan_src(a, ch + 1, h);
+            Slab sc = Sc + par * kSeqCB;
+            Ucols ul = Ul + par * kSeqCB;
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                load2(nxt, src, x);
+                const v4f sb = *reinterpret_cast<const v4f*>(&sc[lr][64 + 16 * x + 4 * lq]);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[4 + x][e], sb[e], Z[e], 0, 0, 0);
+            }
+            v4f y0 = ((Z[0] + Z[1]) + (Z[2] + Z[3])) * cur.ev, y1 = zero;
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 if (x > mt) break;
-                const v4f uv = *reinterpret_cast<const v4f*>(&Ul[lr][16 * x + 4 * lq]);
+                const v4f uv = *reinterpret_cast<const v4f*>(&ul[lr][16 * x + 4 * lq]);
                 y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][0], uv[0], y0, 0, 0, 0);
                 y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][1], uv[1], y1, 0, 0, 0);
                 y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][2], uv[2], y0, 0, 0, 0);
                 y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][3], uv[3], y1, 0, 0, 0);
             }
-            Zs = y0 + y1;
-        }
-        lds_barrier();   // new state complete, U consumed
-        // y rows past S fall out of the buffer range and are dropped, as are
-        // the stores of waves 0-3 (every wave has the same operations in
-        // flight, so the waits for operands count the same everywhere)
+            const v4f y = y0 + y1;
+            // rows past S fall out of the buffer range and are dropped
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float yv = Zs[j];
-            const int off = (((ch * kChunk + 16 * mt + 4 * lq + j) * Hv + h) * kDV + c0 + lr) * 4;
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ry, w >= 4 ? off : 0x7ffffff0, 0, 0);
+            for (int j = 0; j < 4; j++) {
+                const float yv = y[j];
+                const int off = (((ch * kChunk + 16 * mt + 4 * lq + j) * Hv + h) * kDV + c0 + lr) * 4;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ry, off, 0, 0);
+            }
+        };
+        {
+            const ScanSrc s = scan_src(a, 0, h);
+#pragma unroll
+            for (int x = 0; x < 4; x++) opA.q[x] = scan_ld(s.rk, qo + x * 1024);
+#pragma unroll
+            for (int x = 0; x < 4; x++) load2(opA, s, x);
         }
-    };
-    // pairs of chunks, then an odd last one: inside the loop both halves run
-    // unconditionally, so the loads a half issues for the other are not sunk
-    // into a conditional block next to their use
-    int ch = 0;
-    for (; ch + 1 < n_chunks; ch += 2) {
-        chunk(opA, opB, ch);
-        chunk(opB, opA, ch + 1);
-    }
-    if (ch < n_chunks) chunk(opA, opB, ch);
-    for (int e = tid; e < kDK * kSeqCB; e += kMsNT) {
-        const int i = e / kSeqCB, c = e % kSeqCB;
-        Sp[(size_t)i * kDV + c0 + c] = Sc[c][i];
+        __syncthreads();
+        lds_barrier();
+        first(opA, opB, 0, 0);
+        lds_barrier();
+        // (the state waves' chunk ch: finish ch - 1 | barrier | first half of ch | barrier)
+        int ch = 1;
+        for (; ch + 1 < n_chunks; ch += 2) {
+            finish(opA, opB, ch - 1, 0);
+            lds_barrier();
+            first(opB, opA, ch, 1);
+            lds_barrier();
+            finish(opB, opA, ch, 1);
+            lds_barrier();
+            first(opA, opB, ch + 1, 0);
+            lds_barrier();
+        }
+        if (ch < n_chunks) {
+            finish(opA, opB, ch - 1, 0);
+            lds_barrier();
+            first(opB, opA, ch, 1);
+            lds_barrier();
+            finish(opB, opA, ch, 1);
+        } else {
+            finish(opA, opB, ch - 1, 0);
+        }
     }
 }
 
