@@ -432,6 +432,9 @@ __device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x
 //   product.  Ut tiles are stored as they are, Wm tiles transposed in quads.
 // LDS matrices are row-major with 16-byte chunks XOR-swizzled by (row & 15);
 // 66 KB, so two workgroups share a CU (one's serial phases overlap the other).
+// Bound: memory (134 MB read, 224 MB of records written for 4096 tokens of 32
+// heads: 65 us at 5.5 TB/s) and the vector units (conv and SiLU): 102 us, where
+// conv pass and preparation took 77 + 140.
 constexpr int kPmNT = 512;
 constexpr int kPmK = 0;                        // K rows [64][128]
 constexpr int kPmR = kCMat;                    // Q rows [64][128] for the Gram tiles, then:
@@ -542,6 +545,44 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
             *reinterpret_cast<v4f*>(kr + kKT + ((w * 4 + x) * 64 + lane) * 4) = kt;
         }
     }
+    // A value head's memory operands, requested ahead of the phase before their
+    // use: the V rows 16 r + 4 lk + e of the wave's tile (CONV: the inputs of
+    // the three tokens before them too), and token `lane`'s gates
+    constexpr int NI = CONV ? 7 : 4;
+    float vx[4][NI], ga = 0.f, gb = 0.f;
+    float4 wv = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_head = [&](int h) __attribute__((always_inline)) {
+        int lt = threadIdx.x & 63;
+        asm volatile("" : "+v"(lt));   // (addresses are formed here, not held)
+        const int lm = lt & 15, lk = lt >> 4;
+        // (rows of a chunk: 32-bit offsets)
+        const int last = S - 1 - t0, col = 16 * w + lm;
+        const int pd = CONV ? (int)p.pd : Hv * kDV;
+        const int cv = CONV ? 2 * Hk * kDK + h * kDV + col : h * kDV + col;
+        const float* pv = (CONV ? p.proj : p.v) + (size_t)t0 * pd + cv;
+        if constexpr (CONV) wv = *reinterpret_cast<const float4*>(p.conv_w + (size_t)cv * 4);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                int t = min(16 * r + 4 * lk + i - (NI - 4), last);
+                if (r == 0 && i < NI - 4) t = max(t, -t0);
+                vx[r][i] = pv[t * pd];
+            }
+        if constexpr (CONV) {
+            if (t0 == 0 && lk == 0) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) vx[0][i] = ring_input(p, cv, i - 3);
+            }
+        }
+        if (w == 7) {
+            const size_t gi = (size_t)(t0 + min(lt, L - 1)) * p.as + h;
+            ga = p.a[gi];
+            gb = p.b[gi];
+        }
+    };
+    const int h0 = kh * (Hv / Hk) + blockIdx.z * p.per_wg;
+    load_head(h0);
     // ---- Gram tiles: 10 lower tiles of K K^T (ids 0..9) and of Q K^T (10..19);
     // wave w takes ids w, w + 8, w + 16.  Element e of lane (lm, lk) is row
     // 16 ti + lm, column 16 tj + 4 lk + e
@@ -568,59 +609,30 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
     }
     lds_barrier();   // the query rows are no longer read: their space takes Am
     for (int g = 0; g < p.per_wg; g++) {
-        const int h = kh * (Hv / Hk) + blockIdx.z * p.per_wg + g;
+        const int h = h0 + g;
         float* out = p.vrec + ((size_t)c * Hv + h) * kVRec;
         // lane-derived addresses are recomputed per value head, not held across the loop
         int ltid = tid;
         asm volatile("" : "+v"(ltid));
         const int lane = ltid & 63, lm = lane & 15, lk = lane >> 4;
-        // this wave's memory operands, issued first: V rows 16 r + 4 lk + e of
-        // its tile (CONV: the inputs of the three tokens before them too)
+        // this head's V rows 16 r + 4 lk + e, column lm of the wave's tile
         float pre[4][4];
-        if constexpr (CONV) {
-            const int cv = 2 * Hk * kDK + h * kDV + 16 * w + lm;
-            const float4 wv = *reinterpret_cast<const float4*>(p.conv_w + (size_t)cv * 4);
-            float x[4][7];
-            const float* pv = p.proj + (size_t)t0 * p.pd + cv;
-            const int ipd = (int)p.pd, last = S - 1 - t0;   // (rows of a chunk: 32-bit offsets)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int i = 0; i < 7; i++) {
-                    int t = min(16 * r + 4 * lk + i - 3, last);
-                    if (r == 0 && i < 3) t = max(t, -t0);
-                    x[r][i] = pv[t * ipd];
-                }
-            if (t0 == 0 && lk == 0) {
-#pragma unroll
-                for (int i = 0; i < 3; i++) x[0][i] = ring_input(p, cv, i - 3);
+            for (int e = 0; e < 4; e++) {
+                float y;
+                if constexpr (CONV) y = conv_tap4(vx[r][e], vx[r][e + 1], vx[r][e + 2], vx[r][e + 3], wv);
+                else y = vx[r][e];
+                pre[r][e] = 16 * r + 4 * lk + e < L ? y : 0.f;
             }
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float y = conv_tap4(x[r][e], x[r][e + 1], x[r][e + 2], x[r][e + 3], wv);
-                    pre[r][e] = 16 * r + 4 * lk + e < L ? y : 0.f;
-                }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = 16 * r + 4 * lk + e;
-                    const float y = p.v[((size_t)(t0 + min(t, L - 1)) * Hv + h) * kDV + 16 * w + lm];
-                    pre[r][e] = t < L ? y : 0.f;
-                }
-        }
         // ---- beta = sigmoid(b) and log decay = -A softplus(a + dt_bias)
         // (qwen3_5.cpp:896-898); lg[t + 1] = sum_{j <= t} log decay_j (wave 7)
         if (w == 7) {
-            const bool in = lane < L;
             float x = 0.f, bv = 0.f;
-            if (in) {
-                const size_t gi = (size_t)(t0 + lane) * p.as + h;
-                bv = 1.0f / (1.0f + expf(-p.b[gi]));
-                x = -p.A[h] * logf(1.0f + expf(p.a[gi] + p.dt_bias[h]));
+            if (lane < L) {
+                bv = 1.0f / (1.0f + expf(-gb));
+                x = -p.A[h] * logf(1.0f + expf(ga + p.dt_bias[h]));
             }
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
@@ -685,6 +697,7 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
             for (int t = 0; t < 16; t++) Am[sw64(16 * b + t, 16 * b + j)] = x[t];
         }
         lds_barrier();
+        if (g + 1 < p.per_wg) load_head(h + 1);
         // ---- X of this wave's two tiles (u 0: V, u 1: K), block row by block row
         v4f X[2][4];
 #pragma unroll
@@ -748,7 +761,9 @@ constexpr int kSlabs = kDV / kSeqCB;
 // memory straight into registers (1 KiB fragments), the next chunk's loads
 // spread over this chunk's products: issued all at once they fill the CU's
 // memory queue and the waves stall at their next memory instruction.
-// Bound: @SCAN@
+// Bound: the fp32 matrix units and the chain above: a chunk takes 5300 clocks
+// of which 3400 are the two waves' products; 4096 tokens of 32 heads 158 us
+// (195 with all waves on both roles, 270 with row-major records too).
 constexpr int kMsNT = 512;
 constexpr int kScP = kDK + 4;        // slab column pitch (floats): 16-byte reads of 16 lanes hit distinct banks
 constexpr int kUlP = kChunk + 4;     // U column pitch, likewise
@@ -799,6 +814,109 @@ struct OutOps {
     v4f ev;         // exp(lg) of its rows
 };
 
+// Wave 4 + MT of the scan: the outputs of chunk rows [16 MT, 16 MT + 16).
+template <int MT>
+__device__ __forceinline__ void scan_outputs(const ScanArgs& a, float (*Sc)[kScP], float (*Ul)[kUlP], int h, int c0,
+                                             int lane) {
+    const int lr = lane & 15, lq = lane >> 4, Hv = a.Hv, n_chunks = a.n_chunks;
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    const __amdgpu_buffer_rsrc_t ry =
+        __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (int)((size_t)a.S * Hv * kDV * 4), 0x00020000);
+    const int qo = (MT * 8 * 64 + lane) * 16, po = (kVP + (MT * (MT + 1) / 2 * 64 + lane) * 4) * 4;
+    const int eo = (kVE + 16 * MT + 4 * lq) * 4;
+    OutOps opA, opB;
+    v4f Z[4];
+    // part x (0..3) of a chunk's second loads (the first four Q tiles are loaded a step earlier)
+    auto load2 = [&](OutOps& o, const ScanSrc& s, int x) __attribute__((always_inline)) {
+        o.q[4 + x] = scan_ld(s.rk, qo + (4 + x) * 1024);
+        if (x <= MT) o.p[x] = scan_ld(s.rv, po + x * 1024);
+        if (x == 0) o.ev = scan_ld(s.rv, eo);
+    };
+    // Q S0 of chunk ch, state rows 0..63, the first operands of chunk ch + 1 requested
+    auto first = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
+        const ScanSrc src = scan_src(a, ch + 1, h);
+        float (*sc)[kScP] = Sc + par * kSeqCB;
+        v4f sb[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) sb[x] = *reinterpret_cast<const v4f*>(&sc[lr][16 * x + 4 * lq]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) Z[e] = zero;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            nxt.q[x] = scan_ld(src.rk, qo + x * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[x][e], sb[x][e], Z[e], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // the rest of chunk ch's outputs, the other operands of chunk ch + 1 requested
+    auto finish = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
+        const ScanSrc src = scan_src(a, ch + 1, h);
+        float (*sc)[kScP] = Sc + par * kSeqCB;
+        float (*ul)[kUlP] = Ul + par * kSeqCB;
+        v4f uv[MT + 1], sb[4], T[4];
+#pragma unroll
+        for (int x = 0; x <= MT; x++) uv[x] = *reinterpret_cast<const v4f*>(&ul[lr][16 * x + 4 * lq]);
+#pragma unroll
+        for (int x = 0; x < 4; x++) sb[x] = *reinterpret_cast<const v4f*>(&sc[lr][64 + 16 * x + 4 * lq]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) T[e] = zero;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            load2(nxt, src, x);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (x <= MT) T[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][e], uv[x][e], T[e], 0, 0, 0);
+                Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[4 + x][e], sb[x][e], Z[e], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const v4f y = ((Z[0] + Z[1]) + (Z[2] + Z[3])) * cur.ev + ((T[0] + T[1]) + (T[2] + T[3]));
+        // rows past S fall out of the buffer range and are dropped
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float yv = y[j];   // (a bit_cast of a vector element is lowered as element 0)
+            const int off = (((ch * kChunk + 16 * MT + 4 * lq + j) * Hv + h) * kDV + c0 + lr) * 4;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ry, off, 0, 0);
+        }
+    };
+    {
+        const ScanSrc s = scan_src(a, 0, h);
+#pragma unroll
+        for (int x = 0; x < 4; x++) opA.q[x] = scan_ld(s.rk, qo + x * 1024);
+#pragma unroll
+        for (int x = 0; x < 4; x++) load2(opA, s, x);
+    }
+    __syncthreads();
+    lds_barrier();
+    first(opA, opB, 0, 0);
+    lds_barrier();
+    // (beside the state waves' chunk ch: finish ch - 1 | barrier | first half of ch | barrier)
+    int ch = 1;
+    for (; ch + 1 < n_chunks; ch += 2) {
+        finish(opA, opB, ch - 1, 0);
+        lds_barrier();
+        first(opB, opA, ch, 1);
+        lds_barrier();
+        finish(opB, opA, ch, 1);
+        lds_barrier();
+        first(opA, opB, ch + 1, 0);
+        lds_barrier();
+    }
+    if (ch < n_chunks) {
+        finish(opA, opB, ch - 1, 0);
+        lds_barrier();
+        first(opB, opA, ch, 1);
+        lds_barrier();
+        finish(opB, opA, ch, 1);
+    } else {
+        finish(opA, opB, ch - 1, 0);
+    }
+}
+
 __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dn_chunk_scan_kernel(
     const ScanArgs a) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -807,7 +925,7 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     Slab Sc = reinterpret_cast<Slab>(smem);                            // [2 x 16] columns: slab of even / odd chunks
     Ucols Ul = reinterpret_cast<Ucols>(smem + 2 * kSeqCB * kScP);      // [2 x 16] U of even / odd chunks
     Ucols Ud = Ul + 2 * kSeqCB;                                        // decayed U of this chunk
-    const int S = a.S, Hv = a.Hv, n_chunks = a.n_chunks;
+    const int S = a.S, n_chunks = a.n_chunks;
     // XCD-aware: the 8 slabs of a head share its chunk records, so they go to
     // one XCD (workgroup id mod 8 selects the XCD; Hv * 8 workgroups)
     const int nwg = gridDim.x, id = blockIdx.x;
@@ -925,97 +1043,11 @@ __global__ __launch_bounds__(kMsNT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
             for (int j = 0; j < 4; j++) Sp[(size_t)(32 * mt + 16 * t + 4 * lq + j) * kDV + c0 + lr] = Sr[t][j];
     } else {
-        // ------------------------------------------------ output waves
-        const __amdgpu_buffer_rsrc_t ry =
-            __builtin_amdgcn_make_buffer_rsrc(a.y, 0, (int)((size_t)S * Hv * kDV * 4), 0x00020000);
-        const int qo = (mt * 8 * 64 + lane) * 16, po = (kVP + (mt * (mt + 1) / 2 * 64 + lane) * 4) * 4;
-        const int eo = (kVE + 16 * mt + 4 * lq) * 4;
-        OutOps opA, opB;
-        v4f Z[4];
-        // second half of the operands of chunk ch (the first half is loaded a step earlier)
-        auto load2 = [&](OutOps& o, const ScanSrc& s, int x) __attribute__((always_inline)) {
-            o.q[4 + x] = scan_ld(s.rk, qo + (4 + x) * 1024);
-            o.p[x] = x <= mt ? scan_ld(s.rv, po + x * 1024) : zero;
-            if (x == 0) o.ev = scan_ld(s.rv, eo);
-        };
-        // Q S0 of chunk ch, state rows 0..63, the first operands of chunk ch + 1 requested
-        auto first = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
-            const ScanSrc src = scan_src(a, ch + 1, h);
-            Slab sc = Sc + par * kSeqCB;
-#pragma unroll
-            for (int e = 0; e < 4; e++) Z[e] = zero;
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                nxt.q[x] = scan_ld(src.rk, qo + x * 1024);
-                const v4f sb = *reinterpret_cast<const v4f*>(&sc[lr][16 * x + 4 * lq]);
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[x][e], sb[e], Z[e], 0, 0, 0);
-            }
-        };
-        // the rest of chunk ch's outputs, the other operands of chunk ch + 1 requested
-        auto finish = [&](const OutOps& cur, OutOps& nxt, int ch, int par) __attribute__((always_inline)) {
-            const ScanSrc src = scan_src(a, ch + 1, h);
-            Slab sc = Sc + par * kSeqCB;
-            Ucols ul = Ul + par * kSeqCB;
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                load2(nxt, src, x);
-                const v4f sb = *reinterpret_cast<const v4f*>(&sc[lr][64 + 16 * x + 4 * lq]);
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    Z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[4 + x][e], sb[e], Z[e], 0, 0, 0);
-            }
-            v4f y0 = ((Z[0] + Z[1]) + (Z[2] + Z[3])) * cur.ev, y1 = zero;
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                if (x > mt) break;
-                const v4f uv = *reinterpret_cast<const v4f*>(&ul[lr][16 * x + 4 * lq]);
-                y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][0], uv[0], y0, 0, 0, 0);
-                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][1], uv[1], y1, 0, 0, 0);
-                y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][2], uv[2], y0, 0, 0, 0);
-                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x][3], uv[3], y1, 0, 0, 0);
-            }
-            const v4f y = y0 + y1;
-            // rows past S fall out of the buffer range and are dropped
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float yv = y[j];
-                const int off = (((ch * kChunk + 16 * mt + 4 * lq + j) * Hv + h) * kDV + c0 + lr) * 4;
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, yv), ry, off, 0, 0);
-            }
-        };
-        {
-            const ScanSrc s = scan_src(a, 0, h);
-#pragma unroll
-            for (int x = 0; x < 4; x++) opA.q[x] = scan_ld(s.rk, qo + x * 1024);
-#pragma unroll
-            for (int x = 0; x < 4; x++) load2(opA, s, x);
-        }
-        __syncthreads();
-        lds_barrier();
-        first(opA, opB, 0, 0);
-        lds_barrier();
-        // (the state waves' chunk ch: finish ch - 1 | barrier | first half of ch | barrier)
-        int ch = 1;
-        for (; ch + 1 < n_chunks; ch += 2) {
-            finish(opA, opB, ch - 1, 0);
-            lds_barrier();
-            first(opB, opA, ch, 1);
-            lds_barrier();
-            finish(opB, opA, ch, 1);
-            lds_barrier();
-            first(opA, opB, ch + 1, 0);
-            lds_barrier();
-        }
-        if (ch < n_chunks) {
-            finish(opA, opB, ch - 1, 0);
-            lds_barrier();
-            first(opB, opA, ch, 1);
-            lds_barrier();
-            finish(opB, opA, ch, 1);
-        } else {
-            finish(opA, opB, ch - 1, 0);
+        switch (mt) {
+            case 0: scan_outputs<0>(a, Sc, Ul, h, c0, lane); break;
+            case 1: scan_outputs<1>(a, Sc, Ul, h, c0, lane); break;
+            case 2: scan_outputs<2>(a, Sc, Ul, h, c0, lane); break;
+            default: scan_outputs<3>(a, Sc, Ul, h, c0, lane); break;
         }
     }
 }
