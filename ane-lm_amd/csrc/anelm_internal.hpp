@@ -249,14 +249,59 @@ __device__ __forceinline__ float partner(float v) {
     return __int_as_float(r);
 }
 
+// Exchange of two values across the wave without LDS (v_permlane32_swap,
+// v_permlane16_swap): M = 32: r[0] holds x's lower half in lanes < 32 and y's
+// lower half in the others, r[1] the upper halves; M = 16 the same for the two
+// 16-lane rows of each half.  r[0] + r[1] is then x's (lane bit M clear) or y's
+// (set) sum over the lanes that differ in bit M.
+struct Swapped {
+    float r[2];
+};
+template <int M>
+__device__ __forceinline__ Swapped lane_swap(float x, float y) {
+    static_assert(M == 32 || M == 16, "half-wave or row exchange");
+    const uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
+    Swapped s;
+    if constexpr (M == 32) {
+        const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        s.r[0] = __uint_as_float(v[0]);
+        s.r[1] = __uint_as_float(v[1]);
+    } else {
+        const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        s.r[0] = __uint_as_float(v[0]);
+        s.r[1] = __uint_as_float(v[1]);
+    }
+    return s;
+}
+
+// v and its stage-M partner's v, summed / the larger (as v + partner<M>(v)).
+template <int M>
+__device__ __forceinline__ float pair_sum(float v) {
+    if constexpr (M >= 16) {
+        const Swapped s = lane_swap<M>(v, v);
+        return s.r[0] + s.r[1];
+    } else {
+        return v + partner<M>(v);
+    }
+}
+template <int M>
+__device__ __forceinline__ float pair_max(float v) {
+    if constexpr (M >= 16) {
+        const Swapped s = lane_swap<M>(v, v);
+        return fmaxf(s.r[0], s.r[1]);
+    } else {
+        return fmaxf(v, partner<M>(v));
+    }
+}
+
 template <int M = 32>
 __device__ __forceinline__ float wave_sum_from(float v) {
-    if constexpr (M >= 1) return wave_sum_from<M / 2>(v + partner<M>(v));
+    if constexpr (M >= 1) return wave_sum_from<M / 2>(pair_sum<M>(v));
     return v;
 }
 template <int M = 32>
 __device__ __forceinline__ float wave_max_from(float v) {
-    if constexpr (M >= 1) return wave_max_from<M / 2>(fmaxf(v, partner<M>(v)));
+    if constexpr (M >= 1) return wave_max_from<M / 2>(pair_max<M>(v));
     return v;
 }
 

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include <algorithm>
+#include <atomic>
 #include <math.h>
 #include <vector>
 
@@ -1065,6 +1066,425 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void a
     }
 }
 
+// ---- ring decode on the matrix cores (fp16 ring, head_dim 256, 4 query heads
+// per kv head)
+//
+// The matrix instructions take fp16, and the ring's rows are fp16 exactly; the
+// fp32 query and the fp32 weights are taken as three fp16 terms each (x = x1 +
+// x2 + x3, each the rounding of what is left, after an exact power-of-two
+// scaling: 33 bits, so nothing is lost against fp32).  Only 4 of the 16
+// columns of a 16x16 tile are query heads, so the terms ride along for free:
+// column (or row) n = head n % 4, term n / 4, n < 12.
+//   S = K Q^T   v_mfma_f32_16x16x32_f16, A = 16 K rows (lane (q, n) = key n,
+//               dims 32 s + 8 q .. +8), B = the query terms; the three term
+//               columns are then added across lanes: every lane (q, n) holds
+//               the scores of head n % 4 for keys 4 q + (0..3).
+//   O = P V     v_mfma_f32_16x16x16f16 per 16-dim tile, A = the weight terms
+//               (lane (q, n): row n, keys 4 q + (0..3)), B = V rows read from
+//               the wave's LDS copy by transposing reads, as in the paged
+//               kernel; rows 4 t + g of the result are term t of head g.
+// A workgroup (8 waves) takes p.kps keys of one kv head, 16-key block b going
+// to wave b % 8, the next block's loads in flight while one is used; each wave
+// has its own online softmax, merged through LDS at the end.  Splits as above.
+// Bound: instruction issue and latency of one pass (the whole kernel is some
+// 1500 instructions per wave, executed once); whole call before (fp32 vector
+// products, 64-key splits) and now: 513 keys 8q/2kv 11.4 -> 9.8 us, 8192 keys
+// 16q/4kv 23.2 -> 13.4 us (33.6 MB; merge kernel 4 of it), errors against 64
+// bits 1.9e-7 and 2.3e-7 as before.
+constexpr int kRNT = 512;
+constexpr int kRW = kRNT / 64;
+constexpr int kRBlk = 16;
+constexpr int kRVB = kRBlk * 256 * 2;          // bytes of one block's V rows
+constexpr int kRQ = 256 + 8;                   // query term row pitch (halfs): rows 4 banks apart
+constexpr float kRPScale = 256.f;              // of the weights, an exact power of two
+
+// Adds the values of lanes n, n + 4, n + 8, n + 12 of each 16-lane row.
+__device__ __forceinline__ float row_quad_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));   // row_ror:8
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false));   // row_ror:4
+    return v;
+}
+
+__global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void attn_ring_mfma_kernel(
+    const uint16_t* k_cache, const uint16_t* v_cache, const float* q_rows, int q_stride, int tok_stride, int head_rows,
+    int start, int len, int cap, int kps, int n_splits, const DecodeParams p) {
+    constexpr int D = 256, G = 4, KS = D / 32, NTD = D / 16, REC = D + 2;
+    extern __shared__ __attribute__((aligned(16))) char vdyn[];   // V blocks: [1 or 2][8 waves][kRVB]
+    __shared__ __attribute__((aligned(16))) _Float16 q16[12][kRQ];
+    __shared__ __attribute__((aligned(16))) uint16_t nkv[2][D];   // the new key and value as stored
+    __shared__ float qscale[G];                                   // undoes the query scaling
+    __shared__ float red_m[kRW][G], red_l[kRW][G];
+    __shared__ float ml_s[kInlineMaxSplits][G][2];
+    __shared__ float wl_s[kInlineMaxSplits][G];
+    __shared__ int last_s;
+    const int split = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, q = lane >> 4, n = lane & 15;
+    const int k0 = split * kps, kend = min(k0 + kps, len);
+    if (k0 >= len) return;
+    const int nblk = (kend - k0 + kRBlk - 1) / kRBlk;
+
+    // ---- K and V of the wave's first block
+    const uint16_t* kc = k_cache + (size_t)kvh * head_rows * D;
+    const uint16_t* vc = v_cache + (size_t)kvh * head_rows * D;
+    auto request = [&](int blk, int buf, half8_t (&ka)[KS]) __attribute__((always_inline)) {
+        // (a key past the last: the last one again, masked below)
+        int row = start + min(k0 + blk * kRBlk + n, kend - 1);
+        row -= row >= cap ? cap : 0;
+        const size_t base = (size_t)row * tok_stride + 8 * q;
+#pragma unroll
+        for (int s = 0; s < KS; s++) ka[s] = *reinterpret_cast<const half8_t*>(kc + base + 32 * s);
+        // V rows straight to LDS: key n, dims 8 (4 i + q) .. +8 at byte (16 (4 i + q) + n) * 16
+        char* vb = vdyn + (buf * kRW + w) * kRVB;
+#pragma unroll
+        for (int i = 0; i < KS; i++)
+            __builtin_amdgcn_global_load_lds(vc + base + 32 * i, (lds_void_ptr)(vb + i * 1024), 16, 0, 0);
+    };
+    half8_t ka[KS];
+    request(w, 0, ka);   // (a wave without a block: the last key's rows, unused)
+    asm volatile("" ::: "memory");
+    const bool inline_merge = p.arrivals != nullptr;
+    const bool owner = p.fused && split == n_splits - 1;   // holds the newest key
+    const float* qh = q_rows + (size_t)kvh * G * q_stride;
+    // ---- prologue: wave w < 4 the query row of head w, wave 4 the new key
+    // (RMSNorm, RoPE: models/llm/qwen3_5.cpp:952-971), wave 5 the new value;
+    // lane l holds dims 4 l .. 4 l + 3.  Every operand is requested before the
+    // first is used, without branches (a load under a branch is waited for
+    // where the branch ends), in 16-byte loads from dword-aligned rows
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+    const bool isq = w < G, newk = owner && w == G, newv = owner && w == G + 1;
+    const float* kn = p.k_new + (size_t)kvh * D;
+    const float* vn = p.v_new + (size_t)kvh * D;
+    // the new row as stored: to its ring slot (8 bytes per lane) and to LDS
+    const size_t slot_off = (size_t)p.new_slot * tok_stride + (size_t)kvh * head_rows * D;
+    uint16_t* const kw = const_cast<uint16_t*>(k_cache) + slot_off + 4 * lane;
+    uint16_t* const vw = const_cast<uint16_t*>(v_cache) + slot_off + 4 * lane;
+    auto append = [&](int which, f4u v) __attribute__((always_inline)) {
+        const half4_t h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        *reinterpret_cast<half4_t*>(which ? vw : kw) = h;
+        *reinterpret_cast<half4_t*>(&nkv[which][4 * lane]) = h;
+    };
+    const float* src = (newk ? kn : newv ? vn : qh + (size_t)(w & (G - 1)) * q_stride) + 4 * lane;
+    const float* nw = newk ? p.k_norm_w : p.q_norm_w;
+    const bool norm = p.fused && nw != nullptr;
+    f4u x = *reinterpret_cast<const f4u*>(src);
+    const f4u wv = *reinterpret_cast<const f4u*>(norm ? nw + 4 * lane : src);   // (without weights: the row again)
+    // this lane's rotation angles, through pointers into the argument segment:
+    // interleaved pairs 2 l, 2 l + 1; half-split pair d mod rp of each dim d
+    const float* csp = p.cs;
+    const float* snp = p.sn;
+    const int rp = p.rot_pairs;
+    float cv[4], sv[4];
+    {
+        const bool il = p.rope_mode == ANELM_ROPE_INTERLEAVED;
+        #pragma unroll
+        for (int i = 0; i < 4; i++) {
+            int j = il ? 2 * lane + i / 2 : 4 * lane + i < rp ? 4 * lane + i : 4 * lane + i - rp;
+            j = min(max(j, 0), kMaxRotPairs - 1);
+            cv[i] = csp[j];
+            sv[i] = snp[j];
+        }
+    }
+    // this thread's two outputs: dims od, od + 1 of head og; their gate logits
+    // (without a gate: not used)
+    const int og = tid >> 7, od = 2 * (tid & 127);
+    const f2u gl = *reinterpret_cast<const f2u*>(qh + (size_t)og * q_stride + (p.gate ? D : 0) + od);
+    if (isq || newk) {
+        if (p.fused) {
+            if (norm) {
+                float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+                ss = wave_sum(ss);
+                const float inv = 1.0f / sqrtf(ss / (float)D + p.eps);
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[i] = (x[i] * inv) * wv[i];
+            }
+            if (p.rope_mode == ANELM_ROPE_INTERLEAVED) {
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const int j = (4 * lane + i) / 2;
+                    if (j < rp) {
+                        float o0, o1;
+                        rotate_pair(o0, o1, x[i], x[i + 1], cv[i], sv[i]);
+                        x[i] = o0;
+                        x[i + 1] = o1;
+                    }
+                }
+            } else {
+                // dim i's mate is i + rp (i < rp) or i - rp (rp <= i < 2 rp)
+                float mate[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int d = 4 * lane + i, md = d < rp ? d + rp : d < 2 * rp ? d - rp : d;
+                    mate[i] = 0.f;
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const float got = __shfl(x[u], md / 4, 64);
+                        if (md % 4 == u) mate[i] = got;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int d = 4 * lane + i;
+                    if (d >= 2 * rp) continue;
+                    const bool lo = d < rp;
+                    float o0, o1;
+                    rotate_pair(o0, o1, lo ? x[i] : mate[i], lo ? mate[i] : x[i], cv[i], sv[i]);
+                    x[i] = lo ? o0 : o1;
+                }
+            }
+        }
+        if (isq) {
+            // the row scaled by a power of two to at most 2^8, then its three terms
+            const float mx = wave_max(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+            const int e = min(max(__builtin_amdgcn_frexp_expf(mx), -100), 120);
+            const float up = ldexpf(1.0f, 8 - e);
+            half4_t t1, t2, t3;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float v = x[i] * up;
+                t1[i] = (_Float16)v;
+                const float r1 = v - (float)t1[i];
+                t2[i] = (_Float16)r1;
+                t3[i] = (_Float16)(r1 - (float)t2[i]);
+            }
+            *reinterpret_cast<half4_t*>(&q16[w][4 * lane]) = t1;
+            *reinterpret_cast<half4_t*>(&q16[4 + w][4 * lane]) = t2;
+            *reinterpret_cast<half4_t*>(&q16[8 + w][4 * lane]) = t3;
+            if (lane == 0) qscale[w] = ldexpf(1.0f, e - 8);
+        } else {
+            append(0, x);
+        }
+    } else if (newv) {
+        append(1, x);
+    }
+    lds_barrier();
+    half8_t qb[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        qb[s] = *reinterpret_cast<const half8_t*>(&q16[min(n, 11)][32 * s + 8 * q]);
+        if (n >= 12) qb[s] = half8_t{};
+    }
+    const float scale = p.scale * qscale[n & 3];
+
+    f32x4_t o[NTD];
+#pragma unroll
+    for (int t = 0; t < NTD; t++) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;   // head n % 4 of this wave
+    const int tr_off = (16 * ((n & 3) >> 1) + 4 * q + (n >> 2)) * 16 + (n & 1) * 8;
+    int buf = 0;
+    for (int blk = w; blk < nblk; blk += kRW, buf ^= 1) {
+        half8_t kn[KS];
+        const bool more = blk + kRW < nblk;   // (then there are two V buffers)
+        if (more) request(blk + kRW, buf ^ 1, kn);
+        char* const vb = vdyn + (buf * kRW + w) * kRVB;
+        const int left = kend - k0 - blk * kRBlk;   // valid keys from here on
+        const bool patch = owner && left <= kRBlk;
+        if (patch) {
+            // the row loads ran before the append: the newest key (and the
+            // rows past it, which repeat its slot) come from the prologue
+            if (n >= left - 1) {
+#pragma unroll
+                for (int s = 0; s < KS; s++) ka[s] = *reinterpret_cast<const half8_t*>(&nkv[0][32 * s + 8 * q]);
+            }
+        }
+        f32x4_t sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; s += 2) {
+            sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[s], qb[s], sa, 0, 0, 0);
+            sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[s + 1], qb[s + 1], sb, 0, 0, 0);
+        }
+        float sc[4], bm = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float full = row_quad_sum(sa[i] + sb[i]);   // (n >= 12: zero columns)
+            sc[i] = 4 * q + i < left ? full * scale : -INFINITY;
+            bm = fmaxf(bm, sc[i]);
+        }
+        bm = pair_max<16>(pair_max<32>(bm));
+        const float m_new = fmaxf(m_run, bm);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;   // no valid key yet: weights 0
+        const float alpha = __expf(m_run - m_use);              // 0 while m_run is -inf
+        half4_t pa;
+        float psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float e = __expf(sc[i] - m_use);   // masked keys: 0
+            psum += e;
+            // this lane's term of the weight
+            const float v = e * kRPScale;
+            const _Float16 t1 = (_Float16)v;
+            const float r1 = v - (float)t1;
+            const _Float16 t2 = (_Float16)r1, t3 = (_Float16)(r1 - (float)t2);
+            pa[i] = n < 4 ? t1 : n < 8 ? t2 : n < 12 ? t3 : (_Float16)0.f;
+        }
+        l_run = l_run * alpha + psum;
+        m_run = m_new;
+        // O row 4 t + g is head g: its factor is that column's alpha
+        if (blk != w && __any(alpha != 1.f)) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float ai = __shfl(alpha, i, 64);
+#pragma unroll
+                for (int t = 0; t < NTD; t++) o[t][i] *= ai;
+            }
+        }
+        // V of this block has landed once only the next block's loads (8 K, 8 V) remain
+        if (more) __builtin_amdgcn_s_waitcnt(0x4F70);   // vmcnt(16)
+        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        asm volatile("" ::: "memory");
+        if (patch) {
+            for (int r = left - 1; r < kRBlk; r++)
+                if (lane < 32)
+                    *reinterpret_cast<uint4*>(vb + (16 * lane + r) * 16) =
+                        *reinterpret_cast<const uint4*>(&nkv[1][8 * lane]);
+        }
+        // (one statement with its wait: as separate builtins the reads would
+        // wait for every load in flight, the next block's too)
+        s16x4_t vt[NTD];
+        {
+            const uint32_t va =
+                (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const char*)(vb + tr_off));
+            asm volatile(
+                "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:512\n\t"
+                "ds_read_b64_tr_b16 %2, %16 offset:1024\n\tds_read_b64_tr_b16 %3, %16 offset:1536\n\t"
+                "ds_read_b64_tr_b16 %4, %16 offset:2048\n\tds_read_b64_tr_b16 %5, %16 offset:2560\n\t"
+                "ds_read_b64_tr_b16 %6, %16 offset:3072\n\tds_read_b64_tr_b16 %7, %16 offset:3584\n\t"
+                "ds_read_b64_tr_b16 %8, %16 offset:4096\n\tds_read_b64_tr_b16 %9, %16 offset:4608\n\t"
+                "ds_read_b64_tr_b16 %10, %16 offset:5120\n\tds_read_b64_tr_b16 %11, %16 offset:5632\n\t"
+                "ds_read_b64_tr_b16 %12, %16 offset:6144\n\tds_read_b64_tr_b16 %13, %16 offset:6656\n\t"
+                "ds_read_b64_tr_b16 %14, %16 offset:7168\n\tds_read_b64_tr_b16 %15, %16 offset:7680\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(vt[0]), "=&v"(vt[1]), "=&v"(vt[2]), "=&v"(vt[3]), "=&v"(vt[4]), "=&v"(vt[5]), "=&v"(vt[6]),
+                  "=&v"(vt[7]), "=&v"(vt[8]), "=&v"(vt[9]), "=&v"(vt[10]), "=&v"(vt[11]), "=&v"(vt[12]), "=&v"(vt[13]),
+                  "=&v"(vt[14]), "=&v"(vt[15])
+                : "v"(va)
+                : "memory");
+        }
+#pragma unroll
+        for (int t = 0; t < NTD; t++)
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, __builtin_bit_cast(half4_t, vt[t]), o[t], 0, 0, 0);
+        if (more) {
+#pragma unroll
+            for (int s = 0; s < KS; s++) ka[s] = kn[s];
+        }
+    }
+
+    // ---- merge the waves.  The three term rows of a head (lanes q = 0, 1, 2;
+    // row 3 is zero) are added by two half exchanges: lane (q, n) ends with
+    // tiles 4 a + q, a < 4
+    l_run = pair_sum<16>(pair_sum<32>(l_run));
+    if (lane < G) {
+        red_m[w][lane] = m_run;
+        red_l[w][lane] = l_run;
+    }
+    float* ro = reinterpret_cast<float*>(vdyn + w * kRVB);   // this wave's O rows [G][D], over its own V block
+    f32x4_t h1[NTD / 2];
+#pragma unroll
+    for (int a = 0; a < NTD / 4; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)   // tiles 4 a + b (lanes < 32) and 4 a + b + 2
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const Swapped s = lane_swap<32>(o[4 * a + b][i], o[4 * a + b + 2][i]);
+                h1[2 * a + b][i] = s.r[0] + s.r[1];
+            }
+#pragma unroll
+    for (int a = 0; a < NTD / 4; a++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {   // tiles (lane bit 4 clear) 2 a' and (set) 2 a' + 1
+            const Swapped s = lane_swap<16>(h1[2 * a][i], h1[2 * a + 1][i]);
+            ro[i * D + 16 * (4 * a + q) + n] = s.r[0] + s.r[1];
+        }
+    lds_barrier();
+    float* const out = p.out + (size_t)kvh * G * D;
+    float* const part = p.part + (size_t)kvh * p.max_splits * G * REC;
+    typedef uint32_t f2u32 __attribute__((ext_vector_type(2)));
+    auto store_out = [&](float o0, float o1, float L) __attribute__((always_inline)) {
+        o0 = o0 / L;
+        o1 = o1 / L;
+        if (p.gate) {
+            o0 = o0 / (1.0f + expf(-gl[0]));
+            o1 = o1 / (1.0f + expf(-gl[1]));
+        }
+        *reinterpret_cast<f2u*>(out + 2 * tid) = f2u{o0, o1};
+    };
+    const __amdgpu_buffer_rsrc_t rr =
+        __builtin_amdgcn_make_buffer_rsrc(part, 0, n_splits > 1 ? n_splits * G * REC * 4 : 0, 0x00020000);
+    {
+        float M = red_m[0][og];
+#pragma unroll
+        for (int ww = 1; ww < kRW; ww++) M = fmaxf(M, red_m[ww][og]);
+        float L = 0.f, O0 = 0.f, O1 = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < kRW; ww++) {
+            // (a wave without keys: m = -inf, weight 0, O = 0)
+            const float wt = __expf(red_m[ww][og] - M);
+            const float2 ov = reinterpret_cast<const float2*>(vdyn + ww * kRVB)[tid];
+            L = fmaf(red_l[ww][og], wt, L);
+            O0 = fmaf(ov.x, wt, O0);
+            O1 = fmaf(ov.y, wt, O1);
+        }
+        O0 *= 1.0f / kRPScale;
+        O1 *= 1.0f / kRPScale;
+        if (n_splits == 1) {
+            store_out(O0, O1, L);
+        } else if (inline_merge) {
+            const int ri = (split * G + og) * REC;
+            __builtin_amdgcn_raw_buffer_store_b64(f2u32{__float_as_uint(O0), __float_as_uint(O1)}, rr, (ri + 2 + od) * 4, 0,
+                                                  kCoherent);
+            if (od == 0)
+                __builtin_amdgcn_raw_buffer_store_b64(f2u32{__float_as_uint(M), __float_as_uint(L)}, rr, ri * 4, 0,
+                                                      kCoherent);
+        } else {
+            float* rec = part + ((size_t)split * G + og) * REC;
+            *reinterpret_cast<float2*>(rec + 2 + od) = make_float2(O0, O1);
+            if (od == 0) *reinterpret_cast<float2*>(rec) = make_float2(M, L);
+        }
+    }
+    if (!inline_merge) return;
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // this thread's record stores completed
+    __syncthreads();
+    uint32_t* const ctr = p.arrivals + kvh;
+    if (tid == 0) last_s = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                           (uint32_t)(n_splits - 1);
+    __syncthreads();
+    if (!last_s) return;
+    if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // ---- merge of the splits; every record load is issued before the first
+    // is used (one memory round trip)
+    f2u32 ov[kInlineMaxSplits], ml = {0u, 0u};
+    if (tid < n_splits * G)   // record tid / G, head tid % G
+        ml = __builtin_amdgcn_raw_buffer_load_b64(rr, tid * REC * 4, 0, kCoherent);
+#pragma unroll
+    for (int sp = 0; sp < kInlineMaxSplits; sp++)   // past the last split: 0 (buffer range)
+        ov[sp] = __builtin_amdgcn_raw_buffer_load_b64(rr, ((sp * G + og) * REC + 2 + od) * 4, 0, kCoherent);
+    if (tid < 64) {
+        // lane 4 s + g: weight of split s for head g, zero past the last split;
+        // maximum and sum over the lanes of one head
+        const uint32_t mb = ml[0], lb = ml[1];
+        const float mv = tid < n_splits * G ? __uint_as_float(mb) : -INFINITY, lv = __uint_as_float(lb);
+        float M = mv;
+        M = pair_max<16>(pair_max<32>(M));
+        M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x128, 0xF, 0xF, false)));
+        M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x124, 0xF, 0xF, false)));
+        const float wt = tid < n_splits * G ? __expf(mv - M) : 0.f;
+        float L = lv * wt;
+        L = row_quad_sum(pair_sum<16>(pair_sum<32>(L)));
+        wl_s[tid >> 2][tid & 3] = wt;
+        if (tid < G) ml_s[0][tid][1] = L;
+    }
+    lds_barrier();
+    float O0 = 0.f, O1 = 0.f;
+#pragma unroll
+    for (int sp = 0; sp < kInlineMaxSplits; sp++) {
+        const uint32_t b0 = ov[sp][0], b1 = ov[sp][1];
+        O0 = fmaf(wl_s[sp][og], __uint_as_float(b0), O0);
+        O1 = fmaf(wl_s[sp][og], __uint_as_float(b1), O1);
+    }
+    store_out(O0, O1, ml_s[0][og][1]);
+}
+
 // Log-sum-exp merge of the split partials of one (sequence, q head) for 64
 // output dims per workgroup: M = max m_s, L = sum l_s e^(m_s-M),
 // O = sum o_s e^(m_s-M), out = O / L, then the sigmoid gate.  Splits are
@@ -1143,6 +1563,10 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const DecodeParams p)
     }
 }
 
+// Rings the matrix-core kernel takes.
+template <typename KV>
+constexpr bool ring_mfma(int D, int G) { return std::is_same<KV, uint16_t>::value && D == 256 && G == 4; }
+
 template <typename KV, int D, int G>
 int launch_g(DecodeParams& p, dim3 grid, hipStream_t st) {
     if (p.paged) {
@@ -1169,6 +1593,20 @@ int launch_g(DecodeParams& p, dim3 grid, hipStream_t st) {
             hipLaunchKernelGGL((attn_paged_mfma_kernel<D, G>), pgrid, dim3(kNT), 0, st, p);
             ANELM_LAUNCHED("attn_paged_mfma_kernel");
         }
+    } else if constexpr (ring_mfma<KV>(D, G)) {
+        static std::atomic<bool> attr{false};
+        if (!attr.load(std::memory_order_acquire)) {
+            ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_mfma_kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kRW * kRVB));
+            attr.store(true, std::memory_order_release);
+        }
+        // a second set of V buffers where a wave walks several blocks
+        const int bufs = std::min(p.kps, p.len) > kRW * kRBlk ? 2 : 1;
+        hipLaunchKernelGGL(attn_ring_mfma_kernel, grid, dim3(kRNT), bufs * kRW * kRVB, st,
+                           static_cast<const uint16_t*>(p.k_cache), static_cast<const uint16_t*>(p.v_cache), p.q,
+                           p.q_stride, (int)p.tok_stride, (int)(p.head_stride / D), p.start, p.len, p.cap, p.kps,
+                           (p.len + p.kps - 1) / p.kps, p);
+        ANELM_LAUNCHED("attn_ring_mfma_kernel");
     } else {
         hipLaunchKernelGGL((attn_decode_kernel<KV, D, G>), grid, dim3(ring_threads<G>()), 0, st, p);
         ANELM_LAUNCHED("attn_decode_kernel");
@@ -1214,6 +1652,17 @@ size_t part_bytes(int n_heads, int n_kv_heads, int D, int n_seqs, int max_len, b
     return (size_t)n_seqs * n_kv_heads * max_splits * G * (D + 2) * sizeof(float);
 }
 
+// Keys per split of the matrix-core ring kernel, a multiple of its 128 keys
+// per round of blocks: one round while that gives at most a workgroup per CU
+// (a further round costs its memory latency, 3 us: 513 keys of 2 kv heads 9.7
+// us in 5 splits of one round, 12.8 in 3 of two; 8192 keys of 4 kv heads 13.4
+// and 16.0), then as many rounds as keep one workgroup per CU (32768 keys of 4
+// kv heads: 27.7 us in 64 splits of four rounds, 31.7 in 128, 30.6 in 43).
+int ring_split_keys(int len, int Hkv, int cus) {
+    const long round = kRW * kRBlk;
+    return (int)(round * std::max(1L, ((long)len * Hkv + round * cus - 1) / (round * cus)));
+}
+
 // Sets the split layout and partials buffer for one decode call, then
 // launches.  A split is 256/G keys (ring mode: every lane of the workgroup
 // then loads all of its K and V rows at once) or kPagedSplit keys (paged
@@ -1224,7 +1673,12 @@ int run_decode(DecodeParams& p, int kv_dtype, int n_heads, int D, int n_seqs, in
                hipStream_t st, float* part = nullptr, size_t part_cap = 0) {
     const int Hkv = p.n_kv_heads;
     const int G = n_heads / Hkv;
-    const int kps = p.paged ? kPagedSplit : 256 / G;
+    int kps = p.paged ? kPagedSplit : 256 / G;
+    if (!p.paged && kv_dtype == ANELM_F16 && ring_mfma<uint16_t>(D, G)) {
+        Device* dev = device();
+        if (dev == nullptr) return ANELM_EHIP;
+        kps = ring_split_keys(max_len, Hkv, dev->num_cus);
+    }
     const int max_splits = (max_len + kps - 1) / kps;
     p.kps = kps;
     p.max_splits = max_splits;
@@ -1233,7 +1687,8 @@ int run_decode(DecodeParams& p, int kv_dtype, int n_heads, int D, int n_seqs, in
         p.tok_stride = (long)Hkv * D;
         p.head_stride = D;
     }
-    const size_t need = part_bytes(n_heads, Hkv, D, n_seqs, max_len, p.paged != 0);
+    const size_t need =
+        max_splits > 1 ? (size_t)n_seqs * Hkv * max_splits * G * (D + 2) * sizeof(float) : 0;
     // ring mode with few splits: merged in the split kernel (arrival counters)
     const bool merge_inline = !p.paged && max_splits >= 2 && max_splits <= kInlineMaxSplits &&
                               Hkv * n_seqs <= kArrivalWords;

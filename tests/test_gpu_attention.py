@@ -107,6 +107,67 @@ def test_full_attn_decode_split_merge(anelm, orc, dev, n_heads, n_kv_heads, head
     _check_decode(_run_decode(anelm, c, dev), _oracle_decode(orc, c))
 
 
+@pytest.mark.parametrize("Hq,Hkv,cached,start,rope_mode,rot,gate,scale", [
+    (8, 2, 0, 0, 0, 64, True, 1.0),          # the new key alone: one wave has a key, seven none
+    (16, 4, 15, 3, 1, 64, True, 1.0),        # a whole 16-key block, half-split pairs
+    (4, 1, 16, 0, 0, 0, False, 1.0),         # the new key alone in its block; no rotation, no gate
+    (16, 4, 127, 100, 1, 96, True, 1.0),     # one full split; pairs that are no multiple of a lane's dims apart
+    (8, 2, 128, 7, 0, 64, True, 1.0),        # the new key alone in its split
+    (8, 2, 2047, 60, 0, 64, True, 1e-4),     # 16 splits, merged in the kernel; tiny rows
+    (8, 2, 2048, 60, 0, 64, True, 3e4),      # 17 splits: the merge kernel; rows past fp16's range
+    (16, 4, 16500, 900, 0, 64, True, 1.0),   # three rounds of blocks per wave, a part-filled last one
+])
+def test_full_attn_decode_matrix_core_ring(anelm, dev, Hq, Hkv, cached, start, rope_mode, rot, gate, scale):
+    """fp16 rings of head_dim 256 with 4 query heads per kv head, at the edges
+    of the kernel's blocks, splits and merges, every unused ring slot NaN.
+    Against float64 over the same fp16 keys: the fp32 query and weights enter
+    the products whole (three fp16 terms each), so the error is that of fp32
+    sums of 256 products and of the weights' exponential, 2^-24 * 16 * |score|
+    at the scores met here: relative 1e-5.  Without norm weights, so `scale`
+    is the rows' scale; large rows make one weight 1 and the output a value."""
+    D, cap = 256, cached + 9
+    c = attn_decode_case(340 + cached % 89, n_heads=Hq, n_kv_heads=Hkv, cached=cached, capacity=cap, start=start % cap,
+                         rot_dim=rot)
+    used = (c.start + np.arange(cached)) % cap
+    free = np.setdiff1d(np.arange(cap), used)
+    c.k_cache[free] = c.v_cache[free] = 0x7e00
+    c.q_gate[:, :D] *= scale
+    kc, vc = to_dev(c.k_cache, dev), to_dev(c.v_cache, dev)
+    ring = anelm.ops.KVRing(cap, c.start, cached)
+    # the rotation's fp32 cos and sin are given, so both sides use the same
+    ang = float(c.pos) * c.theta ** (-np.arange(0, rot, 2) / max(rot, 1))
+    cs, sn = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    out = anelm.ops.full_attn_decode(to_dev(c.q_gate, dev), to_dev(c.k, dev), to_dev(c.v, dev), kc, vc, None, None, ring,
+                                     Hq, Hkv, D, rot, c.pos, c.theta, c.eps, rope_mode, gate, cs if rot else None,
+                                     sn if rot else None)
+
+    def rotate(x):
+        x = x.astype(np.float64).copy()
+        a, b = (x[:, 0:rot:2], x[:, 1:rot:2]) if rope_mode == 0 else (x[:, :rot // 2], x[:, rot // 2:rot])
+        a, b = a * cs - b * sn, a * sn + b * cs   # (float64 products of the fp32 rows)
+        if rope_mode == 0:
+            x[:, 0:rot:2], x[:, 1:rot:2] = a, b
+        else:
+            x[:, :rot // 2], x[:, rot // 2:rot] = a, b
+        return x
+
+    slots = np.append(used, (c.start + cached) % cap)
+    gk, gv = widen(to_host(kc))[slots].astype(np.float64), widen(to_host(vc))[slots].astype(np.float64)
+    assert_close(gk[-1].astype(np.float32), rotate(c.k).astype(np.float32), rel=1e-3, max_abs=4e-3, what="new key")
+    assert np.array_equal(to_host(vc)[slots[-1]], f16(c.v))
+    q = rotate(c.q_gate[:, :D])
+    got = to_host(out)
+    for h in range(Hq):
+        s = gk[:, h * Hkv // Hq] @ q[h] / 16.0
+        p = np.exp(s - s.max())
+        want = (p / p.sum()) @ gv[:, h * Hkv // Hq]
+        if gate:
+            want = want / (1.0 + np.exp(-c.q_gate[h, D:].astype(np.float64)))
+        err = np.linalg.norm(got[h] - want) / np.linalg.norm(want)
+        tol = max(1e-5, 2.0 ** -24 * 16 * np.abs(s).max())
+        assert err <= tol, (h, err, tol)
+
+
 def test_full_attn_decode_table_row(anelm, orc, dev):
     """cos/sin passed as the reference's table row give the same step."""
     c = attn_decode_case(305)
