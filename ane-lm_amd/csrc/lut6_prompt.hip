@@ -287,15 +287,23 @@ void prompt_gemm_kernel(const PromptArgs a) {
 // tile's stage; `full`: a stage of 256 tiles running at once, where the chip's
 // throughput bounds it; a partly filled round lies between.  Column slices
 // (partial sums added by split_sum in a fixed order) fill the chip when there
-// are few tiles; they cost their traffic.  Measured against the model: 4096 x
-// 2560 x 9216 256x256 207 us (model 182), 1024 x 18432 x 2560 256x128 121
-// (117), 512 x 2560 x 9216 256x128 in 4 slices 42 (42), 64 x 18432 x 2560
-// 64x128 17 (17).
+// are few tiles; they cost their traffic, which mostly stays in the last-level
+// cache.  The constants are a fit to 77 shapes (65..6000 inputs of seven
+// projections) x 20 pairs: what the model picks is within 1 % of the best
+// pair on average and 7 % at most.  256 x 192 is there for the counts that
+// leave 256 x 256 a nearly empty last round or too few tiles (whole call, us,
+// without it and with it: 4096 x 2560 x 9216 269 -> 239, 1024 x 18432 x 2560
+// 151 -> 134, 2048 x 2560 x 9216 150 -> 141, 300 x 18432 x 2560 85 -> 77).
 struct Tile {
     int bm, bn;
     float one, full;
 };
-constexpr Tile kTiles[] = {{256, 256, 0.55f, 1.01f}, {256, 128, 0.36f, 0.55f}, {128, 128, 0.28f, 0.38f}, {64, 128, 0.21f, 0.256f}};
+constexpr Tile kTiles[] = {{256, 256, 0.642f, 0.837f},
+                           {256, 192, 0.513f, 0.678f},
+                           {256, 128, 0.409f, 0.519f},
+                           {128, 128, 0.295f, 0.358f},
+                           {64, 128, 0.207f, 0.244f}};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kSplits[] = {1, 2, 4, 8};
 
 struct Plan {
@@ -307,7 +315,7 @@ struct Plan {
 Plan make_plan(int m, int n, int nk, bool may_split, int cus) {
     Plan p{m, n, nk, -1, 1, 0, 0, 0, 0, 0};
     float best = 0.f;
-    for (int t = 0; t < 4; t++)
+    for (int t = 0; t < kNumTiles; t++)
         for (int s : kSplits) {
             if (s > 1 && (!may_split || nk / s < 8)) continue;
             const Tile& k = kTiles[t];
@@ -315,7 +323,7 @@ Plan make_plan(int m, int n, int nk, bool may_split, int cus) {
             const long rounds = units / cus, rem = units % cus;
             const float stage = (float)rounds * k.full + (rem ? std::max(k.one, k.full * (float)rem / (float)cus) : 0.f);
             float us = stage * (float)nk / (float)s;
-            if (s > 1) us += 4.f + (float)(2 * s + 1) * (float)m * (float)n * 4.f / 4.0e6f;
+            if (s > 1) us += 1.6f + (float)(2 * s + 1) * (float)m * (float)n * 4.f / 5.9e6f;
             if (p.tile < 0 || us < best) best = us, p.tile = t, p.splits = s;
         }
     const Tile& k = kTiles[p.tile];
@@ -415,8 +423,9 @@ int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const floa
             int rc;
             switch (p.tile) {
                 case 0: rc = gemm_launch<256, 256, 2, 4>(a, st); break;
-                case 1: rc = gemm_launch<256, 128, 4, 2>(a, st); break;
-                case 2: rc = gemm_launch<128, 128, 2, 2>(a, st); break;
+                case 1: rc = gemm_launch<256, 192, 4, 2>(a, st); break;
+                case 2: rc = gemm_launch<256, 128, 4, 2>(a, st); break;
+                case 3: rc = gemm_launch<128, 128, 2, 2>(a, st); break;
                 default: rc = gemm_launch<64, 128, 1, 4>(a, st); break;
             }
             if (rc == ANELM_OK && sum) rc = lut6_split_sum(yb, parts, (long)p.m * p.n, p.splits, accumulate, st);

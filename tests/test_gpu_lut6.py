@@ -286,7 +286,10 @@ def test_layer_projections(anelm, orc, dev, out_dim, in_dim, norm, acc):
     (65, 2560, 9216, 0),    # few tiles: column slices and their sum
     (257, 1024, 3584, 0),   # one input past 256
     (300, 12352, 2560, 0),  # more tiles than compute units, ragged in both
-    (1030, 18432, 1024, 0),  # the largest tile
+    (1030, 18432, 1024, 0),  # one input past four 256-input tiles
+    (1500, 18432, 1040, 0),  # the largest tile
+    (500, 18400, 1040, 0),  # 192-row weight tiles, ragged in both
+    (1000, 2080, 4112, 0),  # the same in column slices
 ])
 def test_prompt_gemm(anelm, dev, batch, out_dim, in_dim, shift):
     """Batches past two passes of 32: weights decoded to fp16 once and one fp16
