@@ -483,6 +483,22 @@ __device__ __forceinline__ void gemv_decode(const Buf<3 * NI>& b, Buf<8 * NA>& d
     }
 }
 
+// Wave sum and max of this kernel: the stage partners' values by DPP and
+// swizzle.  The lane-swap form of wave_sum needs a second register per stage;
+// here, where every register is taken by weights in flight, that spilled (128
+// bytes a lane instead of 24) and cost the 4B step at context 8192 0.8 % (868
+// us, 862 with this form).
+template <int M = 32>
+__device__ __forceinline__ float step_wave_sum(float v) {
+    if constexpr (M >= 1) return step_wave_sum<M / 2>(v + partner<M>(v));
+    return v;
+}
+template <int M = 32>
+__device__ __forceinline__ float step_wave_max(float v) {
+    if constexpr (M >= 1) return step_wave_max<M / 2>(fmaxf(v, partner<M>(v)));
+    return v;
+}
+
 // Sums 8 values over each 32-lane half: afterwards lane li (li < 8) of each
 // half holds the half's total of value li in v[0].
 // After the transpose, lanes li and li ^ 8 hold the same value index, so the
@@ -674,7 +690,7 @@ __device__ void attn_stage_fin(const PArgs& a, const PLayer& L, int lane, char* 
             w[i] = isk ? r.kw[i] : r.qw[i];
             ss += v[i] * v[i];
         }
-        ss = wave_sum(ss);
+        ss = step_wave_sum(ss);
         const float inv = 1.0f / sqrtf(ss / (float)kAttnD + a.eps);
         float* dst = isk ? reinterpret_cast<float*>(lds + kAscOff) : qs + row * kAttnD;  // k temp in sc
 #pragma unroll
@@ -788,14 +804,14 @@ __device__ void attn_compute(Buf<4 * NKJ>& b, const PArgs& a, const PLayer& L, i
         const int g = wave;
         float m = -INFINITY;
         for (int t = lane; t < nk; t += 64) m = fmaxf(m, sc[g * 160 + t]);
-        m = wave_max(m);
+        m = step_wave_max(m);
         float l = 0.f;
         for (int t = lane; t < nk; t += 64) {
             const float e = __expf(sc[g * 160 + t] - m);
             sc[g * 160 + t] = e;
             l += e;
         }
-        l = wave_sum(l);
+        l = step_wave_sum(l);
         if (lane == 0) {
             ml[g] = m;
             ml[kAttnG + g] = l;
@@ -935,8 +951,8 @@ __device__ void dn_stage_fin(const PArgs& a, const PLayer& L, int lane, char* ld
     float* s = reinterpret_cast<float*>(lds + kDqOff);
     float q0 = r.q0, q1 = r.q1, k0 = r.k0, k1 = r.k1;
     if (L.dn_flags & ANELM_DN_L2NORM) {
-        const float sq = wave_sum(q0 * q0 + q1 * q1);
-        const float sk = wave_sum(k0 * k0 + k1 * k1);
+        const float sq = step_wave_sum(q0 * q0 + q1 * q1);
+        const float sk = step_wave_sum(k0 * k0 + k1 * k1);
         const float iq = 1.0f / sqrtf(sq + 1e-12f), ik = 1.0f / sqrtf(sk + 1e-12f);
         q0 = q0 * iq; q1 = q1 * iq; k0 = k0 * ik; k1 = k1 * ik;
     }
@@ -1038,7 +1054,7 @@ __device__ float dn_compute(Buf<kDnBuf>& b, const PArgs& a, const PLayer& L, int
             for (int w = 0; w < 8; w++) y += ry[w * kDnCols + lane];
         }
         if (L.dn_flags & ANELM_DN_GATED_NORM) {
-            const float ss = wave_sum(lane < kDnCols ? y * y : 0.f);
+            const float ss = step_wave_sum(lane < kDnCols ? y * y : 0.f);
             if (lane == 0) stf_sc(a.dnss + hd * kDnSlabs + c, ss);
         } else if (lane < kDnCols) {
             L.core_out[(size_t)hd * kDnD + kDnCols * c + lane] = y;
@@ -1060,7 +1076,7 @@ __device__ void dn_finish(const PArgs& a, const PLayer& L, float y, int lane) {
         z = L.dn_z[(size_t)hd * kDnD + kDnCols * c + lane];
         w = L.dn_norm_w[kDnCols * c + lane];
     }
-    const float ss = wave_sum(part);
+    const float ss = step_wave_sum(part);
     const float inv = 1.0f / sqrtf(ss / (float)kDnD + 1e-6f);
     if (lane < kDnCols) {
         float o = (y * inv) * w;
@@ -1116,9 +1132,9 @@ __device__ __forceinline__ void attn_merge_fin(const PArgs& a, const PLayer& L, 
     if (kvh >= a.Hkv) return;
     const int g = rr / (kAttnD / 16), j = rr - g * (kAttnD / 16);
     const int hq = kvh * kAttnG + g;
-    const float M = wave_max(r.m);
+    const float M = step_wave_max(r.m);
     const float wt = r.m != -INFINITY ? __expf(r.m - M) : 0.f;
-    const float Ls = wave_sum(r.l * wt);
+    const float Ls = step_wave_sum(r.l * wt);
 #pragma unroll
     for (int k = 0; k < 16; k++) r.o[k] *= wt;
     // 16 sums over the 64 lanes: lane li < 16 of each 16-lane row ends with
@@ -1267,7 +1283,7 @@ __device__ __forceinline__ void stage_x_fin(const PArgs& a, int lane, char* lds)
         const f32x4 xv = xpark[lane + 64 * j];
         ss += xv.x * xv.x + xv.y * xv.y + xv.z * xv.z + xv.w * xv.w;
     }
-    ss = wave_sum(ss);
+    ss = step_wave_sum(ss);
     const float inv = 1.0f / sqrtf(ss / (float)a.H + a.eps);
     u32x2* xs = reinterpret_cast<u32x2*>(lds + kLdsXs);
 #pragma unroll
