@@ -225,3 +225,41 @@ def test_deltanet_prefill_from_proj_matches_decode_steps(anelm, orc, dev, S, Hk,
     assert pos.value == p
     assert_close(to_host(Sd), St, what="state")
     assert np.array_equal(to_host(csd), cs), "conv ring"
+
+
+@pytest.mark.parametrize("S,Hk,Hv,flags,pos0,K", [
+    (1, 16, 32, 5, 2, 4),      # one token
+    (3, 16, 16, 7, 1, 4),      # as many tokens as the conv ring holds
+    (63, 2, 4, 5, 0, 4),       # one token short of a chunk
+    (64, 2, 2, 7, 2, 4),       # one whole chunk
+    (65, 2, 4, 7, 0, 4),       # one token past it
+    (2060, 16, 32, 5, 1, 4),   # enough chunks for both value heads of a key head in one workgroup
+    (130, 2, 4, 5, 1, 3),      # another conv width: the conv in a pass of its own
+    (130, 3, 3, 7, 0, 4),      # rows not 16-byte aligned: likewise
+])
+def test_deltanet_prefill_from_proj_cuts(anelm, orc, dev, S, Hk, Hv, flags, pos0, K):
+    """The prompt pass from projection rows at the edges of its 64-token chunks
+    and of its choices, token by token against the decode recurrence (the same
+    bars as above; the conv ring holds projection values, bit for bit)."""
+    rng = np.random.default_rng(1850 + S + Hv + flags + K)
+    d = 128
+    qkv = 2 * Hk * d + Hv * d
+    St = (0.1 * rng.standard_normal((Hv, d, d))).astype(np.float32)
+    conv_w = (0.5 * rng.standard_normal((qkv, K))).astype(np.float32)
+    cs = (0.5 * rng.standard_normal((qkv, K - 1))).astype(np.float32)
+    A = np.exp(rng.uniform(0, np.log(16), Hv)).astype(np.float32)
+    dtb = rng.standard_normal(Hv).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    proj = rng.standard_normal((S, qkv + Hv * d + 2 * Hv)).astype(np.float32)
+    Sd, csd = to_dev(St, dev), to_dev(cs, dev)
+    pos = ctypes.c_int(pos0)
+    y = to_host(anelm.ops.deltanet_prefill_from_proj(Sd, csd, pos, to_dev(proj, dev), to_dev(conv_w, dev),
+                                                     to_dev(A, dev), to_dev(dtb, dev), to_dev(nw, dev), Hk,
+                                                     flags, K))
+    p = pos0
+    for t in range(S):
+        yw, St, cs, p = orc.deltanet_from_proj(St, cs, p, proj[t], conv_w, A, dtb, nw, Hk, Hv, K, flags)
+        assert_close(y[t], yw, what=f"y token {t}")
+    assert pos.value == p
+    assert_close(to_host(Sd), St, what="state")
+    assert np.array_equal(to_host(csd), cs), "conv ring"
