@@ -1563,9 +1563,30 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const DecodeParams p)
     }
 }
 
-// Rings the matrix-core kernel takes.
+// Shapes of the matrix-core ring kernel, and the rings it takes: its LDS loads
+// need 16-byte aligned rows (attn_decode_kernel takes the others).
 template <typename KV>
 constexpr bool ring_mfma(int D, int G) { return std::is_same<KV, uint16_t>::value && D == 256 && G == 4; }
+bool ring_aligned(const DecodeParams& p) {
+    return ((reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 15) == 0;
+}
+
+int launch_ring_mfma(const DecodeParams& p, dim3 grid, hipStream_t st) {
+    static std::atomic<bool> attr{false};
+    if (!attr.load(std::memory_order_acquire)) {
+        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_mfma_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kRW * kRVB));
+        attr.store(true, std::memory_order_release);
+    }
+    // a second set of V buffers where a wave walks several blocks
+    const int bufs = std::min(p.kps, p.len) > kRW * kRBlk ? 2 : 1;
+    hipLaunchKernelGGL(attn_ring_mfma_kernel, grid, dim3(kRNT), bufs * kRW * kRVB, st,
+                       static_cast<const uint16_t*>(p.k_cache), static_cast<const uint16_t*>(p.v_cache), p.q,
+                       p.q_stride, (int)p.tok_stride, (int)(p.head_stride / 256), p.start, p.len, p.cap, p.kps,
+                       (p.len + p.kps - 1) / p.kps, p);
+    ANELM_LAUNCHED("attn_ring_mfma_kernel");
+    return ANELM_OK;
+}
 
 template <typename KV, int D, int G>
 int launch_g(DecodeParams& p, dim3 grid, hipStream_t st) {
@@ -1593,20 +1614,9 @@ int launch_g(DecodeParams& p, dim3 grid, hipStream_t st) {
             hipLaunchKernelGGL((attn_paged_mfma_kernel<D, G>), pgrid, dim3(kNT), 0, st, p);
             ANELM_LAUNCHED("attn_paged_mfma_kernel");
         }
-    } else if constexpr (ring_mfma<KV>(D, G)) {
-        static std::atomic<bool> attr{false};
-        if (!attr.load(std::memory_order_acquire)) {
-            ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_mfma_kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kRW * kRVB));
-            attr.store(true, std::memory_order_release);
-        }
-        // a second set of V buffers where a wave walks several blocks
-        const int bufs = std::min(p.kps, p.len) > kRW * kRBlk ? 2 : 1;
-        hipLaunchKernelGGL(attn_ring_mfma_kernel, grid, dim3(kRNT), bufs * kRW * kRVB, st,
-                           static_cast<const uint16_t*>(p.k_cache), static_cast<const uint16_t*>(p.v_cache), p.q,
-                           p.q_stride, (int)p.tok_stride, (int)(p.head_stride / D), p.start, p.len, p.cap, p.kps,
-                           (p.len + p.kps - 1) / p.kps, p);
-        ANELM_LAUNCHED("attn_ring_mfma_kernel");
+    } else if (ring_mfma<KV>(D, G) && ring_aligned(p)) {
+        const int rc = launch_ring_mfma(p, grid, st);
+        if (rc) return rc;
     } else {
         hipLaunchKernelGGL((attn_decode_kernel<KV, D, G>), grid, dim3(ring_threads<G>()), 0, st, p);
         ANELM_LAUNCHED("attn_decode_kernel");
@@ -1674,7 +1684,7 @@ int run_decode(DecodeParams& p, int kv_dtype, int n_heads, int D, int n_seqs, in
     const int Hkv = p.n_kv_heads;
     const int G = n_heads / Hkv;
     int kps = p.paged ? kPagedSplit : 256 / G;
-    if (!p.paged && kv_dtype == ANELM_F16 && ring_mfma<uint16_t>(D, G)) {
+    if (!p.paged && kv_dtype == ANELM_F16 && ring_mfma<uint16_t>(D, G) && ring_aligned(p)) {
         Device* dev = device();
         if (dev == nullptr) return ANELM_EHIP;
         kps = ring_split_keys(max_len, Hkv, dev->num_cus);

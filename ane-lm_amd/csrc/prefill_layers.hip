@@ -354,8 +354,10 @@ extern "C" int anelm_full_attn_prefill(float* out, const float* q_gate, const fl
     // the prompt's keys straight to their slots (free ones: L <= cap).  Once it
     // overflows inside the prompt, early rows still see keys that later ones
     // overwrite: the keys are gathered into one sequence, and those that
-    // survive are written to the ring afterwards.
-    const bool direct = L <= cap && (size_t)cap * n_kv_heads * D * 2 < 0x7fffffffu;
+    // survive are written to the ring afterwards.  The core's LDS loads need
+    // 16-byte aligned rows, so a ring elsewhere is gathered too.
+    const bool aligned = ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) == 0;
+    const bool direct = aligned && L <= cap && (size_t)cap * n_kv_heads * D * 2 < 0x7fffffffu;
     const size_t qb = ((size_t)S * n_heads * D * 2 + 255) & ~(size_t)255;
     const size_t kb = direct ? 0 : ((size_t)L * n_kv_heads * D * 2 + 255) & ~(size_t)255;
     char* ws = static_cast<char*>(workspace2(qb + 2 * kb, st));

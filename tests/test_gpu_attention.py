@@ -107,17 +107,18 @@ def test_full_attn_decode_split_merge(anelm, orc, dev, n_heads, n_kv_heads, head
     _check_decode(_run_decode(anelm, c, dev), _oracle_decode(orc, c))
 
 
-@pytest.mark.parametrize("Hq,Hkv,cached,start,rope_mode,rot,gate,scale", [
-    (8, 2, 0, 0, 0, 64, True, 1.0),          # the new key alone: one wave has a key, seven none
-    (16, 4, 15, 3, 1, 64, True, 1.0),        # a whole 16-key block, half-split pairs
-    (4, 1, 16, 0, 0, 0, False, 1.0),         # the new key alone in its block; no rotation, no gate
-    (16, 4, 127, 100, 1, 96, True, 1.0),     # one full split; pairs that are no multiple of a lane's dims apart
-    (8, 2, 128, 7, 0, 64, True, 1.0),        # the new key alone in its split
-    (8, 2, 2047, 60, 0, 64, True, 1e-4),     # 16 splits, merged in the kernel; tiny rows
-    (8, 2, 2048, 60, 0, 64, True, 3e4),      # 17 splits: the merge kernel; rows past fp16's range
-    (16, 4, 16500, 900, 0, 64, True, 1.0),   # three rounds of blocks per wave, a part-filled last one
+@pytest.mark.parametrize("Hq,Hkv,cached,start,rope_mode,rot,gate,scale,off", [
+    (8, 2, 0, 0, 0, 64, True, 1.0, 0),          # the new key alone: one wave has a key, seven none
+    (16, 4, 15, 3, 1, 64, True, 1.0, 0),        # a whole 16-key block, half-split pairs
+    (4, 1, 16, 0, 0, 0, False, 1.0, 0),         # the new key alone in its block; no rotation, no gate
+    (16, 4, 127, 100, 1, 96, True, 1.0, 0),     # one full split; pairs that are no multiple of a lane's dims apart
+    (8, 2, 128, 7, 0, 64, True, 1.0, 0),        # the new key alone in its split
+    (8, 2, 2047, 60, 0, 64, True, 1e-4, 0),     # 16 splits, merged in the kernel; tiny rows
+    (8, 2, 2048, 60, 0, 64, True, 3e4, 0),      # 17 splits: the merge kernel; rows past fp16's range
+    (16, 4, 16500, 900, 0, 64, True, 1.0, 0),   # three rounds of blocks per wave, a part-filled last one
+    (16, 4, 300, 9, 0, 64, True, 1.0, 2),       # rows at 4-byte aligned addresses: the vector kernel
 ])
-def test_full_attn_decode_matrix_core_ring(anelm, dev, Hq, Hkv, cached, start, rope_mode, rot, gate, scale):
+def test_full_attn_decode_matrix_core_ring(anelm, dev, Hq, Hkv, cached, start, rope_mode, rot, gate, scale, off):
     """fp16 rings of head_dim 256 with 4 query heads per kv head, at the edges
     of the kernel's blocks, splits and merges, every unused ring slot NaN.
     Against float64 over the same fp16 keys: the fp32 query and weights enter
@@ -132,7 +133,8 @@ def test_full_attn_decode_matrix_core_ring(anelm, dev, Hq, Hkv, cached, start, r
     free = np.setdiff1d(np.arange(cap), used)
     c.k_cache[free] = c.v_cache[free] = 0x7e00
     c.q_gate[:, :D] *= scale
-    kc, vc = to_dev(c.k_cache, dev), to_dev(c.v_cache, dev)
+    kc, vc = (torch.cat([torch.zeros(off, dtype=torch.float16, device=dev), to_dev(x, dev).flatten()])
+              [off:].view(x.shape) for x in (c.k_cache, c.v_cache))
     ring = anelm.ops.KVRing(cap, c.start, cached)
     # the rotation's fp32 cos and sin are given, so both sides use the same
     ang = float(c.pos) * c.theta ** (-np.arange(0, rot, 2) / max(rot, 1))

@@ -127,17 +127,18 @@ def test_full_attn_prefill_4096_rows(anelm, orc, dev):
         assert_close(got[t], want, what=f"row {t}")
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,cap,start,len0,rope_mode,pad,table_rows", [
-    (1, 8, 2, 64, 3, 0, 0, 0, 0),              # one token, nothing cached
-    (15, 8, 2, 4096, 4090, 4000, 0, 0, 4096),  # part-filled group, many key parts, wrap inside a tile
-    (17, 16, 4, 512, 500, 10, 1, 0, 512),      # one token past a group; wrap inside the prompt
-    (40, 16, 4, 64, 0, 10, 0, 1, 64),          # rows not 16-byte aligned; a column's first tile wholly masked
-    (33, 4, 1, 256, 255, 95, 1, 3, 20),        # one kv head; positions past the RoPE table
-    (24, 12, 3, 300, 7, 200, 0, 0, 300),       # kv heads that do not divide the XCDs
-    (500, 16, 4, 1024, 600, 300, 0, 0, 1024),  # several key parts of 16-token groups, wrapped ring
-    (2100, 16, 4, 4096, 0, 0, 0, 0, 4096),     # more workgroups than compute units
+@pytest.mark.parametrize("S,Hq,Hkv,cap,start,len0,rope_mode,pad,table_rows,off", [
+    (1, 8, 2, 64, 3, 0, 0, 0, 0, 0),              # one token, nothing cached
+    (15, 8, 2, 4096, 4090, 4000, 0, 0, 4096, 0),  # part-filled group, many key parts, wrap inside a tile
+    (17, 16, 4, 512, 500, 10, 1, 0, 512, 0),      # one token past a group; wrap inside the prompt
+    (40, 16, 4, 64, 0, 10, 0, 1, 64, 0),          # rows not 16-byte aligned; a column's first tile wholly masked
+    (33, 4, 1, 256, 255, 95, 1, 3, 20, 0),        # one kv head; positions past the RoPE table
+    (24, 12, 3, 300, 7, 200, 0, 0, 300, 0),       # kv heads that do not divide the XCDs
+    (500, 16, 4, 1024, 600, 300, 0, 0, 1024, 0),  # several key parts of 16-token groups, wrapped ring
+    (2100, 16, 4, 4096, 0, 0, 0, 0, 4096, 0),     # more workgroups than compute units
+    (40, 16, 4, 128, 100, 10, 0, 0, 64, 2),       # a ring at a 4-byte aligned address: gathered
 ])
-def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_mode, pad, table_rows):
+def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_mode, pad, table_rows, off):
     """Head_dim 256 with 4 query heads per kv head at the edges of its token
     groups, key tiles and key parts, reading the ring in place.  Against the
     layer's formulas in float64 on the GPU, over q and new keys rounded to fp16
@@ -150,7 +151,9 @@ def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_m
     proj[:, :Hq * 2 * D] = c["q_gate"].reshape(S, -1)
     proj[:, Hq * 2 * D:Hq * 2 * D + Hkv * D] = c["k"].reshape(S, -1)
     proj[:, Hq * 2 * D + Hkv * D:Hq * 2 * D + 2 * Hkv * D] = c["v"].reshape(S, -1)
-    pd, kc, vc = to_dev(proj, dev), to_dev(c["kc"], dev), to_dev(c["vc"], dev)
+    pd = to_dev(proj, dev)
+    kc, vc = (torch.cat([torch.zeros(off, dtype=torch.float16, device=dev), to_dev(c[x], dev).flatten()])[off:]
+              .view(c[x].shape) for x in ("kc", "vc"))
     qw, kw = to_dev(c["qw"], dev), to_dev(c["kw"], dev)
     ring = anelm.ops.KVRing(cap, start, len0)
     tab = anelm.ops.rope_table(rot, table_rows, 1e7, dev) if table_rows else None
