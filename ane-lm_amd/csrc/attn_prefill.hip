@@ -351,18 +351,17 @@ __host__ __device__ inline int split_steps(int KP, int grp, int S, int qoff) {
     return (qoff + end + 32 * KP - 1) / (32 * KP);
 }
 
-// Four output values (dims d .. d + 3 of row (tok, h)), normalised and gated.
+// Four output values (dims d .. d + 3 of row (tok, h)), gated by g, and the
+// gate logits of such a place (rows of any stride: dword aligned).
+typedef float f4_dw __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f4_dw split_gate(const float* gate, int gtok, int ghead, int tok, int h, int d) {
+    return *reinterpret_cast<const f4_dw*>(gate + (size_t)tok * gtok + (size_t)h * ghead + d);
+}
 template <bool OUT16, bool GATE>
-__device__ __forceinline__ void split_store(void* out, const float* gate, int gtok, int ghead, int tok, int h, int Hq,
-                                            int d, float4 x, float inv) {
-    x = make_float4(x.x * inv, x.y * inv, x.z * inv, x.w * inv);
-    if constexpr (GATE) {   // (rows of any stride: four dword loads)
-        const float* g = gate + (size_t)tok * gtok + (size_t)h * ghead + d;
-        x.x = x.x / (1.0f + expf(-g[0]));
-        x.y = x.y / (1.0f + expf(-g[1]));
-        x.z = x.z / (1.0f + expf(-g[2]));
-        x.w = x.w / (1.0f + expf(-g[3]));
-    }
+__device__ __forceinline__ void split_store(void* out, int tok, int h, int Hq, int d, float4 x, f4_dw g) {
+    if constexpr (GATE)
+        x = make_float4(x.x * sigmoid_short(g[0]), x.y * sigmoid_short(g[1]), x.z * sigmoid_short(g[2]),
+                        x.w * sigmoid_short(g[3]));
     const size_t off = ((size_t)tok * Hq + h) * 256 + d;
     if constexpr (OUT16)
         *reinterpret_cast<half4*>(static_cast<_Float16*>(out) + off) =
@@ -565,18 +564,39 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
         __syncthreads();
     }
     // this wave holds dim blocks QB * b .. + QB - 1 with b = kp (its bits high to low)
-    const int tok = tok0 + ((ln & 31) >> 2), h = kvh * 4 + (ln & 3), eh = ln >> 5;
     if (steps <= a.sps) {
-        if (tok >= a.S) return;
+        // Through the wave's own LDS (the exchange is over), so a store writes
+        // 256 consecutive bytes of four rows, and the gate logits are read
+        // that way, instead of 32 bytes of 32 rows; 64 dims at a time.  With
+        // the short sigmoid, 4096 tokens of 16 heads, us: the gated layer 222
+        // -> 209, fp32 rows without a gate 165 -> 161.
+        constexpr int ROW = 64 + 4;   // (rows start 4 banks apart)
+        float* const tr = reinterpret_cast<float*>(lds) + w * 32 * ROW;
         const float inv = 1.0f / lt;
+        const int d = 4 * (ln & 15), h = kvh * 4 + (ln >> 4);
 #pragma unroll
-        for (int j = 0; j < QB; j++)
+        for (int r = 0; r < QB / 2; r++) {
+            const int d0 = 32 * (QB * kp + 2 * r) + d;
+            f4_dw g[8];
+            if constexpr (GATE) {
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++)
-                split_store<OUT16, GATE>(a.out, a.gate, a.gtok, a.ghead, tok, h, a.Hq,
-                                         32 * (QB * kp + j) + 8 * g4 + 4 * eh,
-                                         make_float4(o[j][4 * g4], o[j][4 * g4 + 1], o[j][4 * g4 + 2], o[j][4 * g4 + 3]),
-                                         inv);
+                for (int i = 0; i < 8; i++)
+                    g[i] = split_gate(a.gate, a.gtok, a.ghead, min(tok0 + i, a.S - 1), h, d0);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; g4++) {
+                    const float16_t& c = o[2 * r + j];
+                    *reinterpret_cast<float4*>(tr + (ln & 31) * ROW + 32 * j + 8 * g4 + 4 * (ln >> 5)) =
+                        make_float4(c[4 * g4] * inv, c[4 * g4 + 1] * inv, c[4 * g4 + 2] * inv, c[4 * g4 + 3] * inv);
+                }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4 x = *reinterpret_cast<const float4*>(tr + (4 * i + (ln >> 4)) * ROW + d);
+                if (tok0 + i < a.S) split_store<OUT16, GATE>(a.out, tok0 + i, h, a.Hq, d0, x, g[i]);
+            }
+        }
         return;
     }
     float* rec = a.rec + ((size_t)(kvh * a.ngrp + grp) * a.parts + part) * split_rec_floats<KP>();
@@ -639,8 +659,11 @@ __global__ __launch_bounds__(kGNT) void prefill_split_combine(const SplitArgs a)
         }
         M = Mn;
     }
-    split_store<OUT16, GATE>(a.out, a.gate, a.gtok, a.ghead, tok, kvh * 4 + (ln & 3), a.Hq,
-                             32 * (QB * kp + slot / 4) + 8 * (slot % 4) + 4 * (ln >> 5), acc, 1.0f / lt);
+    const float inv = 1.0f / lt;
+    const int h = kvh * 4 + (ln & 3), d = 32 * (QB * kp + slot / 4) + 8 * (slot % 4) + 4 * (ln >> 5);
+    f4_dw g = {};
+    if constexpr (GATE) g = split_gate(a.gate, a.gtok, a.ghead, tok, h, d);
+    split_store<OUT16, GATE>(a.out, tok, h, a.Hq, d, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv), g);
 }
 
 // How a prompt is cut: the least estimated time over both KP and 1 .. 16 parts
