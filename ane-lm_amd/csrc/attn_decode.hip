@@ -1378,6 +1378,10 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
         red_m[w][lane] = m_run;
         red_l[w][lane] = l_run;
     }
+    // (a wave without a block has not waited for its V loads, which land where
+    // its rows are about to be written)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" ::: "memory");
     float* ro = reinterpret_cast<float*>(vdyn + w * kRVB);   // this wave's O rows [G][D], over its own V block
     f32x4_t h1[NTD / 2];
 #pragma unroll

@@ -170,6 +170,25 @@ def test_full_attn_decode_matrix_core_ring(anelm, dev, Hq, Hkv, cached, start, r
         assert err <= tol, (h, err, tol)
 
 
+@pytest.mark.parametrize("cached", [0, 40, 111, 128])
+def test_full_attn_decode_idle_waves(anelm, dev, cached):
+    """Splits with fewer 16-key blocks than waves: the waves without a block
+    load the last key's slot too (here still unwritten, every pair of its
+    halves a NaN as fp32, which a weight of 0 would not silence) over the LDS
+    that they then give their empty rows in; those loads have landed by then."""
+    c = attn_decode_case(360 + cached, n_heads=4, n_kv_heads=1, cached=cached, capacity=256, start=0)
+
+    def step():
+        return to_host(anelm.ops.full_attn_decode(
+            to_dev(c.q_gate, dev), to_dev(c.k, dev), to_dev(c.v, dev), to_dev(c.k_cache, dev), to_dev(c.v_cache, dev),
+            to_dev(c.q_norm_w, dev), to_dev(c.k_norm_w, dev), anelm.ops.KVRing(c.capacity, c.start, c.length),
+            c.n_heads, c.n_kv_heads, c.head_dim, c.rot_dim, c.pos, c.theta, c.eps))
+
+    clean = step()
+    c.v_cache[cached:] = 0x7fff
+    assert np.array_equal(step(), clean)
+
+
 def test_full_attn_decode_table_row(anelm, orc, dev):
     """cos/sin passed as the reference's table row give the same step."""
     c = attn_decode_case(305)
