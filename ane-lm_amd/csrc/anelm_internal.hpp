@@ -54,8 +54,10 @@ struct StreamState {
     size_t ws_bytes = 0;
     void* ws2 = nullptr;      // second slot: split-K partials of the batched GEMM
     size_t ws2_bytes = 0;
+    void* wsp = nullptr;      // operands of the LUT6 prompt product
+    size_t wsp_bytes = 0;
     uint32_t* counters = nullptr;
-    std::mutex mu;            // guards growth of ws / ws2
+    std::mutex mu;            // guards growth of ws / ws2 / wsp
 };
 
 struct Device {
@@ -79,6 +81,10 @@ int stream_release(hipStream_t stream);
 void* workspace(size_t bytes, hipStream_t stream);
 // Same, from a second buffer of the stream (for callees of a workspace user).
 void* workspace2(size_t bytes, hipStream_t stream);
+// The LUT6 prompt product's own buffer: a long prompt takes hundreds of MB, and
+// growing one of the others would free what a graph captured from a smaller
+// call still points to.  (That product is never captured.)
+void* prompt_workspace(size_t bytes, hipStream_t stream);
 
 // Workgroup barrier for LDS exchange only: this wave's LDS operations
 // complete, then s_barrier.  __syncthreads() also carries a release fence that

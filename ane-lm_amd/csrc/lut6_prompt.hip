@@ -397,7 +397,7 @@ int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const floa
     size_t bytes = 0;
     for (int b0 = 0; b0 < batch; b0 += kMaxRows)
         for (int n0 = 0; n0 < out_dim; n0 += n_max) bytes = std::max(bytes, plan(b0, n0).bytes);
-    char* ws = static_cast<char*>(workspace2(bytes, st));
+    char* ws = static_cast<char*>(prompt_workspace(bytes, st));
     if (!ws) {
         (void)hipGetLastError();   // a failed allocation is no launch error of the path taken instead
         return ANELM_ENOMEM;

@@ -113,6 +113,12 @@ void* workspace2(size_t bytes, hipStream_t stream) {
     return grow(s, s->ws2, s->ws2_bytes, bytes);
 }
 
+void* prompt_workspace(size_t bytes, hipStream_t stream) {
+    StreamState* s = stream_state(stream);
+    if (!s) return nullptr;
+    return grow(s, s->wsp, s->wsp_bytes, bytes);
+}
+
 uint32_t* counters(size_t n, CounterUser user, hipStream_t stream) {
     static_assert((size_t)kCtrUsers * kCounterRange <= kCounterPool, "counter ranges exceed the pool");
     if (n > kCounterRange) {
@@ -141,6 +147,7 @@ int stream_release(hipStream_t stream) {
     hipError_t e = hipStreamSynchronize(stream);
     if (s->ws) (void)hipFree(s->ws);
     if (s->ws2) (void)hipFree(s->ws2);
+    if (s->wsp) (void)hipFree(s->wsp);
     (void)hipFree(s->counters);
     delete s;
     if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");

@@ -1,5 +1,7 @@
 """GPU parity of the LUT6 kernels: exhaustive unpack, GEMV, the fused
 SwiGLU FFN block with residual, and the top-k LM head."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -66,6 +68,37 @@ def test_gemm_batched(anelm, orc, dev, out_dim, in_dim, batch):
     # repeated call: same bits (no state carried between launches)
     again = to_host(anelm.ops.lut6_gemm(to_dev(packed, dev), to_dev(lut, dev), to_dev(x, dev), out_dim, in_dim))
     assert np.array_equal(got, again)
+
+
+def test_prompt_call_leaves_captured_gemm(anelm, dev):
+    """A graph captured from a 32-input product in column slices holds the
+    stream's scratch; a prompt-sized product later on that stream takes its
+    own buffer, so every replay gives the eager result."""
+    out_dim, in_dim = 2560, 9216
+    packed, lut, _ = lut6_matrix(690, out_dim, in_dim)
+    w, lut = to_dev(packed, dev), to_dev(lut, dev)
+    g = torch.Generator(device=dev).manual_seed(691)
+    x = torch.randn(32, in_dim, generator=g, device=dev)
+    prompt = torch.randn(4096, in_dim, generator=g, device=dev)
+    y = torch.empty(32, out_dim, device=dev)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        want = anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim).clone()
+        graph = torch.cuda.CUDAGraph()
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim, out=y)
+        first = None
+        for rows in (100, 4096, 700):
+            big = anelm.ops.lut6_gemm(w, lut, prompt[:rows], out_dim, in_dim)
+            y.zero_()
+            graph.replay()
+            s.synchronize()
+            assert torch.equal(y, want), rows
+            first = big[:100].clone() if first is None else first
+        assert_close(to_host(big[:100]), to_host(first), rel=1e-6, max_abs=1e-4, what="prompt rows beside the replays")
+    del graph
+    anelm.call("anelm_stream_release", ctypes.c_void_p(s.cuda_stream))
 
 
 def test_gemm_accumulate_and_batched_ffn(anelm, orc, dev):
