@@ -205,30 +205,6 @@ __device__ __forceinline__ void rotate_pair(float& o0, float& o1, float v0, floa
     o1 = v0 * s + v1 * c;
 }
 
-// exp(x) = 2^(x log2 e), the product's rounding error and the constant's low
-// part carried to the result: within 2 ulp where it is not below 2^-126 (there
-// 0).  A fifth of expf's instructions; for kernels that evaluate one per few
-// bytes, where expf and an IEEE division bound them instead of memory.
-__device__ __forceinline__ float exp_short(float x) {
-    x = x < -104.f ? -104.f : x;   // (NaN stays; below, the correction would be inf - inf)
-    const float t = x * 1.44269504f;
-    const float lo = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    return fmaf(e, lo * 0.693147181f, e);
-}
-
-// 1 / (1 + exp(-x)) likewise (v_rcp_f32 and one Newton step; 1.6e-38 from
-// -87.3 down).
-__device__ __forceinline__ float sigmoid_short(float x) {
-    const float n = __builtin_amdgcn_fmed3f(-x, -87.f, 87.f);
-    const float t = n * 1.44269504f;
-    const float lo = fmaf(n, 1.92596299e-8f, fmaf(n, 1.44269504f, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    const float d = 1.0f + fmaf(e, lo * 0.693147181f, e);
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-
 __device__ __forceinline__ float shfl_xor(float v, int mask) {
     return __shfl_xor(v, mask, 64);
 }

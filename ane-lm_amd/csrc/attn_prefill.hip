@@ -360,8 +360,8 @@ __device__ __forceinline__ f4_dw split_gate(const float* gate, int gtok, int ghe
 template <bool OUT16, bool GATE>
 __device__ __forceinline__ void split_store(void* out, int tok, int h, int Hq, int d, float4 x, f4_dw g) {
     if constexpr (GATE)
-        x = make_float4(x.x * sigmoid_short(g[0]), x.y * sigmoid_short(g[1]), x.z * sigmoid_short(g[2]),
-                        x.w * sigmoid_short(g[3]));
+        x = make_float4(x.x / (1.0f + expf(-g[0])), x.y / (1.0f + expf(-g[1])), x.z / (1.0f + expf(-g[2])),
+                        x.w / (1.0f + expf(-g[3])));
     const size_t off = ((size_t)tok * Hq + h) * 256 + d;
     if constexpr (OUT16)
         *reinterpret_cast<half4*>(static_cast<_Float16*>(out) + off) =
@@ -567,9 +567,8 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
     if (steps <= a.sps) {
         // Through the wave's own LDS (the exchange is over), so a store writes
         // 256 consecutive bytes of four rows, and the gate logits are read
-        // that way, instead of 32 bytes of 32 rows; 64 dims at a time.  With
-        // the short sigmoid, 4096 tokens of 16 heads, us: the gated layer 222
-        // -> 209, fp32 rows without a gate 165 -> 161.
+        // that way, instead of 32 bytes of 32 rows; 64 dims at a time (4096
+        // tokens of 16 heads, fp32 rows without a gate: 165 -> 161 us).
         constexpr int ROW = 64 + 4;   // (rows start 4 banks apart)
         float* const tr = reinterpret_cast<float*>(lds) + w * 32 * ROW;
         const float inv = 1.0f / lt;

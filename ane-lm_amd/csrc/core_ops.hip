@@ -110,8 +110,8 @@ __global__ __launch_bounds__(kNT) void rmsnorm_gated_rows128_kernel(float* out, 
     const float ss = wave_sum(xv.x * xv.x + xv.y * xv.y);
     const float inv = 1.0f / sqrtf(ss / 128.0f + 1e-6f);
     float o0 = (xv.x * inv) * wv.x, o1 = (xv.y * inv) * wv.y;
-    o0 = o0 * sigmoid_short(zv.x);
-    o1 = o1 * sigmoid_short(zv.y);
+    o0 = o0 / (1.0f + expf(-zv.x));
+    o1 = o1 / (1.0f + expf(-zv.y));
     *reinterpret_cast<float2*>(out + off) = make_float2(o0 * zv.x, o1 * zv.y);
 }
 

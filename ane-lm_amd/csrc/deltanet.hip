@@ -407,7 +407,7 @@ __device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x
     sum += x1 * w.y;
     sum += x2 * w.z;
     const float y = sum + x3 * w.w;
-    return y * sigmoid_short(y);
+    return y / (expf(-y) + 1.0f);
 }
 
 // ------------------------------------------- chunk preparation on fp32 MFMA
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(kPmNT, 2) void dn_chunk_prep_kernel(const ChunkArgs
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int i = i0 + e;
-                const float f = exp_short(lgt - lg[i + 1]);
+                const float f = expf(lgt - lg[i + 1]);
                 if (isA) o4[e] = i < t ? bs * f * gram[u][e] : 0.f;
                 else o4[e] = i <= t ? f * gram[u][e] : 0.f;
             }

@@ -22,6 +22,27 @@ def test_rmsnorm_and_gated(anelm, orc, dev):
     assert_close(got, orc.rmsnorm_gated(x, z, w), rel=1e-6, what="rmsnorm_gated")
 
 
+def test_rmsnorm_gated_special_z(anelm, dev):
+    """SiLU of z as z / (1 + exp(-z)) evaluates in fp32: 0 from -88.73 down (not
+    the least normal number times z), NaN for NaN and for -inf (0 x inf), z
+    itself for large z.  Rows of 128, the one-load-per-lane kernel."""
+    rng = np.random.default_rng(103)
+    x = rng.standard_normal((16, 128)).astype(np.float32)
+    w = (1 + 0.05 * rng.standard_normal(128)).astype(np.float32)
+    z = (20 * rng.standard_normal((16, 128))).astype(np.float32)
+    z[:, :8] = [np.nan, np.inf, -np.inf, -89.0, -100.0, -200.0, 88.0, 1e30]
+    got = to_host(anelm.ops.rmsnorm_gated(to_dev(x, dev), to_dev(z, dev), to_dev(w, dev))).astype(np.float64)
+    n = x.astype(np.float64)
+    n = n / np.sqrt((n * n).mean(-1, keepdims=True) + 1e-6) * w
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = n * np.where(z < -88.73, 0.0, 1.0 / (1.0 + np.exp(-z.astype(np.float64)))) * z
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    # the norm's, exp's (2 ulp), the sum's, the quotient's and the products' rounding
+    assert (np.abs(got[fin] - want[fin]) <= 16 * 2.0 ** -24 * np.abs(want[fin]) + 1e-45).all()
+
+
 def test_l2norm_activations_softmax_matvec(anelm, orc, dev):
     rng = np.random.default_rng(101)
     x = rng.standard_normal((6, 128)).astype(np.float32) * 3

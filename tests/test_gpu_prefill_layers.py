@@ -199,6 +199,39 @@ def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_m
         assert_close(out.view(S, Hq, D)[:, h].cpu().numpy(), want.float().cpu().numpy(), what=f"head {h}")
 
 
+@pytest.mark.parametrize("S,Hq,Hkv,len0", [
+    (24, 8, 2, 0),       # one key part: gated in the kernel
+    (24, 8, 2, 3000),    # several: gated in the merge
+    (24, 4, 2, 0),       # two query heads per kv head
+])
+def test_full_attn_prefill_special_gates(anelm, dev, S, Hq, Hkv, len0):
+    """Gate logits that are NaN, infinite or past where exp overflows give what
+    x / (1 + exp(-g)) gives in fp32: NaN stays NaN, +inf passes the value, -inf
+    and anything below -88.8 gives 0.  Against the call without a gate; finite
+    logits within the quotient's, the sum's and (2 ulp) exp's rounding."""
+    D, cap = 256, 4096
+    c = _attn_case(1950 + len0, S, Hq, Hkv, D, cap, 5, len0)
+    rng = np.random.default_rng(1951)
+    special = np.array([np.nan, np.inf, -np.inf, -100.0, -90.0, -88.0, 88.0, 200.0], np.float32)
+    at = rng.integers(0, S * Hq * D, 400)
+    c["q_gate"][..., D:].reshape(-1)[:] = 0
+    gl = np.ascontiguousarray(c["q_gate"][..., D:]) + (8 * rng.standard_normal((S, Hq, D))).astype(np.float32)
+    gl.reshape(-1)[at] = special[np.arange(400) % len(special)]
+    c["q_gate"][..., D:] = gl
+
+    def run(gate):
+        return _run_prefill(anelm, dev, c, S, Hq, Hkv, D, 64, cap, 5, len0, len0, True, 0, gate)[0]
+
+    plain, got = (run(g).reshape(S, Hq, D).astype(np.float64) for g in (False, True))
+    assert np.isfinite(plain).all()
+    with np.errstate(over="ignore"):
+        # fp32's 1 + exp(-g) is infinite from -88.73 down
+        want = np.where(gl < -88.73, 0.0, plain / (1.0 + np.exp(-gl.astype(np.float64))))
+    assert np.array_equal(np.isnan(got), np.isnan(gl))
+    ok = ~np.isnan(gl)
+    assert (np.abs(got - want)[ok] <= 4 * 2.0 ** -23 * np.abs(want)[ok] + 1e-45).all()
+
+
 @pytest.mark.parametrize("S,Hk,Hv,flags,pos0", [
     (100, 16, 32, 5, 2),      # 4B layer: l2 norm + gated norm, conv ring position 2
     (130, 16, 16, 7, 0),      # 0.8B heads, transformers order
