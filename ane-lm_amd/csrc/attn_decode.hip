@@ -1070,11 +1070,13 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void a
 // per kv head)
 //
 // The matrix instructions take fp16, and the ring's rows are fp16 exactly; the
-// fp32 query and the fp32 weights are taken as three fp16 terms each (x = x1 +
-// x2 + x3, each the rounding of what is left, after an exact power-of-two
-// scaling: 33 bits, so nothing is lost against fp32).  Only 4 of the 16
-// columns of a 16x16 tile are query heads, so the terms ride along for free:
-// column (or row) n = head n % 4, term n / 4, n < 12.
+// fp32 query and the fp32 weights are taken as three fp16 terms each
+// (fp16_terms, after an exact power-of-two scaling of a query row to its
+// largest element: nothing of an element down to 2^-38 of it is lost).  Only 4
+// of the 16 columns of a 16x16 tile are query heads, so the terms ride along
+// for free: column (or row) n = head n % 4, term n / 4, n < 12.  A term that is
+// 0, and the zero columns and rows past 12, would make NaN of an infinity in
+// the ring; a wave that meets one takes its keys again in fp32.
 //   S = K Q^T   v_mfma_f32_16x16x32_f16, A = 16 K rows (lane (q, n) = key n,
 //               dims 32 s + 8 q .. +8), B = the query terms; the three term
 //               columns are then added across lanes: every lane (q, n) holds
@@ -1096,7 +1098,18 @@ constexpr int kRW = kRNT / 64;
 constexpr int kRBlk = 16;
 constexpr int kRVB = kRBlk * 256 * 2;          // bytes of one block's V rows
 constexpr int kRQ = 256 + 8;                   // query term row pitch (halfs): rows 4 banks apart
-constexpr float kRPScale = 256.f;              // of the weights, an exact power of two
+constexpr float kRPScale = 32768.f;            // of the weights, an exact power of two
+constexpr float kRTerm = 1.f / 2048.f;         // of each further term: 2^-11
+
+// v = t[0] + 2^-11 t[1] + 2^-22 t[2], |v| <= 2^15: each term the rounding of
+// what the ones before leave, scaled up so that its own 11 bits are in range.
+// 33 bits of v down to 2^-29 of the largest, all 24 of an fp32 v down to 2^-38.
+__device__ __forceinline__ void fp16_terms(float v, _Float16 (&t)[3]) {
+    t[0] = (_Float16)v;
+    const float r1 = (v - (float)t[0]) * 2048.f;
+    t[1] = (_Float16)r1;
+    t[2] = (_Float16)((r1 - (float)t[1]) * 2048.f);
+}
 
 // Adds the values of lanes n, n + 4, n + 8, n + 12 of each 16-lane row.
 __device__ __forceinline__ float row_quad_sum(float v) {
@@ -1235,23 +1248,23 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
             }
         }
         if (isq) {
-            // the row scaled by a power of two to at most 2^8, then its three terms
+            // the row scaled by a power of two to at most 2^15, then its three terms
             const float mx = wave_max(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
-            const int e = min(max(__builtin_amdgcn_frexp_expf(mx), -100), 120);
-            const float up = ldexpf(1.0f, 8 - e);
+            const int e = min(max(__builtin_amdgcn_frexp_expf(mx), -100), 128);
+            const float up = ldexpf(1.0f, 15 - e);
             half4_t t1, t2, t3;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const float v = x[i] * up;
-                t1[i] = (_Float16)v;
-                const float r1 = v - (float)t1[i];
-                t2[i] = (_Float16)r1;
-                t3[i] = (_Float16)(r1 - (float)t2[i]);
+                _Float16 t[3];
+                fp16_terms(x[i] * up, t);
+                t1[i] = t[0];
+                t2[i] = t[1];
+                t3[i] = t[2];
             }
             *reinterpret_cast<half4_t*>(&q16[w][4 * lane]) = t1;
             *reinterpret_cast<half4_t*>(&q16[4 + w][4 * lane]) = t2;
             *reinterpret_cast<half4_t*>(&q16[8 + w][4 * lane]) = t3;
-            if (lane == 0) qscale[w] = ldexpf(1.0f, e - 8);
+            if (lane == 0) qscale[w] = ldexpf(1.0f, e - 15);
         } else {
             append(0, x);
         }
@@ -1266,11 +1279,13 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
         if (n >= 12) qb[s] = half8_t{};
     }
     const float scale = p.scale * qscale[n & 3];
+    const float term = n < 4 ? 1.f : n < 8 ? kRTerm : n < 12 ? kRTerm * kRTerm : 0.f;   // of this column
 
     f32x4_t o[NTD];
 #pragma unroll
     for (int t = 0; t < NTD; t++) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;   // head n % 4 of this wave
+    float odd = 0.f;                        // NaN once a score or output is not finite
     const int tr_off = (16 * ((n & 3) >> 1) + 4 * q + (n >> 2)) * 16 + (n & 1) * 8;
     int buf = 0;
     for (int blk = w; blk < nblk; blk += kRW, buf ^= 1) {
@@ -1297,7 +1312,8 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
         float sc[4], bm = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float full = row_quad_sum(sa[i] + sb[i]);   // (n >= 12: zero columns)
+            const float full = row_quad_sum((sa[i] + sb[i]) * term);   // (n >= 12: zero columns)
+            odd = fmaf(full, 0.f, odd);
             sc[i] = 4 * q + i < left ? full * scale : -INFINITY;
             bm = fmaxf(bm, sc[i]);
         }
@@ -1312,11 +1328,9 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
             const float e = __expf(sc[i] - m_use);   // masked keys: 0
             psum += e;
             // this lane's term of the weight
-            const float v = e * kRPScale;
-            const _Float16 t1 = (_Float16)v;
-            const float r1 = v - (float)t1;
-            const _Float16 t2 = (_Float16)r1, t3 = (_Float16)(r1 - (float)t2);
-            pa[i] = n < 4 ? t1 : n < 8 ? t2 : n < 12 ? t3 : (_Float16)0.f;
+            _Float16 t[3];
+            fp16_terms(e * kRPScale, t);
+            pa[i] = n < 4 ? t[0] : n < 8 ? t[1] : n < 12 ? t[2] : (_Float16)0.f;
         }
         l_run = l_run * alpha + psum;
         m_run = m_new;
@@ -1373,11 +1387,6 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
     // ---- merge the waves.  The three term rows of a head (lanes q = 0, 1, 2;
     // row 3 is zero) are added by two half exchanges: lane (q, n) ends with
     // tiles 4 a + q, a < 4
-    l_run = pair_sum<16>(pair_sum<32>(l_run));
-    if (lane < G) {
-        red_m[w][lane] = m_run;
-        red_l[w][lane] = l_run;
-    }
     // (a wave without a block has not waited for its V loads, which land where
     // its rows are about to be written)
     __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1387,19 +1396,76 @@ __global__ __launch_bounds__(kRNT) __attribute__((amdgpu_waves_per_eu(2))) void 
 #pragma unroll
     for (int a = 0; a < NTD / 4; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)   // tiles 4 a + b (lanes < 32) and 4 a + b + 2
+        for (int b = 0; b < 2; b++)   // tiles 4 a + b (lanes < 32) and 4 a + b + 2: terms 0 (1) and 2 (3)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const Swapped s = lane_swap<32>(o[4 * a + b][i], o[4 * a + b + 2][i]);
-                h1[2 * a + b][i] = s.r[0] + s.r[1];
+                h1[2 * a + b][i] = fmaf(s.r[1], kRTerm * kRTerm, s.r[0]);
             }
 #pragma unroll
     for (int a = 0; a < NTD / 4; a++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {   // tiles (lane bit 4 clear) 2 a' and (set) 2 a' + 1
+        for (int i = 0; i < 4; i++) {   // tiles (lane bit 4 clear) 2 a' and (set) 2 a' + 1: terms 0 + 2 and 1 (+ 3)
             const Swapped s = lane_swap<16>(h1[2 * a][i], h1[2 * a + 1][i]);
-            ro[i * D + 16 * (4 * a + q) + n] = s.r[0] + s.r[1];
+            const float v = fmaf(s.r[1], kRTerm, s.r[0]);
+            odd = fmaf(v, 0.f, odd);
+            ro[i * D + 16 * (4 * a + q) + n] = v;
         }
+    l_run = pair_sum<16>(pair_sum<32>(l_run));
+    if (lane < G) {
+        red_m[w][lane] = m_run;
+        red_l[w][lane] = l_run;
+    }
+    if (__any(odd != odd)) {
+        // an infinity or NaN among the wave's rows: zero terms and the zero
+        // columns and rows turn it into NaN for every head (0 x inf), so the
+        // wave's keys are taken one by one in fp32, lane = 4 dims
+        float q4[G][4], m4[G], l4[G], o4[G][4];
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            m4[g] = -INFINITY;
+            l4[g] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int d = 4 * lane + i;
+                q4[g][i] = fmaf(fmaf((float)q16[8 + g][d], kRTerm, (float)q16[4 + g][d]), kRTerm, (float)q16[g][d]) *
+                           qscale[g];
+                o4[g][i] = 0.f;
+            }
+        }
+        for (int blk = w; blk < nblk; blk += kRW)
+            for (int key = k0 + blk * kRBlk; key < min(k0 + (blk + 1) * kRBlk, kend); key++) {
+                int row = start + key;
+                row -= row >= cap ? cap : 0;
+                const bool newest = owner && key == len - 1;
+                const half4_t kh = *reinterpret_cast<const half4_t*>(
+                    newest ? &nkv[0][4 * lane] : kc + (size_t)row * tok_stride + 4 * lane);
+                const half4_t vh = *reinterpret_cast<const half4_t*>(
+                    newest ? &nkv[1][4 * lane] : vc + (size_t)row * tok_stride + 4 * lane);
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    float dot = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) dot = fmaf(q4[g][i], (float)kh[i], dot);
+                    const float sv = wave_sum(dot) * p.scale;
+                    const float mn = fmaxf(m4[g], sv), mu = mn == -INFINITY ? 0.f : mn;
+                    const float al = __expf(m4[g] - mu), e = __expf(sv - mu);
+                    l4[g] = fmaf(l4[g], al, e);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) o4[g][i] = fmaf(e, (float)vh[i], o4[g][i] * al);
+                    m4[g] = mn;
+                }
+            }
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) ro[g * D + 4 * lane + i] = o4[g][i] * kRPScale;
+            if (lane == 0) {
+                red_m[w][g] = m4[g];
+                red_l[w][g] = l4[g];
+            }
+        }
+    }
     lds_barrier();
     float* const out = p.out + (size_t)kvh * G * D;
     float* const part = p.part + (size_t)kvh * p.max_splits * G * REC;

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import assert_close, to_dev, to_host
+from gpu_util import assert_close, rel_l2, to_dev, to_host
 from workloads import attn_decode_case, f16, prefill_inputs, widen
 
 pytestmark = pytest.mark.gpu
@@ -187,6 +187,76 @@ def test_full_attn_decode_idle_waves(anelm, dev, cached):
     clean = step()
     c.v_cache[cached:] = 0x7fff
     assert np.array_equal(step(), clean)
+
+
+@pytest.mark.parametrize("what", ["v", "v_last", "v_new", "k_masked", "k_nan"])
+@pytest.mark.parametrize("cached", [20, 700, 9000])
+def test_full_attn_decode_infinite_rows(anelm, dev, what, cached):
+    """Infinities among the ring's used keys (values past fp16's range) give
+    what fp32 products give: an infinite value makes its output dim infinite, a
+    key whose score is -inf weighs nothing, a NaN key makes every head of its
+    kv head NaN -- and nothing else changes.  Query rows of one sign in dim 0,
+    where the infinite key element is, so all four heads score it -inf."""
+    D, Hq, Hkv, cap = 256, 8, 2, cached + 9
+    c = attn_decode_case(370 + cached % 89, n_heads=Hq, n_kv_heads=Hkv, cached=cached, capacity=cap, start=cap // 3,
+                         rot_dim=0)
+    used = (c.start + np.arange(cached)) % cap
+    c.q_gate[:, 0] = np.abs(c.q_gate[:, 0]) + 0.1
+    inf, slot = np.uint16(0x7c00), used[cached // 2]
+    if what == "v":
+        c.v_cache[slot, 0, 17] = inf
+    elif what == "v_last":
+        c.v_cache[used[-1], 0, 17] = inf
+    elif what == "v_new":
+        c.v[0, 17] = 1e5
+    elif what == "k_masked":
+        c.k_cache[slot, 0, 0] = inf | 0x8000
+    else:
+        c.k_cache[slot, 0, 5] = 0x7e00
+    kc, vc = to_dev(c.k_cache, dev), to_dev(c.v_cache, dev)
+    ring = anelm.ops.KVRing(cap, c.start, cached)
+    got = to_host(anelm.ops.full_attn_decode(to_dev(c.q_gate, dev), to_dev(c.k, dev), to_dev(c.v, dev), kc, vc, None,
+                                             None, ring, Hq, Hkv, D, 0, c.pos, c.theta, c.eps)).reshape(Hq, D)
+    slots = np.append(used, (c.start + cached) % cap)
+    kk, vv = widen(to_host(kc))[slots].astype(np.float64), widen(to_host(vc))[slots].astype(np.float64)
+    for h in range(Hq):
+        with np.errstate(invalid="ignore"):
+            s = kk[:, h * Hkv // Hq] @ c.q_gate[h, :D].astype(np.float64) / 16.0
+            p = np.exp(s - s.max())
+            v = np.where((p == 0)[:, None], 0.0, vv[:, h * Hkv // Hq])
+            want = (p / p.sum()) @ v / (1.0 + np.exp(-c.q_gate[h, D:].astype(np.float64)))
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isnan(got[h]), np.isnan(want)), (what, h)
+        assert np.array_equal(got[h][np.isinf(want)], want[np.isinf(want)]), (what, h)
+        if fin.any():
+            assert rel_l2(got[h][fin], want[fin]) <= 1e-5, (what, h)
+
+
+@pytest.mark.parametrize("cached", [60, 1000])
+def test_full_attn_decode_small_elements(anelm, dev, cached):
+    """Query elements and weights far below their row's largest keep fp32's bits:
+    one query element 2^24 times the others over keys that are 0 there, and one
+    key scoring 20 above the others over values that are 0 there."""
+    D, cap = 256, cached + 9
+    c = attn_decode_case(380, n_heads=4, n_kv_heads=1, cached=cached, capacity=cap, start=0, rot_dim=0)
+    c.q_gate[:, 3] = 2.0 ** 24
+    c.q_gate[:, 0] = 8.0
+    c.k_cache[:cached, :, 3] = 0
+    c.k_cache[:cached, :, 0] = f16(np.zeros((cached, 1), np.float32))
+    c.k_cache[cached // 2, 0, 0] = f16(np.array([40.0], np.float32))[0]
+    c.v_cache[cached // 2] = 0
+    c.k[:, 3] = c.k[:, 0] = 0
+    kc, vc = to_dev(c.k_cache, dev), to_dev(c.v_cache, dev)
+    got = to_host(anelm.ops.full_attn_decode(to_dev(c.q_gate, dev), to_dev(c.k, dev), to_dev(c.v, dev), kc, vc, None,
+                                             None, anelm.ops.KVRing(cap, 0, cached), 4, 1, D, 0, c.pos, c.theta,
+                                             c.eps, gate=False)).reshape(4, D)
+    kk, vv = widen(to_host(kc))[:cached + 1, 0].astype(np.float64), widen(to_host(vc))[:cached + 1, 0].astype(np.float64)
+    for h in range(4):
+        s = kk @ c.q_gate[h, :D].astype(np.float64) / 16.0
+        p = np.exp(s - s.max())
+        want = (p / p.sum()) @ vv
+        # fp32 sums of 256 products, the weights' exponential at |score| up to 25
+        assert rel_l2(got[h], want) <= 2.0 ** -24 * 16 * np.abs(s).max(), h
 
 
 def test_full_attn_decode_table_row(anelm, orc, dev):
