@@ -7,8 +7,8 @@
 // 128 times, 5.1 ms for the 2560 -> 2 x 9216 -> 2560 FFN block.  Here the
 // weights are decoded once into fp16 (exactly: a LUT entry is an fp16 value),
 // the inputs are rounded to fp16 once (as every LUT6 path takes them), and one
-// fp16 MFMA product with fp32 accumulation follows: that block takes 805 us
-// (weights and inputs prepared in 56 + 31 us, products 390 + 269).
+// fp16 MFMA product with fp32 accumulation follows: that block takes 795 us
+// (the two products with their preparation 410 + 235).
 // Reference math: matvec (core/cpu_ops.cpp:77-80) on the dequantised weights,
 // per input.
 //
@@ -24,6 +24,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
+#include <utility>
 
 namespace anelm {
 namespace {
@@ -34,6 +36,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kKB = 32;            // columns per block (one pipeline stage)
 constexpr int kRowB = kKB * 2;     // bytes of one row in one block
+constexpr int kChain = 8;          // column blocks per accumulation chain (256 columns)
 
 // Byte offset of 16-byte chunk c of row r in its column block.
 __device__ __forceinline__ int chunk_off(int r, int c) { return r * kRowB + ((c ^ (r >> 1)) & 3) * 16; }
@@ -157,17 +160,27 @@ struct PromptArgs {
     int accumulate;
 };
 
+template <int... S, class F>
+__device__ __forceinline__ void for_each_stage(std::integer_sequence<int, S...>, F f) {
+    (f(std::integral_constant<int, S>{}), ...);
+}
+
 // Tile of BM inputs x BN weight rows, WM x WN waves; wave tile (BM / WM) x
 // (BN / WN) in 32x32 blocks of v_mfma_f32_32x32x16_f16 (A = inputs, B = weight
 // rows, so 32 lanes hold 32 consecutive outputs of one input).  NS stages of
 // 32 columns in LDS, NS - 1 ahead in flight; the operands of the second half
 // of a stage are read while the first half is multiplied, those of the next
 // stage's first half (behind the one barrier per stage) while the second is.
-// Bound: at 256 x 256 the matrix units' power (with every CU busy 1.06 PFLOP/s
-// at 4096 x 18432 x 2560, stores of the 302 MB result included; 1.19 for the
-// library's 8192^3 product on the same card; with 160 of 256 CUs busy each CU
-// runs 1.6 times faster).  8 waves of 128 x 64 beat 4 of 128 x 128 (364 against
-// 410-434 us there): two waves per SIMD cover each other's waits.
+// The products accumulate in chains of kChain stages, each added to a sum in
+// fp32: one chain over all columns rounds at the size of the whole sum every
+// time, 3.2e-7 off 64 bits at 2560 columns and 6.1e-7 at 9216, where the passes
+// of 32 inputs and these chains are 1.2e-7 and 1.3 to 1.5e-7 off.  A wave's
+// blocks end their chains in different stages, so the additions hide behind the
+// other blocks' products (all at once they cost 5 % of the FFN block).
+// Bound: the matrix units' power (whole call with the preparation, us: 4096 x
+// 18432 x 2560 410, 4096 x 2560 x 9216 235; the library's 8192^3 product runs
+// at 1.19 PFLOP/s on the same card; with 160 of 256 CUs busy each CU runs 1.6
+// times faster).
 template <int BM, int BN, int WM, int WN, int NS>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WM * WN / 4, WM * WN / 4)))
 void prompt_gemm_kernel(const PromptArgs a) {
@@ -212,11 +225,11 @@ void prompt_gemm_kernel(const PromptArgs a) {
     // chunk 2 ks + lh of row lr (+ 32 j) of the wave's rows; rows 32 apart keep the permutation
     const int a_off = (wm * (BM / WM) + lr) * kRowB, b_off = BM * kRowB + (wn * (BN / WN) + lr) * kRowB;
     const int sw = (lr >> 1) & 3;
-    float16_t acc[MI][NI];
+    float16_t acc[MI][NI], sum[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; i++)
 #pragma unroll
-        for (int j = 0; j < NI; j++) acc[i][j] = float16_t{};
+        for (int j = 0; j < NI; j++) acc[i][j] = sum[i][j] = float16_t{};
     half8 fa[2][MI], fb[2][NI];
     auto read = [&](int i, int ks) __attribute__((always_inline)) {
         const char* base = lds + (i % NS) * STAGE + (((2 * ks + lh) ^ sw) & 3) * 16;
@@ -225,12 +238,16 @@ void prompt_gemm_kernel(const PromptArgs a) {
 #pragma unroll
         for (int j = 0; j < NI; j++) fb[ks][j] = *reinterpret_cast<const half8*>(base + b_off + j * 32 * kRowB);
     };
-    auto mul = [&](int ks) __attribute__((always_inline)) {
+    constexpr int NB = MI * NI;
+    static_assert(NB <= kChain, "a stage of the chain for every block");
+    // `last`: the block multiplied last, `fresh`: it starts a new chain
+    auto mul = [&](int ks, int last, bool fresh) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
+        for (int b = 0; b < NB; b++) {
+            const int e = (last + 1 + b) % NB, i = e / NI, j = e % NI;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[ks][i], fb[ks][j],
+                                                              fresh && e == last ? float16_t{} : acc[i][j], 0, 0, 0);
+        }
     };
     constexpr int VM = (NS - 2) * LPW;   // loads that may stay in flight while the next stage is used
     constexpr int kWait = 0x0070 | (VM & 15) | ((VM >> 4) << 14);   // vmcnt(VM), lgkmcnt(0)
@@ -239,13 +256,18 @@ void prompt_gemm_kernel(const PromptArgs a) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(0, 0);
-    for (int i = 0; i < nk; i++) {
+    // Stage i.  FL in 0 .. NB - 1: block FL of the wave's ends its chain of
+    // kChain stages here: it is added to the sum while the other blocks' products run.
+    auto stage = [&](int i, auto fl) __attribute__((always_inline)) {
+        constexpr int FL = decltype(fl)::value;
+        constexpr bool flush = FL >= 0 && FL < NB;
         issue(i + NS - 1);
         read(i, 1);
-        mul(0);
+        if constexpr (flush) sum[FL / NI][FL % NI] += acc[FL / NI][FL % NI];
+        mul(0, flush ? FL : NB - 1, flush);
         // interleave: one load or read between the products
 #pragma unroll
-        for (int s = 0; s < MI * NI; s++) {
+        for (int s = 0; s < NB; s++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
@@ -255,13 +277,23 @@ void prompt_gemm_kernel(const PromptArgs a) {
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         read(i + 1, 0);
-        mul(1);
+        mul(1, NB - 1, false);
 #pragma unroll
-        for (int s = 0; s < MI * NI; s++) {
+        for (int s = 0; s < NB; s++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-    }
+    };
+    int i = 0;
+    for (; i + kChain <= nk; i += kChain)
+        for_each_stage(std::make_integer_sequence<int, kChain>{}, [&](auto s) __attribute__((always_inline)) {
+            stage(i + decltype(s)::value, s);
+        });
+    for (; i < nk; i++) stage(i, std::integral_constant<int, -1>{});
+#pragma unroll
+    for (int x = 0; x < MI; x++)
+#pragma unroll
+        for (int y = 0; y < NI; y++) sum[x][y] += acc[x][y];
     __builtin_amdgcn_s_waitcnt(0x0F70);   // no load into LDS outlives the workgroup
     float* y = a.y + blockIdx.y * a.sy;
     // C layout: element e of lane l is input row 8 (e / 4) + 4 (l / 32) + e % 4,
@@ -277,32 +309,29 @@ void prompt_gemm_kernel(const PromptArgs a) {
             for (int j = 0; j < NI; j++) {
                 const int col = n0 + wn * (BN / WN) + j * 32 + lr;
                 if (col >= a.n) continue;
-                yr[col] = a.accumulate ? yr[col] + acc[i][j][e] : acc[i][j][e];
+                yr[col] = a.accumulate ? yr[col] + sum[i][j][e] : sum[i][j][e];
             }
         }
 }
 
-// Which tile and how many column slices: estimated time of each pair, from
-// what the kernels measured on MI355X (us per 32-column stage).  `one`: a lone
-// tile's stage; `full`: a stage of 256 tiles running at once, where the chip's
-// throughput bounds it; a partly filled round lies between.  Column slices
-// (partial sums added by split_sum in a fixed order) fill the chip when there
-// are few tiles; they cost their traffic, which mostly stays in the last-level
-// cache.  The constants are a fit to 77 shapes (65..6000 inputs of seven
-// projections) x 20 pairs: what the model picks is within 1 % of the best
-// pair on average and 7 % at most.  256 x 192 is there for the counts that
-// leave 256 x 256 a nearly empty last round or too few tiles (whole call, us,
-// without it and with it: 4096 x 2560 x 9216 269 -> 239, 1024 x 18432 x 2560
-// 151 -> 134, 2048 x 2560 x 9216 150 -> 141, 300 x 18432 x 2560 85 -> 77).
+// Which tile and how many column slices: estimated time of each pair.  `one`:
+// a lone tile's 32-column stage; `full`: a stage of 256 tiles running at once,
+// where the chip's throughput bounds it; a partly filled round lies between.
+// Column slices (partial sums added by split_sum in a fixed order) fill the
+// chip when there are few tiles; they cost their traffic, which mostly stays in
+// the last-level cache.  The constants are a fit of the order of the pairs'
+// whole-call times (their unit is near a microsecond) over 77 shapes (65..4096
+// inputs of seven projections) x 16 pairs: what the model picks is within 0.3 %
+// of the best pair on average and 4 % at most.  256 x 192 is the largest tile
+// whose accumulators and sums fit a wave's 256 registers.
 struct Tile {
     int bm, bn;
     float one, full;
 };
-constexpr Tile kTiles[] = {{256, 256, 0.642f, 0.837f},
-                           {256, 192, 0.513f, 0.678f},
-                           {256, 128, 0.409f, 0.519f},
-                           {128, 128, 0.295f, 0.358f},
-                           {64, 128, 0.207f, 0.244f}};
+constexpr Tile kTiles[] = {{256, 192, 0.774f, 0.898f},
+                           {256, 128, 0.476f, 0.711f},
+                           {128, 128, 0.447f, 0.454f},
+                           {64, 128, 0.249f, 0.285f}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kSplits[] = {1, 2, 4, 8};
 
@@ -323,7 +352,7 @@ Plan make_plan(int m, int n, int nk, bool may_split, int cus) {
             const long rounds = units / cus, rem = units % cus;
             const float stage = (float)rounds * k.full + (rem ? std::max(k.one, k.full * (float)rem / (float)cus) : 0.f);
             float us = stage * (float)nk / (float)s;
-            if (s > 1) us += 1.6f + (float)(2 * s + 1) * (float)m * (float)n * 4.f / 5.9e6f;
+            if (s > 1) us += 2.63f + (float)(2 * s + 1) * (float)m * (float)n * 4.f / 5.37e6f;
             if (p.tile < 0 || us < best) best = us, p.tile = t, p.splits = s;
         }
     const Tile& k = kTiles[p.tile];
@@ -422,10 +451,9 @@ int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const floa
                          sum ? 0 : accumulate};
             int rc;
             switch (p.tile) {
-                case 0: rc = gemm_launch<256, 256, 2, 4>(a, st); break;
-                case 1: rc = gemm_launch<256, 192, 4, 2>(a, st); break;
-                case 2: rc = gemm_launch<256, 128, 4, 2>(a, st); break;
-                case 3: rc = gemm_launch<128, 128, 2, 2>(a, st); break;
+                case 0: rc = gemm_launch<256, 192, 4, 2>(a, st); break;
+                case 1: rc = gemm_launch<256, 128, 4, 2>(a, st); break;
+                case 2: rc = gemm_launch<128, 128, 2, 2>(a, st); break;
                 default: rc = gemm_launch<64, 128, 1, 4>(a, st); break;
             }
             if (rc == ANELM_OK && sum) rc = lut6_split_sum(yb, parts, (long)p.m * p.n, p.splits, accumulate, st);

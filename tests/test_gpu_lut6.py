@@ -349,3 +349,23 @@ def test_prompt_gemm(anelm, dev, batch, out_dim, in_dim, shift):
     assert bool(((acc.double() - want).abs() <= (in_dim + 2) * 2.0 ** -24 * mag).all())
     # repeated call: same bits
     assert torch.equal(got, anelm.ops.lut6_gemm(w, lut_d, xd, out_dim, in_dim))
+
+
+@pytest.mark.parametrize("batch,out_dim,in_dim", [(100, 2560, 2560), (300, 18432, 2560), (2048, 2560, 9216),
+                                                  (1500, 1024, 3584)])
+def test_prompt_gemm_error(anelm, dev, batch, out_dim, in_dim):
+    """A prompt's product is no less exact than the same inputs in passes of 32
+    (whose waves sum 256 columns each): both round about as often at about the
+    same magnitudes, so their relative errors differ by less than a quarter."""
+    packed, lut, idx = lut6_matrix(730 + batch, out_dim, in_dim)
+    w, lut_d = to_dev(packed, dev), to_dev(lut, dev)
+    x = torch.from_numpy(np.random.default_rng(731 + batch).standard_normal((batch, in_dim)).astype(np.float32)).to(dev)
+    want = x.half().double() @ torch.from_numpy(lut6_dense(idx, lut)).to(dev).double().t()
+
+    def err(y):
+        return float((y.double() - want).norm() / want.norm())
+
+    whole = err(anelm.ops.lut6_gemm(w, lut_d, x, out_dim, in_dim))
+    passes = err(torch.cat([anelm.ops.lut6_gemm(w, lut_d, x[b:b + 32].contiguous(), out_dim, in_dim)
+                            for b in range(0, batch, 32)]))
+    assert whole <= 1.25 * passes, (whole, passes)
