@@ -83,8 +83,9 @@ void* workspace(size_t bytes, hipStream_t stream);
 void* workspace2(size_t bytes, hipStream_t stream);
 // The LUT6 prompt product's own buffer: a long prompt takes hundreds of MB, and
 // growing one of the others would free what a graph captured from a smaller
-// call still points to.  (That product is never captured.)
-void* prompt_workspace(size_t bytes, hipStream_t stream);
+// call still points to.  (That product is never captured.)  ANELM_ENOMEM: the
+// memory is not there; ANELM_EHIP: another failure, as of an earlier launch.
+int prompt_workspace(void** p, size_t bytes, hipStream_t stream);
 
 // Workgroup barrier for LDS exchange only: this wave's LDS operations
 // complete, then s_barrier.  __syncthreads() also carries a release fence that

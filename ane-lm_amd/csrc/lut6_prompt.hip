@@ -382,9 +382,10 @@ int gemm_launch(const PromptArgs& a, hipStream_t st) {
     return ANELM_OK;
 }
 
-// Bounds of one preparation: 8192 inputs and 256 MiB of decoded weights at a
-// time, so the workspace stays bounded whatever the shape (both are far past
-// where the chip is full).
+// Bounds of one preparation: 8192 inputs (176 MiB at the longest rows, 11264)
+// and 256 MiB of decoded weights at a time, both far past where the chip is
+// full, rounded up to whole tiles.  Partial sums of column slices come on top:
+// slices are chosen only where the tiles are fewer than the compute units.
 constexpr int kMaxRows = 8192;
 constexpr size_t kMaxW16 = (size_t)256 << 20;
 
@@ -426,11 +427,10 @@ int lut6_prompt_gemm(float* y, const uint8_t* w, const uint16_t* lut, const floa
     size_t bytes = 0;
     for (int b0 = 0; b0 < batch; b0 += kMaxRows)
         for (int n0 = 0; n0 < out_dim; n0 += n_max) bytes = std::max(bytes, plan(b0, n0).bytes);
-    char* ws = static_cast<char*>(prompt_workspace(bytes, st));
-    if (!ws) {
-        (void)hipGetLastError();   // a failed allocation is no launch error of the path taken instead
-        return ANELM_ENOMEM;
-    }
+    void* buf = nullptr;
+    const int got = prompt_workspace(&buf, bytes, st);
+    if (got) return got;
+    char* ws = static_cast<char*>(buf);
     for (int b0 = 0; b0 < batch; b0 += kMaxRows)
         for (int n0 = 0; n0 < out_dim; n0 += n_max) {
             const Plan p = plan(b0, n0);

@@ -77,46 +77,52 @@ StreamState* stream_state(hipStream_t stream) {
 
 // Grows one buffer of a stream's state.  Only work queued on that stream can
 // still use the old buffer, so syncing that stream before the free suffices.
-static void* grow(StreamState* s, void*& buf, size_t& have, size_t bytes) {
+// ANELM_ENOMEM: the memory is not there, or another stream's capture forbids
+// allocating (no error left pending); ANELM_EHIP: the sync, the free or the
+// allocation failed for another reason, such as an earlier launch's.
+static int grow(StreamState* s, void*& buf, size_t& have, size_t bytes, void** out) {
     std::lock_guard<std::mutex> lk(s->mu);
-    if (bytes <= have) return buf;
+    *out = buf;
+    if (bytes <= have) return ANELM_OK;
+    *out = nullptr;
     size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
     want = (want + 0xffff) & ~size_t(0xffff);
     if (buf) {
-        hipError_t e = hipStreamSynchronize(s->stream);
-        if (e != hipSuccess) { hip_fail(e, "hipStreamSynchronize"); return nullptr; }
-        e = hipFree(buf);
-        if (e != hipSuccess) { hip_fail(e, "hipFree(workspace)"); return nullptr; }
+        ANELM_HIP(hipStreamSynchronize(s->stream));
+        ANELM_HIP(hipFree(buf));
         buf = nullptr;
         have = 0;
     }
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) {
-        set_error(ANELM_ENOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
-        return nullptr;
+    if (e == hipErrorOutOfMemory || e == hipErrorStreamCaptureUnsupported) {
+        (void)hipGetLastError();
+        return set_error(ANELM_ENOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
     }
-    buf = p;
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc(workspace)");
+    *out = buf = p;
     have = want;
-    return p;
+    return ANELM_OK;
 }
 
 void* workspace(size_t bytes, hipStream_t stream) {
     StreamState* s = stream_state(stream);
-    if (!s) return nullptr;
-    return grow(s, s->ws, s->ws_bytes, bytes);
+    void* p = nullptr;
+    if (s) (void)grow(s, s->ws, s->ws_bytes, bytes, &p);
+    return p;
 }
 
 void* workspace2(size_t bytes, hipStream_t stream) {
     StreamState* s = stream_state(stream);
-    if (!s) return nullptr;
-    return grow(s, s->ws2, s->ws2_bytes, bytes);
+    void* p = nullptr;
+    if (s) (void)grow(s, s->ws2, s->ws2_bytes, bytes, &p);
+    return p;
 }
 
-void* prompt_workspace(size_t bytes, hipStream_t stream) {
+int prompt_workspace(void** p, size_t bytes, hipStream_t stream) {
+    *p = nullptr;
     StreamState* s = stream_state(stream);
-    if (!s) return nullptr;
-    return grow(s, s->wsp, s->wsp_bytes, bytes);
+    return s ? grow(s, s->wsp, s->wsp_bytes, bytes, p) : ANELM_EHIP;
 }
 
 uint32_t* counters(size_t n, CounterUser user, hipStream_t stream) {

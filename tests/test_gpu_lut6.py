@@ -369,3 +369,32 @@ def test_prompt_gemm_error(anelm, dev, batch, out_dim, in_dim):
     passes = err(torch.cat([anelm.ops.lut6_gemm(w, lut_d, x[b:b + 32].contiguous(), out_dim, in_dim)
                             for b in range(0, batch, 32)]))
     assert whole <= 1.25 * passes, (whole, passes)
+
+
+def test_prompt_gemm_without_workspace(anelm, dev):
+    """A prompt whose operand buffer (450 MB here) does not fit the memory left
+    takes the passes of 32 instead, and says nothing of the failed allocation
+    afterwards; with the memory back it takes its own path again."""
+    batch, out_dim, in_dim = 8192, 11776, 11264
+    g = torch.Generator(device=dev).manual_seed(740)
+    w = torch.randint(0, 256, (out_dim, in_dim * 3 // 4), generator=g, device=dev, dtype=torch.uint8)
+    lut = (0.02 * torch.randn(out_dim // 32, 64, generator=g, device=dev)).half()
+    x = torch.randn(batch, in_dim, generator=g, device=dev)
+    y, z = torch.empty(batch, out_dim, device=dev), torch.empty(batch, out_dim, device=dev)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    rest = []   # all but some 300 MB (the first block leaves more than it was asked to)
+    while torch.cuda.mem_get_info()[0] > 380 << 20 and len(rest) < 8:
+        rest.append(torch.empty(torch.cuda.mem_get_info()[0] - (300 << 20), dtype=torch.uint8, device=dev))
+    assert torch.cuda.mem_get_info()[0] <= 380 << 20
+    with torch.cuda.stream(s):
+        anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim, out=y)
+        s.synchronize()
+        del rest
+        torch.cuda.empty_cache()
+        anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim, out=z)
+        s.synchronize()
+    anelm.call("anelm_stream_release", ctypes.c_void_p(s.cuda_stream))
+    assert not torch.equal(y, z)   # (two paths, two orders of summation)
+    assert float((y - z).norm() / z.norm()) <= 1e-6
