@@ -398,3 +398,54 @@ def test_prompt_gemm_without_workspace(anelm, dev):
     anelm.call("anelm_stream_release", ctypes.c_void_p(s.cuda_stream))
     assert not torch.equal(y, z)   # (two paths, two orders of summation)
     assert float((y - z).norm() / z.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("batch,out_dim,in_dim", [
+    (8200, 64, 80),      # past 8192 inputs: two preparations
+    (70, 52512, 2560),   # past 256 MiB of decoded weights: two column ranges of the output, the second ragged
+])
+def test_prompt_gemm_in_pieces(anelm, dev, batch, out_dim, in_dim):
+    """Calls past what one preparation takes, also accumulating; each output
+    within its roundings of the sum of magnitudes, as in test_prompt_gemm."""
+    packed, lut, idx = lut6_matrix(750 + batch, out_dim, in_dim)
+    g = torch.Generator(device=dev).manual_seed(751)
+    x, y0 = torch.randn(batch, in_dim, generator=g, device=dev), torch.randn(batch, out_dim, generator=g, device=dev)
+    w, lut_d = to_dev(packed, dev), to_dev(lut, dev)
+    got = anelm.ops.lut6_gemm(w, lut_d, x, out_dim, in_dim)
+    acc = anelm.ops.lut6_gemm(w, lut_d, x, out_dim, in_dim, out=y0.clone(), accumulate=True)
+    wd = torch.from_numpy(lut6_dense(idx, lut)).to(dev)
+    for r in range(0, out_dim, 16384):
+        wr = wd[r:r + 16384].double()
+        want, mag = x.half().double() @ wr.t(), x.half().double().abs() @ wr.t().abs()
+        n = slice(r, r + wr.shape[0])
+        assert bool(((got[:, n].double() - want).abs() <= (in_dim + 1) * 2.0 ** -24 * mag).all())
+        want, mag = want + y0[:, n], mag + y0[:, n].abs()
+        assert bool(((acc[:, n].double() - want).abs() <= (in_dim + 2) * 2.0 ** -24 * mag).all())
+
+
+def test_prompt_gemm_captured(anelm, dev):
+    """Under capture a prompt takes the passes of 32: every replay gives their
+    bits, whatever prompts run on the stream in between."""
+    out_dim, in_dim, batch = 1024, 1024, 100
+    packed, lut, _ = lut6_matrix(760, out_dim, in_dim)
+    w, lut = to_dev(packed, dev), to_dev(lut, dev)
+    g = torch.Generator(device=dev).manual_seed(761)
+    x, y = torch.randn(batch, in_dim, generator=g, device=dev), torch.empty(batch, out_dim, device=dev)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        want = torch.cat([anelm.ops.lut6_gemm(w, lut, x[b:b + 32].contiguous(), out_dim, in_dim)
+                          for b in range(0, batch, 32)])
+        eager = anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim).clone()
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim, out=y)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            s.synchronize()
+            assert torch.equal(y, want)
+            assert torch.equal(anelm.ops.lut6_gemm(w, lut, x, out_dim, in_dim), eager)
+    del graph
+    assert float((eager - want).norm() / want.norm()) <= 1e-6
+    anelm.call("anelm_stream_release", ctypes.c_void_p(s.cuda_stream))
