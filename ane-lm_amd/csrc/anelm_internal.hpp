@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/anelm.h"
+#include "device_once.hpp"
 
 namespace anelm {
 
@@ -70,6 +71,10 @@ struct Device {
 // Current device's state (lazily initialised).  nullptr on failure with the
 // error recorded.
 Device* device();
+
+// Lets `kernel` take `bytes` of dynamic LDS on the current device, once per
+// device (`once` belongs to the kernel).
+int allow_lds(DeviceOnce& once, const void* kernel, int bytes);
 
 // State of `stream` on the current device (created on first use).
 StreamState* stream_state(hipStream_t stream);

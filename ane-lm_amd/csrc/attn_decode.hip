@@ -14,7 +14,6 @@
 #include <type_traits>
 
 #include <algorithm>
-#include <atomic>
 #include <math.h>
 #include <vector>
 
@@ -1642,12 +1641,9 @@ bool ring_aligned(const DecodeParams& p) {
 }
 
 int launch_ring_mfma(const DecodeParams& p, dim3 grid, hipStream_t st) {
-    static std::atomic<bool> attr{false};
-    if (!attr.load(std::memory_order_acquire)) {
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_mfma_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kRW * kRVB));
-        attr.store(true, std::memory_order_release);
-    }
+    static DeviceOnce lds;
+    const int rc = allow_lds(lds, reinterpret_cast<const void*>(&attn_ring_mfma_kernel), 2 * kRW * kRVB);
+    if (rc) return rc;
     // a second set of V buffers where a wave walks several blocks
     const int bufs = std::min(p.kps, p.len) > kRW * kRBlk ? 2 : 1;
     hipLaunchKernelGGL(attn_ring_mfma_kernel, grid, dim3(kRNT), bufs * kRW * kRVB, st,

@@ -18,7 +18,6 @@
 
 #include <math.h>
 
-#include <atomic>
 #include <type_traits>
 
 namespace anelm {
@@ -714,15 +713,10 @@ int launch_split(const SplitArgs& a, bool out16, hipStream_t st) {
                                  {prefill_split_kernel<KP, true, false>, prefill_split_kernel<KP, true, true>}};
     static const K comb[2][2] = {{prefill_split_combine<KP, false, false>, prefill_split_combine<KP, false, true>},
                                  {prefill_split_combine<KP, true, false>, prefill_split_combine<KP, true, true>}};
-    static std::atomic<bool> attr_set{false};
-    if (!attr_set.load(std::memory_order_acquire)) {
-        for (int o = 0; o < 2; o++)
-            for (int g = 0; g < 2; g++)
-                ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern[o][g]),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, split_lds<KP>()));
-        attr_set.store(true, std::memory_order_release);
-    }
+    static DeviceOnce lds[2][2];
     const int o = out16 ? 1 : 0, g = a.gate != nullptr ? 1 : 0, bpk = a.ngrp * a.parts;
+    const int rc = allow_lds(lds[o][g], reinterpret_cast<const void*>(kern[o][g]), split_lds<KP>());
+    if (rc) return rc;
     const int spx = 8 % a.Hkv == 0 ? 8 / a.Hkv : 1;
     const dim3 grid(8 % a.Hkv == 0 ? (bpk + spx - 1) / spx * 8 : bpk * a.Hkv);
     hipLaunchKernelGGL(kern[o][g], grid, dim3(kGNT), split_lds<KP>(), st, a);

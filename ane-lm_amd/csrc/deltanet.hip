@@ -14,7 +14,6 @@
 
 #include <math.h>
 
-#include <atomic>
 
 namespace anelm {
 namespace {
@@ -1065,20 +1064,15 @@ int chunk_prefill(ChunkArgs p, ScanArgs s, bool conv, hipStream_t st) {
     using K = void (*)(const ChunkArgs);
     static const K kern[2][2] = {{dn_chunk_prep_kernel<false, false>, dn_chunk_prep_kernel<false, true>},
                                  {dn_chunk_prep_kernel<true, false>, dn_chunk_prep_kernel<true, true>}};
-    static std::atomic<bool> attr{false};
-    if (!attr.load(std::memory_order_acquire)) {
-        for (int t = 0; t < 2; t++)
-            for (int c = 0; c < 2; c++)
-                ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern[t][c]),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kPmLds));
-        attr.store(true, std::memory_order_release);
-    }
+    static DeviceOnce lds[2][2];
+    const int t = p.flags & ANELM_DN_ORDER_TRANSFORMERS ? 1 : 0, c = conv ? 1 : 0;
+    const int rc = allow_lds(lds[t][c], reinterpret_cast<const void*>(kern[t][c]), kPmLds);
+    if (rc) return rc;
     // a workgroup takes all value heads of its key head where that fills the
     // chip (two workgroups per CU), else one (the Gram tiles formed again)
     const bool each = G > 1 && (long)n_chunks * p.Hk < 2L * dev->num_cus;
     p.per_wg = each ? 1 : G;
-    hipLaunchKernelGGL(kern[p.flags & ANELM_DN_ORDER_TRANSFORMERS ? 1 : 0][conv ? 1 : 0],
-                       dim3(n_chunks, p.Hk, each ? G : 1), dim3(kPmNT), kPmLds, st, p);
+    hipLaunchKernelGGL(kern[t][c], dim3(n_chunks, p.Hk, each ? G : 1), dim3(kPmNT), kPmLds, st, p);
     ANELM_LAUNCHED("dn_chunk_prep_kernel");
     s.vrec = p.vrec;
     s.krec = p.krec;

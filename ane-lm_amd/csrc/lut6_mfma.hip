@@ -467,13 +467,10 @@ int lut6_gemm_launch(float* y, const uint8_t* w, long ldw, const uint16_t* lut, 
     const K kp = np == 2 ? k2[acc][waves] : k1[acc][waves];
     if (!kp) return set_error(ANELM_EINVAL, "lut6_gemm: no kernel for %d waves (np %d)", waves, np);
     // the attribute covers the staged size (the larger of the two per kernel)
-    static bool attr_set[2][2][16] = {};
-    if (!attr_set[acc][np - 1][waves]) {
-        const int full = (int)((size_t)kRedOff + red_bytes + stage_bytes);
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kp), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      full));
-        attr_set[acc][np - 1][waves] = true;
-    }
+    static DeviceOnce once[2][2][16];
+    const int rc = allow_lds(once[acc][np - 1][waves], reinterpret_cast<const void*>(kp),
+                             (int)((size_t)kRedOff + red_bytes + stage_bytes));
+    if (rc) return rc;
     hipLaunchKernelGGL(kp, dim3(grid, nsplit), dim3(waves * 64), lds, st, a);
     ANELM_LAUNCHED("lut6_gemm_kernel");
     return ANELM_OK;

@@ -23,7 +23,6 @@
 #include "anelm_internal.hpp"
 
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 #include <utility>
 
@@ -371,12 +370,9 @@ int gemm_launch(const PromptArgs& a, hipStream_t st) {
     ANELM_REQUIRE(a.mp % BM == 0 && a.np % BN == 0 && a.mp >= a.m && a.np >= a.n && a.nk >= a.ksplit,
                   "prompt_gemm: rows %d of %d, %d of %d, %d stages in %d", a.m, a.mp, a.n, a.np, a.nk, a.ksplit);
     auto kern = prompt_gemm_kernel<BM, BN, WM, WN, NS>;
-    static std::atomic<bool> attr_set{false};
-    if (!attr_set.load(std::memory_order_relaxed)) {
-        ANELM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      kLds));
-        attr_set.store(true, std::memory_order_relaxed);
-    }
+    static DeviceOnce lds;
+    const int rc = allow_lds(lds, reinterpret_cast<const void*>(kern), kLds);
+    if (rc) return rc;
     hipLaunchKernelGGL(kern, dim3((a.mp / BM) * (a.np / BN), a.ksplit), dim3(WM * WN * 64), kLds, st, a);
     ANELM_LAUNCHED("prompt_gemm_kernel");
     return ANELM_OK;

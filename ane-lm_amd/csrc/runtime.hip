@@ -44,6 +44,15 @@ Device* device() {
     return d;
 }
 
+int allow_lds(DeviceOnce& once, const void* kernel, int bytes) {
+    Device* d = device();
+    if (!d) return ANELM_EHIP;
+    return once.run(d->id, [&]() -> int {
+        ANELM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+        return ANELM_OK;
+    });
+}
+
 __global__ void zero_u32_kernel(uint32_t* p, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         p[i] = 0u;

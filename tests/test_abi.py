@@ -40,6 +40,34 @@ def test_library_exports_every_declared_symbol(anelm):
     assert set(declared_symbols()) == bound
 
 
+def test_device_once(tmp_path):
+    """A kernel's LDS limit holds for one device, so it is set on every device's
+    first launch, again after a failure, and not afterwards."""
+    src = tmp_path / "once.cpp"
+    src.write_text(
+        '#include "device_once.hpp"\n'
+        "#include <cstdio>\n"
+        "int main() {\n"
+        "  static anelm::DeviceOnce once;\n"
+        "  int calls = 0;\n"
+        "  auto set = [&] { calls++; return calls == 2 ? 7 : 0; };   // the second call fails\n"
+        "  const int ids[] = {0, 0, 1, 1, 63, 0, 1, 63};\n"
+        "  for (int id : ids) {\n"
+        "    const int rc = once.run(id, set);\n"
+        "    std::printf(\"%d/%d \", rc, calls);\n"
+        "  }\n"
+        "}\n")
+    exe = str(tmp_path / "once")
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "ane-lm_amd", "csrc"), str(src), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split()
+    assert out == ["0/1", "0/1", "7/2", "0/3", "0/4", "0/4", "0/4", "0/4"]
+    # and no launch keeps a flag of its own for it
+    csrc = os.path.join(ROOT, "ane-lm_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        text = open(os.path.join(csrc, name)).read()
+        assert not re.search(r"static (std::atomic<bool>|bool) \w*attr", text), name
+
+
 def test_cpp_compat_header_compiles_against_library(tmp_path, anelm):
     """A C++ caller written against core/cpu_ops.h's names builds and links
     with the drop-in header (compile + link only, nothing runs)."""
