@@ -16,7 +16,7 @@
 //   and the prompt's keys that survive are written to their slots at the end.
 // Gated DeltaNet (qwen3_5.cpp:849-908 per token), conv width 4: the chunked
 // prefill reads the projection rows itself (deltanet.hip), then rmsnorm_gated
-// in place.  Other widths and unaligned rows:
+// in place.  Other widths, unaligned rows and outputs over the rows:
 //   1. the causal conv1d over [conv ring | prompt] + SiLU per channel
 //      (cpu_ops.cpp:89-129, :6-13), split into q / k / v, with z, a, b
 //      gathered alongside; the ring keeps the prompt's last inputs;
@@ -435,9 +435,12 @@ extern "C" int anelm_deltanet_prefill_from_proj(float* y, float* state, float* c
     // conv width 4 on aligned rows (the models'): the conv runs inside the
     // chunk preparation and z is read where it lies, so nothing but y is
     // written between (4096 tokens of 32 heads: the separate passes below took
-    // 77 us for the conv and the copies, and their arrays 330 MB)
+    // 77 us for the conv and the copies, and their arrays 330 MB).  y over the
+    // rows takes the passes: they have read all of them before the first of y
+    const uintptr_t y0 = reinterpret_cast<uintptr_t>(y), p0 = reinterpret_cast<uintptr_t>(proj);
+    const bool apart = y0 + (size_t)S * nz * 4 <= p0 || p0 + (size_t)S * pd * 4 <= y0;
     const bool y8 = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(norm_w)) & 7) == 0;
-    if (deltanet_prefill_proj_fits(proj, conv_w, pd, conv_kernel) && (!gated || y8)) {
+    if (apart && deltanet_prefill_proj_fits(proj, conv_w, pd, conv_kernel) && (!gated || y8)) {
         int rc = deltanet_prefill_proj(y, state, conv_state, *conv_pos, proj, conv_w, A, dt_bias, S, Hk, Hv, pd,
                                        flags & 3, st);
         if (rc == ANELM_OK && gated) rc = rmsnorm_gated_heads(y, proj + C, pd, norm_w, S, Hv, st);

@@ -299,3 +299,29 @@ def test_deltanet_prefill_from_proj_cuts(anelm, orc, dev, S, Hk, Hv, flags, pos0
     assert pos.value == p
     assert_close(to_host(Sd), St, what="state")
     assert np.array_equal(to_host(csd), cs), "conv ring"
+
+
+@pytest.mark.parametrize("flags,off", [(5, 0), (1, 0), (5, 3 * 128)])
+def test_deltanet_prefill_from_proj_over_its_rows(anelm, dev, flags, off):
+    """The output may lie over the projection rows: they are read whole first
+    (against the call with an output of its own, whose passes round otherwise)."""
+    S, Hk, Hv, K, d = 200, 2, 4, 4, 128
+    rng = np.random.default_rng(1870 + flags + off)
+    qkv, pd = 2 * Hk * d + Hv * d, 2 * Hk * d + 2 * Hv * d + 2 * Hv
+    t = {n: to_dev(x.astype(np.float32), dev) for n, x in dict(
+        St=0.1 * rng.standard_normal((Hv, d, d)), cs=0.5 * rng.standard_normal((qkv, K - 1)),
+        w=0.5 * rng.standard_normal((qkv, K)), A=np.exp(rng.uniform(0, np.log(16), Hv)), dtb=rng.standard_normal(Hv),
+        nw=1 + 0.1 * rng.standard_normal(d), proj=rng.standard_normal((S, pd))).items()}
+
+    def run(inside):
+        St, cs, proj = t["St"].clone(), t["cs"].clone(), t["proj"].clone()
+        y = proj.view(-1)[off:off + S * Hv * d] if inside else torch.empty(S * Hv * d, device=dev)
+        pos, p = ctypes.c_int(1), ctypes.c_void_p
+        anelm.call("anelm_deltanet_prefill_from_proj", p(y.data_ptr()), p(St.data_ptr()), p(cs.data_ptr()),
+                   ctypes.byref(pos), p(proj.data_ptr()), p(t["w"].data_ptr()), p(t["A"].data_ptr()),
+                   p(t["dtb"].data_ptr()), p(t["nw"].data_ptr()), S, Hk, Hv, d, d, K, flags,
+                   p(torch.cuda.current_stream().cuda_stream))
+        return to_host(y.clone()), to_host(St), to_host(cs)
+
+    for got, want, what in zip(run(True), run(False), ("y", "state", "conv ring")):
+        assert_close(got, want, rel=1e-5, max_abs=1e-3, what=what)
