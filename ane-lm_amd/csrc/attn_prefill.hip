@@ -199,10 +199,10 @@ __global__ __launch_bounds__(HB * RB * 64) void prefill_kernel(void* out, const 
 //   16-lane group reads with ds_read_b64_tr_b16 (4 keys x 16 dims, delivered
 //   transposed: lane n gets dim n of the 4 keys) fall on distinct banks.  That
 //   transposing read builds the V^T operand of O^T += V^T P^T from the V rows
-//   as stored.  KP 2: two steps of tiles in LDS, the next step's loads behind
-//   the one barrier of a step.  KP 4: one step in LDS; the next step's K tiles
-//   are requested once the scores are formed, its V tiles once the outputs
-//   are (four barriers per step).
+//   as stored.  KP 1 and 2: four and two steps of tiles in LDS, the loads of
+//   the step three and one ahead behind the one barrier of a step.  KP 4: one
+//   step in LDS; the next step's K tiles are requested once the scores are
+//   formed, its V tiles once the outputs are (four barriers per step).
 // * Scores S^T = K Q^T (v_mfma_f32_32x32x16_f16).  The A-operand lane i reads
 //   key row pi(i) (bits 2 and 3 of i swapped): lane (r, h) of the accumulator
 //   then holds the scores of column r for keys 8h..8h+7 and 16+8h..16+8h+7,
@@ -416,10 +416,11 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
         __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.rg.v), 0, a.rg.cap * a.Hkv * 512, 0x00020000);
     constexpr int PERW = 16 / CG;   // chunks of its part's K (and V) tile that a wave loads
     char* const mine = lds + kp * kGTile;
-    constexpr int kStage = KP * kGTile;   // KP 2: step s in stage s % 2
-    auto issue = [&](int s, auto is_v) __attribute__((always_inline)) {
+    constexpr int NST = 4 / KP, kStage = KP * kGTile;   // step s in stage s % NST
+    // the K or V part of step s's tiles, to the stage of step `to`
+    auto issue = [&](int s, auto is_v, int to) __attribute__((always_inline)) {
         constexpr bool values = decltype(is_v)::value;
-        char* base = mine + (KP == 2 ? (s & 1) * kStage : 0) + (values ? kGKBytes : 0);
+        char* base = mine + (to & (NST - 1)) * kStage + (values ? kGKBytes : 0);
         const int j0 = (s * KP + kp) * kGKeys, at = j0 + a.rg.start, row = at - (at >= a.rg.cap ? a.rg.cap : 0);
         int ln = threadIdx.x & 63;
         asm volatile("" : "+v"(ln));   // lane offsets are recomputed here, not held across the loop
@@ -446,8 +447,16 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
     };
     constexpr std::integral_constant<bool, false> K{};
     constexpr std::integral_constant<bool, true> V{};
-    issue(s0, K);
-    issue(s0, V);
+    // (KP 1: past the last step its tiles again, so that as many loads are in flight at every wait)
+    auto request = [&](int s) __attribute__((always_inline)) {
+        issue(KP == 1 ? min(s, s1 - 1) : s, K, s);
+        issue(KP == 1 ? min(s, s1 - 1) : s, V, s);
+    };
+    request(s0);
+    if constexpr (KP == 1) {
+        request(s0 + 1);
+        request(s0 + 2);
+    }
     half8 qf[KS];
     {
         const int lane = threadIdx.x & 63, tok = min(tok0 + ((lane & 31) >> 2), a.S - 1);
@@ -461,20 +470,18 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
     float m = kNoKey, l = 0.f;
     const float sl2 = (1.0f / 16.0f) * 1.4426950408889634f;   // 1/sqrt(256) * log2(e)
     const int first = a.qoff + tok0, last = a.qoff + min(tok0 + 7, a.S - 1);   // last keys of the wave's tokens
-    if constexpr (KP == 2) {
+    if constexpr (KP <= 2) {
         for (int s = s0; s < s1; s++) {
-            __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's loads of step s have landed
-            lds_barrier();                      // every wave's; the other stage is free
-            if (s + 1 < s1) {
-                issue(s + 1, K);
-                issue(s + 1, V);
-            }
+            // this wave's loads of step s have landed (KP 1: those of the next two may be in flight)
+            __builtin_amdgcn_s_waitcnt(0x0F70 | (KP == 1 ? 4 * PERW : 0));
+            lds_barrier();                      // every wave's; the stage of step s - 1 is free
+            if (KP == 1 || s + 1 < s1) request(s + NST - 1);
             const int j0 = (s * KP + kp) * kGKeys;
             int ln = threadIdx.x & 63;
             asm volatile("" : "+v"(ln));
             // (wave-uniform) a tile past the wave's last token has nothing for it
             if (tok0 < a.S && j0 <= last) {
-                const char* base = mine + (s & 1) * kStage;
+                const char* base = mine + (s & (NST - 1)) * kStage;
                 half8 pf[2];
                 tile_softmax(tile_scores(base, ln, qf), pf, o, m, l, sl2, ln, j0, j0 + 31 > first,
                              a.qoff + tok0 + ((ln & 31) >> 2));
@@ -495,7 +502,7 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
             half8 pf[2] = {};
             if (live) sc = tile_scores(mine, ln, qf);
             lds_barrier();   // K is free
-            if (next) issue(s + 1, K);
+            if (next) issue(s + 1, K, s + 1);
             if (live)
                 tile_softmax(sc, pf, o, m, l, sl2, ln, j0, j0 + 31 > first, a.qoff + tok0 + ((ln & 31) >> 2));
             if (next) __builtin_amdgcn_s_waitcnt(kHalf);   // V of step s (K of step s + 1 behind it)
@@ -503,7 +510,7 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
             lds_barrier();
             if (live) tile_values(mine, ln, pf, o);
             lds_barrier();   // V is free
-            if (next) issue(s + 1, V);
+            if (next) issue(s + 1, V, s + 1);
         }
     }
     // ---- merge the KP key parts of each column group: every wave scales its O
@@ -513,6 +520,7 @@ __global__ __launch_bounds__(kGNT) void prefill_split_kernel(const SplitArgs a) 
     int ln = threadIdx.x & 63;
     asm volatile("" : "+v"(ln));
     float* const ms = reinterpret_cast<float*>(lds + 4 * kGTile);
+    if constexpr (KP == 1) __builtin_amdgcn_s_waitcnt(0x0F70);   // the repeated last tiles
     __syncthreads();   // the tiles are no longer read
     ms[w * 64 + ln] = m;
     ms[512 + w * 64 + ln] = l;
@@ -664,7 +672,7 @@ __global__ __launch_bounds__(kGNT) void prefill_split_combine(const SplitArgs a)
     split_store<OUT16, GATE>(a.out, tok, h, a.Hq, d, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv), g);
 }
 
-// How a prompt is cut: the least estimated time over both KP and 1 .. 16 parts
+// How a prompt is cut: the least estimated time over KP 2 and 4 and 1 .. 16 parts
 // of the longest group.  From sweeps of both (us): a step takes 1.9 (KP 2) or
 // 2.8 (KP 4, half the tokens over twice the keys), a workgroup 9 besides; more
 // workgroups than compute units run one after another (the longest first, so
@@ -673,11 +681,20 @@ __global__ __launch_bounds__(kGNT) void prefill_split_combine(const SplitArgs a)
 // tokens behind 1500 keys 2 kv heads, KP 2: 5 parts 38 (38), 2 parts 49 (52);
 // 4096 tokens 4 kv heads KP 2 184 (194), KP 4 233 (238); 1000 tokens KP 4 34
 // (31), KP 2 43 (39); 2000 tokens KP 2 in 2 parts 77 (77).
+//
+// KP 1 brings half as many tile bytes to LDS per product as KP 2, but its
+// groups are twice as long: it is the faster one where there are enough of
+// them to even out, from 1.4 workgroups per compute unit on (whole layer, us,
+// KP 1 and KP 2: 16384 tokens of 4 kv heads 2140 and 2306, 8192 603 and 646,
+// 6144 (1.5 per unit) 396 and 412, 5000 (1.2) 312 and 299; 12000 of 2 kv heads
+// (1.5) 689 and 687).
 struct SplitPlan {
     int kp, ngrp, parts, sps;
 };
 
 SplitPlan plan_split(int S, int qoff, int Hkv, int cus) {
+    const int n1 = (S + 63) / 64;
+    if (5L * Hkv * n1 >= 7L * cus) return SplitPlan{1, n1, 1, split_steps(1, n1 - 1, S, qoff)};
     SplitPlan best{0, 0, 0, 0};
     float best_us = 0.f;
     for (int kp = 2; kp <= 4; kp += 2) {
@@ -711,8 +728,6 @@ int launch_split(const SplitArgs& a, bool out16, hipStream_t st) {
     using K = void (*)(const SplitArgs);
     static const K kern[2][2] = {{prefill_split_kernel<KP, false, false>, prefill_split_kernel<KP, false, true>},
                                  {prefill_split_kernel<KP, true, false>, prefill_split_kernel<KP, true, true>}};
-    static const K comb[2][2] = {{prefill_split_combine<KP, false, false>, prefill_split_combine<KP, false, true>},
-                                 {prefill_split_combine<KP, true, false>, prefill_split_combine<KP, true, true>}};
     static DeviceOnce lds[2][2];
     const int o = out16 ? 1 : 0, g = a.gate != nullptr ? 1 : 0, bpk = a.ngrp * a.parts;
     const int rc = allow_lds(lds[o][g], reinterpret_cast<const void*>(kern[o][g]), split_lds<KP>());
@@ -721,9 +736,13 @@ int launch_split(const SplitArgs& a, bool out16, hipStream_t st) {
     const dim3 grid(8 % a.Hkv == 0 ? (bpk + spx - 1) / spx * 8 : bpk * a.Hkv);
     hipLaunchKernelGGL(kern[o][g], grid, dim3(kGNT), split_lds<KP>(), st, a);
     ANELM_LAUNCHED("prefill_split_kernel");
-    if (a.parts > 1) {
-        hipLaunchKernelGGL(comb[o][g], dim3(a.ngrp * a.Hkv, 4 * (8 / KP)), dim3(kGNT), 0, st, a);
-        ANELM_LAUNCHED("prefill_split_combine");
+    if constexpr (KP > 1) {   // (KP 1 is never cut)
+        static const K comb[2][2] = {{prefill_split_combine<KP, false, false>, prefill_split_combine<KP, false, true>},
+                                     {prefill_split_combine<KP, true, false>, prefill_split_combine<KP, true, true>}};
+        if (a.parts > 1) {
+            hipLaunchKernelGGL(comb[o][g], dim3(a.ngrp * a.Hkv, 4 * (8 / KP)), dim3(kGNT), 0, st, a);
+            ANELM_LAUNCHED("prefill_split_combine");
+        }
     }
     return ANELM_OK;
 }
@@ -741,7 +760,11 @@ int launch_prefill_split(void* out, bool out16, const void* q, const KeyRing& rg
         a.rec = static_cast<float*>(workspace((size_t)Hkv * sp.ngrp * sp.parts * rec * sizeof(float), st));
         if (!a.rec) return ANELM_ENOMEM;
     }
-    return sp.kp == 2 ? launch_split<2>(a, out16, st) : launch_split<4>(a, out16, st);
+    switch (sp.kp) {
+        case 1: return launch_split<1>(a, out16, st);
+        case 2: return launch_split<2>(a, out16, st);
+        default: return launch_split<4>(a, out16, st);
+    }
 }
 
 template <int D, int HB, int RB>

@@ -352,6 +352,22 @@ def test_prefill_4096_rows(anelm, orc, dev):
     assert_close(got16, got, what="fp16 output")
 
 
+@pytest.mark.parametrize("S,Hq,Hkv", [
+    (700, 4, 1),      # 16-token groups, six key parts merged by the second kernel
+    (1700, 8, 2),     # 32-token groups, three parts, only the long groups cut
+    (5800, 16, 4),    # 64-token groups, one wave per group of 8 tokens, a ragged last one
+])
+def test_prefill_cuts_both_outputs(anelm, orc, dev, S, Hq, Hkv):
+    """The bare core in each of its cuts: sampled rows against the oracle, and
+    fp16 rows that are the fp32 rows rounded."""
+    q, k, v = prefill_inputs(410 + S, S, Hq, Hkv, 256)
+    args = [to_dev(x, dev) for x in (q, k, v)]
+    got = to_host(anelm.ops.attn_prefill(*args))
+    for t in [0, 7, 8, 31, 32, 63, 64, S // 2, S - 41, S - 1]:
+        assert_close(got[t], orc.prefill_attention(q, k, v, t, t + 1)[0], what=f"row {t}")
+    assert np.array_equal(to_host(anelm.ops.attn_prefill(*args, torch.float16)), f16(got))
+
+
 def test_prefill_repeated_calls_are_identical(anelm, orc, dev):
     """Split blocks are merged through per-call counters that each call leaves
     zeroed: back-to-back calls of different sizes (odd block count, middle

@@ -136,6 +136,7 @@ def test_full_attn_prefill_4096_rows(anelm, orc, dev):
     (24, 12, 3, 300, 7, 200, 0, 0, 300, 0),       # kv heads that do not divide the XCDs
     (500, 16, 4, 1024, 600, 300, 0, 0, 1024, 0),  # several key parts of 16-token groups, wrapped ring
     (2100, 16, 4, 4096, 0, 0, 0, 0, 4096, 0),     # more workgroups than compute units
+    (5741, 16, 4, 8192, 7000, 70, 0, 0, 6000, 0),  # groups of 64 tokens (one key part), a ragged last one, wrapped ring
     (40, 16, 4, 128, 100, 10, 0, 0, 64, 2),       # a ring at a 4-byte aligned address: gathered
 ])
 def test_full_attn_prefill_cuts(anelm, dev, S, Hq, Hkv, cap, start, len0, rope_mode, pad, table_rows, off):
