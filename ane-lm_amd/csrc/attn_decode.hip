@@ -1719,13 +1719,9 @@ int launch_kv(DecodeParams& p, int D, int G, dim3 grid, hipStream_t st) {
     }
 }
 
-// Bytes of split partials one decode call needs (0 when one split suffices).
-size_t part_bytes(int n_heads, int n_kv_heads, int D, int n_seqs, int max_len, bool paged) {
-    const int G = n_heads / n_kv_heads;
-    const int kps = paged ? kPagedSplit : 256 / G;
-    const int max_splits = (max_len + kps - 1) / kps;
-    if (max_splits <= 1) return 0;
-    return (size_t)n_seqs * n_kv_heads * max_splits * G * (D + 2) * sizeof(float);
+// Bytes of the records of `splits` splits (0 where one suffices).
+size_t record_bytes(int n_heads, int D, int n_seqs, int splits) {
+    return splits > 1 ? (size_t)n_seqs * splits * n_heads * (D + 2) * sizeof(float) : 0;
 }
 
 // Keys per split of the matrix-core ring kernel, a multiple of its 128 keys
@@ -1740,9 +1736,10 @@ int ring_split_keys(int len, int Hkv, int cus) {
 }
 
 // Sets the split layout and partials buffer for one decode call, then
-// launches.  A split is 256/G keys (ring mode: every lane of the workgroup
-// then loads all of its K and V rows at once) or kPagedSplit keys (paged
-// mode, 16-key blocks per wave).  `max_len` bounds every sequence's key count; `n_seqs`
+// launches.  A split is ring_split_keys keys (the matrix-core ring kernel),
+// 256/G keys (the other rings: every lane of the workgroup then loads all of
+// its K and V rows at once) or kPagedSplit keys (paged mode, 16-key blocks per
+// wave).  `max_len` bounds every sequence's key count; `n_seqs`
 // sequences (1 in ring mode).  The partials go to `part` (part_cap bytes)
 // when it is given, else to the library workspace.
 int run_decode(DecodeParams& p, int kv_dtype, int n_heads, int D, int n_seqs, int max_len,
@@ -1763,8 +1760,7 @@ int run_decode(DecodeParams& p, int kv_dtype, int n_heads, int D, int n_seqs, in
         p.tok_stride = (long)Hkv * D;
         p.head_stride = D;
     }
-    const size_t need =
-        max_splits > 1 ? (size_t)n_seqs * Hkv * max_splits * G * (D + 2) * sizeof(float) : 0;
+    const size_t need = record_bytes(n_heads, D, n_seqs, max_splits);
     // ring mode with few splits: merged in the split kernel (arrival counters)
     const bool merge_inline = !p.paged && max_splits >= 2 && max_splits <= kInlineMaxSplits &&
                               Hkv * n_seqs <= kArrivalWords;
@@ -1961,8 +1957,11 @@ int full_attn_decode_kv_impl(float* out, const float* q_gate, const float* k, co
 }
 
 size_t full_attn_part_bytes(int n_heads, int n_kv_heads, int head_dim, int max_len) {
-    // records, plus the arrival counters at the end of a caller's buffer
-    const size_t b = part_bytes(n_heads, n_kv_heads, head_dim, 1, max_len, false);
+    // records of the shortest splits a ring of this shape may be cut in (256/G
+    // keys: one that is not 16-byte aligned, which is not known here), plus the
+    // arrival counters at the end of a caller's buffer
+    const int kps = 256 / (n_heads / n_kv_heads);
+    const size_t b = record_bytes(n_heads, head_dim, 1, (max_len + kps - 1) / kps);
     return b > 0 ? ((b + 255) & ~(size_t)255) + kArrivalBytes : 0;
 }
 

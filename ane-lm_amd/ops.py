@@ -350,7 +350,7 @@ def lut6_gate_up(x, norm_w, eps, gate, up, hidden, inter):
 
 def lut6_gemm(w, lut, x, out_dim, in_dim, out=None, accumulate=False):
     """y[b] = W x[b] (or y[b] += W x[b]) for a batch x [batch][in_dim]
-    (weights dequantised once per 32 inputs)."""
+    (weights dequantised once per 32 inputs, or once for all of a prompt's)."""
     batch = x.shape[0]
     if out is None:
         if accumulate:

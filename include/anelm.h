@@ -162,9 +162,10 @@ int anelm_full_attn_decode_kv(float* out, const float* q_gate, const float* k, c
  * a static per-device array of 8 MiB (held by every device the library runs
  * on until the process ends), which bounds n_kv_heads * ceil(len / (256 / G))
  * * G * (head_dim + 2) * 4 bytes plus 1 KiB of split-merge counters (len =
- * keys attended after the append, G = n_heads / n_kv_heads): 16 q / 4 kv
- * heads at head_dim 256 attend up to
- * 32448 keys.  Larger calls return ANELM_ERANGE.  Calls that overlap on one
+ * keys attended after the append, G = n_heads / n_kv_heads; the shortest
+ * splits, of 256 / G keys, are what counts, also where a call takes longer
+ * ones): 16 q / 4 kv heads at head_dim 256 attend up to 32448 keys.  Larger
+ * calls return ANELM_ERANGE.  Calls that overlap on one
  * device share that array and race; the library's first call on a device
  * that allocates (e.g. anelm_device_cus) is not needed before this one. */
 int anelm_full_attn_decode_noalloc(float* out, const float* q_gate, const float* k, const float* v,
@@ -391,7 +392,12 @@ int anelm_lut6_swiglu(float* h, const float* x, const float* norm_w, float eps,
  * (accumulate = 1, e.g. the residual add after the FFN down projection) for
  * b < batch (x [batch][in_dim], y [batch][out_dim], fp32; x enters the
  * products as fp16, as in anelm_lut6_gemv).  Each weight is dequantised once
- * per 32 inputs.  No reference counterpart as one call: matvec
+ * per 32 inputs, or once for up to 8192 of them from 65 inputs on (from 33 for
+ * matrices of up to 24 Mi weights).  That path keeps its operands in a buffer
+ * of the stream (fp16 weights and inputs, at most some 450 MB and the partial
+ * sums of small calls) until anelm_stream_release; a stream under capture, or
+ * a device without that memory, takes the passes of 32, whose sums round
+ * otherwise.  No reference counterpart as one call: matvec
  * (core/cpu_ops.cpp:77-80) per input on the dequantised weights. */
 int anelm_lut6_gemm(float* y, const uint8_t* w, const uint16_t* lut, const float* x, int batch,
                     int out_dim, int in_dim, int accumulate, void* stream);
