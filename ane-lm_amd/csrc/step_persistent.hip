@@ -486,7 +486,7 @@ __device__ __forceinline__ void gemv_decode(const Buf<3 * NI>& b, Buf<8 * NA>& d
 // Wave sum and max of this kernel: the stage partners' values by DPP and
 // swizzle.  The lane-swap form of wave_sum needs a second register per stage;
 // here, where every register is taken by weights in flight, that spilled (128
-// bytes a lane instead of 24) and cost the 4B step at context 8192 0.8 % (868
+// bytes a lane instead of 52) and cost the 4B step at context 8192 0.8 % (868
 // us, 862 with this form).
 template <int M = 32>
 __device__ __forceinline__ float step_wave_sum(float v) {
