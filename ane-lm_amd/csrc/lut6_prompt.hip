@@ -288,11 +288,20 @@ void prompt_gemm_kernel(const PromptArgs a) {
         for_each_stage(std::make_integer_sequence<int, kChain>{}, [&](auto s) __attribute__((always_inline)) {
             stage(i + decltype(s)::value, s);
         });
-    for (; i < nk; i++) stage(i, std::integral_constant<int, -1>{});
+    auto end_chains = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int x = 0; x < MI; x++)
+        for (int x = 0; x < MI; x++)
 #pragma unroll
-        for (int y = 0; y < NI; y++) sum[x][y] += acc[x][y];
+            for (int y = 0; y < NI; y++) {
+                sum[x][y] += acc[x][y];
+                acc[x][y] = float16_t{};
+            }
+    };
+    end_chains();
+    if (i < nk) {   // (fewer than kChain stages left)
+        for (; i < nk; i++) stage(i, std::integral_constant<int, -1>{});
+        end_chains();
+    }
     __builtin_amdgcn_s_waitcnt(0x0F70);   // no load into LDS outlives the workgroup
     float* y = a.y + blockIdx.y * a.sy;
     // C layout: element e of lane l is input row 8 (e / 4) + 4 (l / 32) + e % 4,
