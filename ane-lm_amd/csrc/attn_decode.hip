@@ -1090,8 +1090,8 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3))) void a
 // Bound: instruction issue and latency of one pass (the whole kernel is some
 // 1500 instructions per wave, executed once); whole call before (fp32 vector
 // products, 64-key splits) and now: 513 keys 8q/2kv 11.4 -> 9.8 us, 8192 keys
-// 16q/4kv 23.2 -> 13.4 us (33.6 MB; merge kernel 4 of it), errors against 64
-// bits 1.9e-7 and 2.3e-7 as before.
+// 16q/4kv 23.2 -> 14.1 us (33.6 MB; merge kernel 4.7 of it), errors against 64
+// bits 1.9e-7 and 2.4e-7 as before.
 constexpr int kRNT = 512;
 constexpr int kRW = kRNT / 64;
 constexpr int kRBlk = 16;
@@ -1728,7 +1728,7 @@ size_t record_bytes(int n_heads, int D, int n_seqs, int splits) {
 // per round of blocks: one round while that gives at most a workgroup per CU
 // (a further round costs its memory latency, 3 us: 513 keys of 2 kv heads 9.7
 // us in 5 splits of one round, 12.8 in 3 of two; 8192 keys of 4 kv heads 13.4
-// and 16.0), then as many rounds as keep one workgroup per CU (32768 keys of 4
+// and 16.0, with all query terms on one scale), then as many rounds as keep one workgroup per CU (32768 keys of 4
 // kv heads: 27.7 us in 64 splits of four rounds, 31.7 in 128, 30.6 in 43).
 int ring_split_keys(int len, int Hkv, int cus) {
     const long round = kRW * kRBlk;

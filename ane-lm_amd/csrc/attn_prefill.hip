@@ -214,9 +214,8 @@ __global__ __launch_bounds__(HB * RB * 64) void prefill_kernel(void* out, const 
 // 1 us of the CU's matrix time and its operand reads 1 us of its LDS; a step
 // takes 1.9 us, 2.8 us with every CU under load).  Whole layer call, before
 // (64-row blocks in causal pairs, two workgroups per pair, which left the chip
-// to 2 Hkv ceil(S / 128) workgroups) and now: 4096 tokens 16q/4kv 228 -> 217
-// us, 1000 tokens 82 -> 44, 777 tokens 8q/2kv behind 1500 keys 146 -> 44, 16
-// tokens behind 4000 keys 110 -> 22.
+// to 2 Hkv ceil(S / 128) workgroups) and now: 4096 tokens 16q/4kv 230 -> 202
+// us, 1000 tokens 86 -> 45, 777 tokens 8q/2kv behind 1500 keys 150 -> 42.5.
 constexpr int kGKeys = 32;                       // keys per tile
 constexpr int kGKBytes = 16 * 1040;              // K tile: chunk c = rows c, c + 16
 constexpr int kGVChunk = 1088;                   // V tile chunk: rows c, c + 16 + 64 bytes of bank offset

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kNT) void rmsnorm_gated_rows_kernel(float* out, con
 // The 128-element rows of a DeltaNet head (8-byte aligned): lane l holds
 // elements 2l, 2l + 1, one 8-byte load per operand.  Row r's z is at
 // z + (r / heads) * zs + (r % heads) * 128: the z part of a projection row is
-// read where it lies.  Memory-bound (4096 tokens of 32 heads: 201 MB in 36 us).
+// read where it lies.  Memory-bound (4096 tokens of 32 heads: 201 MB in 38.5 us).
 __global__ __launch_bounds__(kNT) void rmsnorm_gated_rows128_kernel(float* out, const float* x, const float* z,
                                                                     const float* w, int n_rows, int heads, long zs) {
     const int row = blockIdx.x * (kNT / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;

@@ -432,8 +432,8 @@ __device__ __forceinline__ float conv_tap4(float x0, float x1, float x2, float x
 // LDS matrices are row-major with 16-byte chunks XOR-swizzled by (row & 15);
 // 66 KB, so two workgroups share a CU (one's serial phases overlap the other).
 // Bound: memory (134 MB read, 224 MB of records written for 4096 tokens of 32
-// heads: 65 us at 5.5 TB/s) and the vector units (conv and SiLU): 102 us, where
-// conv pass and preparation took 77 + 140.
+// heads: 65 us at 5.5 TB/s) and the vector units (conv and SiLU): 114 us, where
+// conv pass and preparation took 77 + 140 (86 us without the conv).
 constexpr int kPmNT = 512;
 constexpr int kPmK = 0;                        // K rows [64][128]
 constexpr int kPmR = kCMat;                    // Q rows [64][128] for the Gram tiles, then:

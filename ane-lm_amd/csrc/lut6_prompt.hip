@@ -397,10 +397,10 @@ constexpr size_t kMaxW16 = (size_t)256 << 20;
 }  // namespace
 
 // From 65 inputs on the one-time decode always wins (128 inputs, us: 18432 x
-// 2560 73 -> 56, 2560 x 9216 76 -> 40, 2560 x 4096 80 -> 30, 7168 x 1024 116 ->
-// 25); 33..64 inputs take two passes of the register-window kernel, which the
+// 2560 72 -> 50, 2560 x 9216 75 -> 37, 2560 x 4096 80 -> 25, 7168 x 1024 117 ->
+// 22); 33..64 inputs take two passes of the register-window kernel, which the
 // one-time decode beats except for the largest matrices (64 inputs: 2560 x
-// 9216 37 -> 33, 7168 x 1024 58 -> 24, but 12352 x 2560 37 -> 38 and 18432 x
+// 9216 36 -> 31, 7168 x 1024 58 -> 23, but 12352 x 2560 37 -> 38 and 18432 x
 // 2560 37 -> 47).  Streams under capture keep the register-window kernel: a
 // captured launch would hold this path's workspace, which a later call may
 // replace.  w needs dword loads, x 16-byte ones.

@@ -81,7 +81,7 @@ template <> struct Row<2> {
 // E l + E - 1: a row is one load and one store per lane (VEC: rows and
 // weights aligned to it; otherwise E dword loads), interleaved pairs stay in
 // the lane and half-split pairs are rot_pairs / E lanes apart, so no row
-// passes through LDS.  Bound: memory (4096 tokens 16q/4kv move 150 MB in 30 us;
+// passes through LDS.  Bound: memory (4096 tokens 16q/4kv move 150 MB in 32 us;
 // with dword loads and rows through LDS 33, and 6.4 more for the keys' second
 // copy into the ring).
 constexpr int kPrepRowsPerWg = 4;
