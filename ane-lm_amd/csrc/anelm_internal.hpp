@@ -57,8 +57,10 @@ struct StreamState {
     size_t ws2_bytes = 0;
     void* wsp = nullptr;      // operands of the LUT6 prompt product
     size_t wsp_bytes = 0;
+    void* wsr = nullptr;      // key-part records of the prompt attention
+    size_t wsr_bytes = 0;
     uint32_t* counters = nullptr;
-    std::mutex mu;            // guards growth of ws / ws2 / wsp
+    std::mutex mu;            // guards growth of ws / ws2 / wsp / wsr
 };
 
 struct Device {
@@ -91,6 +93,10 @@ void* workspace2(size_t bytes, hipStream_t stream);
 // call still points to.  (That product is never captured.)  ANELM_ENOMEM: the
 // memory is not there; ANELM_EHIP: another failure, as of an earlier launch.
 int prompt_workspace(void** p, size_t bytes, hipStream_t stream);
+// The prompt attention's key-part records, likewise apart: a few tokens behind
+// a long ring take megabytes, and the first buffer may be held by a graph
+// captured from a decode call.
+void* record_workspace(size_t bytes, hipStream_t stream);
 
 // Workgroup barrier for LDS exchange only: this wave's LDS operations
 // complete, then s_barrier.  __syncthreads() also carries a release fence that

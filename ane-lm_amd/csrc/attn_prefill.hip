@@ -756,7 +756,7 @@ int launch_prefill_split(void* out, bool out16, const void* q, const KeyRing& rg
                 sp.ngrp, sp.parts, sp.sps};
     if (sp.parts > 1) {
         const size_t rec = sp.kp == 2 ? split_rec_floats<2>() : split_rec_floats<4>();
-        a.rec = static_cast<float*>(workspace((size_t)Hkv * sp.ngrp * sp.parts * rec * sizeof(float), st));
+        a.rec = static_cast<float*>(record_workspace((size_t)Hkv * sp.ngrp * sp.parts * rec * sizeof(float), st));
         if (!a.rec) return ANELM_ENOMEM;
     }
     switch (sp.kp) {

@@ -128,6 +128,13 @@ void* workspace2(size_t bytes, hipStream_t stream) {
     return p;
 }
 
+void* record_workspace(size_t bytes, hipStream_t stream) {
+    StreamState* s = stream_state(stream);
+    void* p = nullptr;
+    if (s) (void)grow(s, s->wsr, s->wsr_bytes, bytes, &p);
+    return p;
+}
+
 int prompt_workspace(void** p, size_t bytes, hipStream_t stream) {
     *p = nullptr;
     StreamState* s = stream_state(stream);
@@ -163,6 +170,7 @@ int stream_release(hipStream_t stream) {
     if (s->ws) (void)hipFree(s->ws);
     if (s->ws2) (void)hipFree(s->ws2);
     if (s->wsp) (void)hipFree(s->wsp);
+    if (s->wsr) (void)hipFree(s->wsr);
     (void)hipFree(s->counters);
     delete s;
     if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");

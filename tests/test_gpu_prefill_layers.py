@@ -326,3 +326,39 @@ def test_deltanet_prefill_from_proj_over_its_rows(anelm, dev, flags, off):
 
     for got, want, what in zip(run(True), run(False), ("y", "state", "conv ring")):
         assert_close(got, want, rel=1e-5, max_abs=1e-3, what=what)
+
+
+def test_short_prompt_leaves_captured_decode(anelm, dev):
+    """A graph captured from a decode step holds the stream's first buffer (its
+    split records); a few tokens behind a long ring on that stream keep the
+    records of their key parts elsewhere, so every replay gives the eager step."""
+    Hq, Hkv, D, cap = 8, 2, 256, 4096
+    c = _attn_case(1990, 1, Hq, Hkv, D, cap, 0, 3000)
+    q, k, v = (to_dev(c[n][0], dev) for n in ("q_gate", "k", "v"))
+    kc, vc, qw, kw = (to_dev(c[n], dev) for n in ("kc", "vc", "qw", "kw"))
+    rng = np.random.default_rng(1991)
+    proj = to_dev(rng.standard_normal((100, Hq * 2 * D + 2 * Hkv * D)).astype(np.float32), dev)
+    out, s = torch.empty(Hq, D, device=dev), torch.cuda.Stream()
+
+    def step():   # (the same slot each time: a fresh ring object, the position fixed)
+        anelm.ops.full_attn_decode(q, k, v, kc, vc, qw, kw, anelm.ops.KVRing(cap, 0, 3000), Hq, Hkv, D, 64, 3000, out=out)
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        step()
+        want = out.clone()
+        graph = torch.cuda.CUDAGraph()
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            step()
+        first = {}
+        for tokens in (24, 100, 24):
+            got = anelm.ops.full_attn_prefill(None, None, None, kc.clone(), vc.clone(), qw, kw,
+                                              anelm.ops.KVRing(cap, 0, 3000), Hq, Hkv, D, 64, 3000, proj=proj[:tokens])
+            out.zero_()
+            graph.replay()
+            s.synchronize()
+            assert torch.equal(out, want), tokens
+            assert torch.equal(got, first.setdefault(tokens, got.clone()))
+    del graph
+    anelm.call("anelm_stream_release", ctypes.c_void_p(s.cuda_stream))
