@@ -90,21 +90,39 @@ def test_full_attn_decode_variants(anelm, orc, dev, rope_mode, gate):
 
 
 @pytest.mark.parametrize("n_heads,n_kv_heads,head_dim,cached", [
-    (8, 2, 256, 127),    # G 4, 64-key splits: 2 splits, the smallest in-kernel merge
-    (8, 2, 256, 1023),   # 16 splits, the largest merged in the split kernel
-    (8, 2, 256, 1024),   # 17 splits: the merge kernel
+    (8, 2, 256, 127),    # G 4 on the matrix cores, 128-key splits: one full split
+    (8, 2, 256, 1023),   # 8 splits, merged in the kernel
+    (8, 2, 256, 1024),   # 9 splits, the last with one key
     (16, 2, 128, 300),   # G 8, 32-key splits: 10 splits
     (4, 2, 128, 700),    # G 2, 128-key splits (workgroup-wide softmax): 6 splits
     (4, 4, 64, 1000),    # G 1, 256-key splits: 4 splits
 ])
 def test_full_attn_decode_split_merge(anelm, orc, dev, n_heads, n_kv_heads, head_dim, cached):
-    """Split counts around the in-kernel merge of the split records (up to 16
-    splits of 256/G keys merged by the last workgroup of each kv head, more by
-    a second kernel) and the other head groupings, over a wrapped ring,
-    against the oracle."""
+    """Split records merged in the kernel (up to 16 splits by the last workgroup
+    of each kv head) for every head grouping, over a wrapped ring, against the
+    oracle."""
     c = attn_decode_case(330 + cached % 97, n_heads=n_heads, n_kv_heads=n_kv_heads, head_dim=head_dim,
                          cached=cached, capacity=cached + 5, start=7)
     _check_decode(_run_decode(anelm, c, dev), _oracle_decode(orc, c))
+
+
+@pytest.mark.parametrize("cached", [
+    127,     # two 64-key splits, the smallest in-kernel merge
+    1023,    # 16 splits, the largest merged in the split kernel
+    1024,    # 17 splits: the merge kernel
+])
+def test_full_attn_decode_split_merge_off_alignment(anelm, orc, dev, cached):
+    """The same for rings of four query heads per kv head at 4-byte aligned
+    addresses, which the vector kernel takes."""
+    c = attn_decode_case(330 + cached % 97, n_heads=8, n_kv_heads=2, head_dim=256, cached=cached, capacity=cached + 5,
+                         start=7)
+    kc, vc = (torch.cat([torch.zeros(2, dtype=torch.float16, device=dev), to_dev(x, dev).flatten()])[2:].view(x.shape)
+              for x in (c.k_cache, c.v_cache))
+    ring = anelm.ops.KVRing(c.capacity, c.start, c.length)
+    out = anelm.ops.full_attn_decode(to_dev(c.q_gate, dev), to_dev(c.k, dev), to_dev(c.v, dev), kc, vc,
+                                     to_dev(c.q_norm_w, dev), to_dev(c.k_norm_w, dev), ring, c.n_heads, c.n_kv_heads,
+                                     c.head_dim, c.rot_dim, c.pos, c.theta, c.eps)
+    _check_decode((to_host(out), to_host(kc), to_host(vc), ring.start.value, ring.len.value), _oracle_decode(orc, c))
 
 
 @pytest.mark.parametrize("Hq,Hkv,cached,start,rope_mode,rot,gate,scale,off", [
@@ -369,9 +387,9 @@ def test_prefill_cuts_both_outputs(anelm, orc, dev, S, Hq, Hkv):
 
 
 def test_prefill_repeated_calls_are_identical(anelm, orc, dev):
-    """Split blocks are merged through per-call counters that each call leaves
-    zeroed: back-to-back calls of different sizes (odd block count, middle
-    unit, split pairs) give bit-identical rows, and match the oracle."""
+    """Key parts leave records in scratch that the next call writes over:
+    back-to-back calls of different sizes and cuts give bit-identical rows, and
+    match the oracle."""
     runs = {}
     for S in (700, 130, 700, 64, 700):
         q, k, v = prefill_inputs(990 + S, S, 16, 4, 256)

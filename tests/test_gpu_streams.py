@@ -22,7 +22,7 @@ class Work:
     current stream from fresh copies of the mutable buffers."""
 
     def __init__(self, seed, dev):
-        # 901 keys over a wrapped ring: 15 key splits of 64, merged in the
+        # 901 keys over a wrapped ring: 8 key splits of 128, merged in the
         # kernel through the stream's arrival counters
         self.c = attn_decode_case(seed, n_heads=16, n_kv_heads=4, head_dim=256, cached=900,
                                   capacity=2048, start=1500)

@@ -49,12 +49,12 @@ def _compare(anelm, c, dev, label):
 
 
 def test_noalloc_matches_full_attn_decode(anelm, dev):
-    # 4B shape over a full 8192-key ring that wraps (128 splits per kv head)
+    # 4B shape over a full 8192-key ring that wraps (64 splits per kv head)
     big = attn_decode_case(950, n_heads=16, n_kv_heads=4, cached=8192, capacity=8192, start=37)
     print("noalloc: 16q/4kv D256, 8192-key wrapping ring", flush=True)
     _compare(anelm, big, dev, "16q/4kv 8192 keys")
     free0, _ = torch.cuda.mem_get_info()
-    # then a smaller call: 0.8B shape, 513 keys (9 splits), stale partials of
+    # then a smaller call: 0.8B shape, 513 keys (5 splits), stale partials of
     # the first call still in the array
     small = attn_decode_case(951)
     print("noalloc: 8q/2kv D256, 513 keys", flush=True)
